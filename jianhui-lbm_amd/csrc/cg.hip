@@ -119,12 +119,12 @@ __device__ __forceinline__ void load_cs<double>(const double *cs, int64_t n, int
 
 template <typename ST, int MODE>
 __device__ __forceinline__ void cg_node_state(const CgArgs<ST> &a, int64_t n, typename Store<ST>::C (&h)[Q],
-                                              typename Store<ST>::C (&m)[Q], uint32_t (&nb)[Q - 1],
+                                              typename Store<ST>::C (&m)[Q], Links<Q - 1> &l,
                                               Macro<typename Store<ST>::C> &mc)
 {
     using C = typename Store<ST>::C;
-    load_nbr(a.nbr, a.P, n, nb);
     if (MODE == K_INIT) {
+        load_links(a.nbr, a.P, n, l);
         mc.rho = C(1);
         mc.drho = C(1) - a.rho0;
         mc.ux = a.ux_i;
@@ -134,16 +134,9 @@ __device__ __forceinline__ void cg_node_state(const CgArgs<ST> &a, int64_t n, ty
         return;
     }
     h[0] = Store<ST>::load(a.src[n], a.inv_scale);
-#pragma unroll
-    for (int q = 1; q < Q; ++q) {
-        if (MODE == K_DIRECT) {
-            h[q] = Store<ST>::load(a.src[(int64_t)q * a.P + n], a.inv_scale);
-        } else {
-            const uint32_t v = nb[q - 1];
-            const int64_t row = (v & BB_FLAG) ? (int64_t)opp(q) : (int64_t)q;
-            h[q] = Store<ST>::load(a.src[row * a.P + (int64_t)(v & ~BB_FLAG)], a.inv_scale);
-        }
-    }
+    gather_links(a.nbr, a.P, n, l, [&](int q) {
+        h[q] = Store<ST>::load(a.src[MODE == K_DIRECT ? (int64_t)q * a.P + n : pull_offset(l, a.P, n, q)], a.inv_scale);
+    });
     moments_fwd(h, m);
     if (MODE == K_DIRECT) {
         mc.rho = a.rho_aux[n];
@@ -165,19 +158,19 @@ __device__ __forceinline__ void cg_collide_node(const CgArgs<ST> &a, int64_t n, 
 {
     using C = typename Store<ST>::C;
     const int32_t own = FAST ? (int32_t)n + w.own : 0;
-    // psi at the site of table column j, whose entry is v (a solid site's value is not used;
-    // its index is the node itself)
-    auto psi_at = [&](int j, uint32_t v) -> C {
-        if (SLOTS > 0 && FAST) {
-            const int32_t up = (int32_t)v + w.d[j];
-            return lpsi[(v & BB_FLAG) ? own : up];
-        }
-        return a.psi[v & ~BB_FLAG];
-    };
     C h[Q], m[Q];
-    uint32_t nb[Q - 1];
+    Links<Q - 1> l;
     Macro<C> mc;
-    cg_node_state<ST, MODE>(a, n, h, m, nb, mc);
+    cg_node_state<ST, MODE>(a, n, h, m, l, mc);
+    // psi at the upstream site of direction q (at the node itself where the site is solid, whose
+    // value is not used)
+    auto psi_at = [&](int q) -> C {
+        if (SLOTS > 0 && FAST) {
+            const int32_t up = (int32_t)l.up[q - 1] + w.d[q - 1];
+            return lpsi[l.solid(q) ? own : up];
+        }
+        return a.psi[l.solid(q) ? n : (int64_t)l.up[q - 1]];
+    };
     using CS = ColourStore<C>;
     const typename CS::T rr_raw = a.col[n], rb_raw = a.col[a.P + n];
     const C rr = (C)CS::real(rr_raw), rb = (C)CS::real(rb_raw), ps = a.psi[n];
@@ -188,11 +181,10 @@ __device__ __forceinline__ void cg_collide_node(const CgArgs<ST> &a, int64_t n, 
     bool wall = false;
 #pragma unroll
     for (int q = 1; q < Q; ++q) {
-        const uint32_t v = nb[opp(q) - 1];
-        const bool solid = (v & BB_FLAG) != 0;
+        const bool solid = l.solid(opp(q));
         wall |= solid;
         // unconditional load, then select
-        const C pv = psi_at(opp(q) - 1, v);
+        const C pv = psi_at(opp(q));
         const C pq = solid ? a.psi_solid : pv;
         const C wq = C(3.0 * weight(q));
         if (EX[q] != 0) cx += C(EX[q]) * wq * pq;
@@ -316,7 +308,7 @@ __device__ __forceinline__ void colour_pull_term(const C (&v)[8], bool bb, C &gr
 
 // The FP64 build's colour sums of one node, direction by direction: begin() with the node's own
 // colour state (the rest population stays on the node: e_0 = 0, no recolouring term), add() the
-// term arriving along q from an upstream state (bb: BB_FLAG when the upstream site is solid and v
+// term arriving along q from an upstream state (bb when the upstream site is solid and v
 // is the node's own state, whose opposite term comes back), then store().  The gather and the
 // staged kernel add the same terms in the same order, so they give the same bits.
 struct ColourSums64 {
@@ -329,10 +321,10 @@ struct ColourSums64 {
         rb = w0 * own[1];
     }
     template <int q>
-    __device__ __forceinline__ void add(uint32_t bb, const double (&v)[8])
+    __device__ __forceinline__ void add(bool bb, const double (&v)[8])
     {
         double gr, gb;
-        colour_pull_term<q>(v, bb != 0, gr, gb);
+        colour_pull_term<q>(v, bb, gr, gb);
         rr += gr;
         rb += gb;
     }
@@ -348,7 +340,7 @@ struct ColourSums64 {
 // groups of three directions with no branch between them, so that each group's gathers are in
 // flight together (measured best: 351 us at 3, 402 us at 6).  A solid upstream site sends back
 // this node's own opposite term: same load address n, sign -1.
-__device__ __forceinline__ void colour_gather64(const double *__restrict__ cs, const uint32_t (&src)[Q - 1], int64_t n,
+__device__ __forceinline__ void colour_gather64(const double *__restrict__ cs, const Links<Q - 1> &src, int64_t n,
                                                 int64_t P, ColourSums64 &acc)
 {
     constexpr int G = 3;
@@ -357,12 +349,11 @@ __device__ __forceinline__ void colour_gather64(const double *__restrict__ cs, c
         double up[G][8];
 #pragma unroll
         for (int j = 0; j < G; ++j) {
-            const uint32_t v = src[q0 + j - 1];
-            load_cs(cs, (v & BB_FLAG) ? n : (int64_t)v, P, up[j]);
+            load_cs(cs, src.solid(q0 + j) ? n : (int64_t)src.up[q0 + j - 1], P, up[j]);
         }
         static_for<0, G>([&](auto jj) {
             constexpr int j = decltype(jj)::value;
-            acc.add<q0 + j>(src[q0 + j - 1] & BB_FLAG, up[j]);
+            acc.add<q0 + j>(src.solid(q0 + j), up[j]);
         });
     });
 }
@@ -375,8 +366,8 @@ __global__ void __launch_bounds__(BLOCK) cg_colour_kernel64(NbrDev nbr, const do
     if (n >= N) return;
     double own[8];
     load_cs(cs, n, P, own);
-    uint32_t src[Q - 1];
-    load_nbr(nbr, P, n, src);
+    Links<Q - 1> src;
+    load_links(nbr, P, n, src);
     ColourSums64 acc;
     acc.begin(own);
     colour_gather64(cs, src, n, P, acc);
@@ -423,9 +414,9 @@ struct ColourSums {
         tr = c0 * ((float)R0 * UNIT);
         tb = c0 * ((float)B0 * UNIT);
     }
-    // bb: BB_FLAG (the sign bit) when the upstream site is solid, else 0
+    // bb: the upstream site is solid
     template <int q>
-    __device__ __forceinline__ void add(uint32_t bb, const float (&vs)[8])
+    __device__ __forceinline__ void add(bool bb, const float (&vs)[8])
     {
         constexpr bool axis = e2_of(q) == 1;
         const int32_t R = __float_as_int(vs[0]), B = __float_as_int(vs[1]);
@@ -436,16 +427,15 @@ struct ColourSums {
         const float wr = (float)R * WU, wb = (float)B * WU;
         const float ux = vs[2], uy = vs[3], uz = vs[4];
         const float uu = ux * ux + uy * uy + uz * uz;
-        // a solid upstream site sends back this node's own opposite share: e_q negated, by
-        // flipping the sign bit
-        const float eu = __int_as_float(__float_as_int(e_dot<q>(ux, uy, uz)) ^ (int32_t)bb);
+        // a solid upstream site sends back this node's own opposite share: e_q negated
+        const float du = e_dot<q>(ux, uy, uz), eu = bb ? -du : du;
         // phi_q - 1 formed from the small terms alone: rounding 1 + small and taking 1 off again
         // would be biased, and would drift the colour totals
         const float s2 = 4.5f * eu * eu - 1.5f * uu;
         const float eps = s2 + 3.0f * eu;
         const float phq = 1.0f + eps, php = 1.0f + (s2 - 3.0f * eu);
         const float mn = fminf(fminf(fminf(wr * phq, wr * php), wb * phq), wb * php);
-        const float en = __int_as_float(__float_as_int(e_dot<q>(vs[5], vs[6], vs[7])) ^ (int32_t)bb);
+        const float dn = e_dot<q>(vs[5], vs[6], vs[7]), en = bb ? -dn : dn;
         tr += wr * eps + mn * en;
         tb += wb * eps - mn * en;
     }
@@ -461,19 +451,18 @@ struct ColourSums {
 template <int q>
 struct ColourStep {
     template <typename F>
-    static __device__ __forceinline__ void run(ColourSums &acc, const uint32_t (&src)[Q - 1], F &&fetch)
+    static __device__ __forceinline__ void run(ColourSums &acc, const Links<Q - 1> &src, F &&fetch)
     {
         float v[8];
-        const uint32_t id = src[q - 1];
-        fetch(q - 1, id, v);
-        acc.add<q>(id & BB_FLAG, v);
+        fetch(q, v);
+        acc.add<q>(src.solid(q), v);
         ColourStep<q + 1>::run(acc, src, fetch);
     }
 };
 template <>
 struct ColourStep<Q> {
     template <typename F>
-    static __device__ __forceinline__ void run(ColourSums &, const uint32_t (&)[Q - 1], F &&)
+    static __device__ __forceinline__ void run(ColourSums &, const Links<Q - 1> &, F &&)
     {
     }
 };
@@ -488,23 +477,23 @@ static_assert((Q - 1) % CW_GROUP == 0, "groups cover the 18 directions");
 // (T: the state's value type; Acc: ColourSums or ColourSums64)
 template <int q, typename T, typename Acc, int i = 0>
 struct ColourAdd {
-    static __device__ __forceinline__ void run(Acc &acc, const uint32_t (&src)[Q - 1], const T (&v)[CW_GROUP][8])
+    static __device__ __forceinline__ void run(Acc &acc, const Links<Q - 1> &src, const T (&v)[CW_GROUP][8])
     {
-        acc.template add<q + i>(src[q + i - 1] & BB_FLAG, v[i]);
+        acc.template add<q + i>(src.solid(q + i), v[i]);
         if constexpr (i + 1 < CW_GROUP) ColourAdd<q, T, Acc, i + 1>::run(acc, src, v);
     }
 };
 template <int q, typename T, typename Acc>
 struct ColourGroups {
     template <typename F>
-    static __device__ __forceinline__ void run(Acc &acc, const uint32_t (&src)[Q - 1], const T (&cur)[CW_GROUP][8],
+    static __device__ __forceinline__ void run(Acc &acc, const Links<Q - 1> &src, const T (&cur)[CW_GROUP][8],
                                                F &&fetch)
     {
         constexpr int qn = q + CW_GROUP;
         T nxt[CW_GROUP][8];
         if constexpr (qn < Q) {
 #pragma unroll
-            for (int j = 0; j < CW_GROUP; ++j) fetch(qn + j - 1, src[qn + j - 1], nxt[j]);
+            for (int j = 0; j < CW_GROUP; ++j) fetch(qn + j, nxt[j]);
         }
         __builtin_amdgcn_sched_barrier(0);
         ColourAdd<q, T, Acc>::run(acc, src, cur);
@@ -522,12 +511,12 @@ __global__ void __launch_bounds__(BLOCK) cg_colour_kernel_fx(NbrDev nbr, const f
     if (n >= N) return;
     float own[8];
     load_cs(cs, n, P, own);
-    uint32_t src[Q - 1];
-    load_nbr(nbr, P, n, src);
+    Links<Q - 1> src;
+    load_links(nbr, P, n, src);
     ColourSums acc;
     acc.begin(own);
     ColourStep<1>::run(acc, src,
-                       [&](int, uint32_t v, float (&out)[8]) { load_cs(cs, (v & BB_FLAG) ? n : (int64_t)v, P, out); });
+                       [&](int q, float (&out)[8]) { load_cs(cs, src.solid(q) ? n : (int64_t)src.up[q - 1], P, out); });
     acc.store(n, P, col, psi);
 }
 
@@ -557,8 +546,8 @@ __global__ void __launch_bounds__(CW_BLOCK) cg_colour_kernel_win(NbrDev nbr, con
     const int64_t n = b * CW_BLOCK + threadIdx.x;
     // the neighbour table first, in flight during the staging (the table has P >= N rows, P a
     // multiple of 256, so a 512-node block can reach past its end: lanes past N load nothing)
-    uint32_t src[Q - 1];
-    if (n < N) load_nbr(nbr, P, n, src);
+    Links<Q - 1> src;
+    if (n < N) load_links(nbr, P, n, src);
     if (w.fast == CW_ALL) {   // the same for the whole block
         // slots threadIdx.x + i CW_BLOCK: all loads in flight before the first LDS write
         constexpr int NS = SLOTS / CW_BLOCK;
@@ -592,13 +581,13 @@ __global__ void __launch_bounds__(CW_BLOCK) cg_colour_kernel_win(NbrDev nbr, con
         // matched with the read above, which would turn the select into a branch per lane group
         int32_t own_sel = own;
         asm volatile("" : "+v"(own_sel));
-        auto fetch = [&](int j, uint32_t v, float (&out)[8]) {
-            const int32_t up = (int32_t)v + w.d[j];
-            lds_state((v & BB_FLAG) ? own_sel : up, out);
+        auto fetch = [&](int q, float (&out)[8]) {
+            const int32_t up = (int32_t)src.up[q - 1] + w.d[q - 1];
+            lds_state(src.solid(q) ? own_sel : up, out);
         };
         float first[CW_GROUP][8];
 #pragma unroll
-        for (int j = 0; j < CW_GROUP; ++j) fetch(j, src[j], first[j]);
+        for (int j = 0; j < CW_GROUP; ++j) fetch(1 + j, first[j]);
         acc.begin(own_v);
         ColourGroups<1, float, ColourSums>::run(acc, src, first, fetch);
         acc.store(n, P, col, psi);
@@ -609,7 +598,7 @@ __global__ void __launch_bounds__(CW_BLOCK) cg_colour_kernel_win(NbrDev nbr, con
     load_cs(cs, n, P, own);
     acc.begin(own);
     ColourStep<1>::run(acc, src,
-                       [&](int, uint32_t v, float (&out)[8]) { load_cs(cs, (v & BB_FLAG) ? n : (int64_t)v, P, out); });
+                       [&](int q, float (&out)[8]) { load_cs(cs, src.solid(q) ? n : (int64_t)src.up[q - 1], P, out); });
     acc.store(n, P, col, psi);
 }
 
@@ -628,8 +617,8 @@ __global__ void __launch_bounds__(CW_BLOCK) cg_colour_kernel_win64(NbrDev nbr, c
     const ColourWin w = wins[b];
     const d2 *__restrict__ cs2 = reinterpret_cast<const d2 *>(cs);   // node m: cs2[4 m .. 4 m + 3]
     const int64_t n = b * CW_BLOCK + threadIdx.x;
-    uint32_t src[Q - 1];
-    if (n < N) load_nbr(nbr, P, n, src);   // lanes past N load nothing (see cg_colour_kernel_win)
+    Links<Q - 1> src;
+    if (n < N) load_links(nbr, P, n, src);   // lanes past N load nothing (see cg_colour_kernel_win)
     if (w.fast == CW_ALL) {   // the same for the whole block
         constexpr int NS = SLOTS / CW_BLOCK;
         static_assert(SLOTS % CW_BLOCK == 0, "whole slots per lane");
@@ -662,13 +651,13 @@ __global__ void __launch_bounds__(CW_BLOCK) cg_colour_kernel_win64(NbrDev nbr, c
         lds_state(own, own_v);
         int32_t own_sel = own;   // kept apart from `own`, as in cg_colour_kernel_win
         asm volatile("" : "+v"(own_sel));
-        auto fetch = [&](int j, uint32_t v, double (&out)[8]) {
-            const int32_t up = (int32_t)v + w.d[j];
-            lds_state((v & BB_FLAG) ? own_sel : up, out);
+        auto fetch = [&](int q, double (&out)[8]) {
+            const int32_t up = (int32_t)src.up[q - 1] + w.d[q - 1];
+            lds_state(src.solid(q) ? own_sel : up, out);
         };
         double first[CW_GROUP][8];
 #pragma unroll
-        for (int j = 0; j < CW_GROUP; ++j) fetch(j, src[j], first[j]);
+        for (int j = 0; j < CW_GROUP; ++j) fetch(1 + j, first[j]);
         acc.begin(own_v);
         ColourGroups<1, double, ColourSums64>::run(acc, src, first, fetch);
         acc.store(n, P, col, psi);
@@ -700,9 +689,9 @@ __global__ void __launch_bounds__(BLOCK) cg_diag_kernel(CgArgs<ST> a, const int3
     for (int k = 0; k < CG_NDIAG; ++k) v[k] = 0.0;
     if (n < a.N) {
         C h[Q], m[Q];
-        uint32_t nb[Q - 1];
+        Links<Q - 1> l;
         Macro<C> mc;
-        cg_node_state<ST, MODE>(a, n, h, m, nb, mc);
+        cg_node_state<ST, MODE>(a, n, h, m, l, mc);
         const double ux = (double)mc.ux, uy = (double)mc.uy, uz = (double)mc.uz, ps = (double)a.psi[n];
         const int32_t s = supinv[n];
         const int32_t nyz = box.ny * box.nz;
@@ -755,13 +744,13 @@ __global__ void __launch_bounds__(BLOCK) cg_get_state_kernel(CgArgs<ST> a, int64
                                                              double *__restrict__ rr_out, double *__restrict__ rb_out)
 {
     using C = typename Store<ST>::C;
-    const int64_t n = group_floor(n0) + (int64_t)blockIdx.x * BLOCK + threadIdx.x;   // see load_nbr
+    const int64_t n = group_floor(n0) + (int64_t)blockIdx.x * BLOCK + threadIdx.x;   // see load_links
     if (n < n0 || n >= n1) return;
     const int64_t l = n - n0;
     C h[Q], m[Q];
-    uint32_t nb[Q - 1];
+    Links<Q - 1> links;
     Macro<C> mc;
-    cg_node_state<ST, MODE>(a, n, h, m, nb, mc);
+    cg_node_state<ST, MODE>(a, n, h, m, links, mc);
     if (f_out) {
         double f[Q];
         if (MODE == K_INIT) {

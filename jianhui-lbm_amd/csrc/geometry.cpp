@@ -97,69 +97,140 @@ bool pores_wrap_along(const SparseGeometry &g, int axis)
     });
 }
 
+namespace {
+
+// link_column, column_link and edge_slot (lattice.h) as tables
+struct ColumnTables {
+    int column[Q] = {}, slot[Q] = {}, at[NCOL + 1] = {}, below[NCOL + 1] = {}, above[NCOL + 1] = {};
+    constexpr ColumnTables()
+    {
+        for (int q = 1; q < Q; ++q) {
+            column[q] = link_column(q);
+            slot[q] = edge_slot(q);
+        }
+        for (int c = 0; c <= NCOL; ++c) {
+            at[c] = column_link(c, 0);
+            below[c] = column_link(c, 1);
+            above[c] = column_link(c, -1);
+        }
+    }
+};
+constexpr ColumnTables COL;
+
+// Upstream word of node n in direction q from the packed form, as load_links decodes it.
+uint32_t unpack_link(const PackedNbr &p, int64_t P, int64_t n, int q)
+{
+    const uint32_t *h = &p.hdr[(size_t)((n >> 6) * HDR_WORDS)];
+    const int lane = (int)(n & 63);
+    auto mask = [h](int at) { return (uint64_t)h[at] | (uint64_t)h[at + 1] << 32; };
+    if (mask(HDR_MASK + 2 * (q - 1)) >> lane & 1) return (uint32_t)n | BB_FLAG;
+    if (h[HDR_WIDE] != HDR_COMPACT) return p.wide[(size_t)(((int64_t)h[HDR_WIDE] * 18 + q - 1) * 64 + lane)];
+    const uint64_t edge = mask(HDR_EDGE);
+    if (EZ[q] != 0 && (edge >> lane & 1)) {
+        const int64_t rec = (int64_t)h[HDR_EDGE_BASE] + __builtin_popcountll(edge & ((1ull << lane) - 1));
+        return p.edge[(size_t)(rec * EDGE_WORDS + COL.slot[q])];
+    }
+    const int c = COL.column[q];
+    if (c == NCOL) return (uint32_t)(n - EZ[q]);
+    const uint32_t r = h[c] + p.res[(size_t)(((c / 4) * P + n) * 4 + c % 4)];
+    if (EZ[q] == 0) return r;
+    return EZ[q] > 0 ? r - 1 : r + (mask(HDR_MASK + 2 * (COL.at[c] - 1)) >> lane & 1 ? 0u : 1u);
+}
+
+}  // namespace
+
 int pack_neighbours(const SparseGeometry &g, PackedNbr &out, std::string &err)
 {
     const int64_t P = g.P, N = g.N, W = P / 64;
-    out.res.assign((size_t)(18 * P), RES_BB);
+    out.res.assign((size_t)(NCOL * P), 0u);
     out.hdr.assign((size_t)(W * HDR_WORDS), 0u);
-    std::vector<uint8_t> is_wide((size_t)W, 0);
-    // bases and the compact/wide decision per wave
+    auto link = [&g, P](int64_t n, int q) { return g.nbr[(size_t)((q - 1) * P + n)]; };
+    auto none = [](uint32_t v) { return (v & BB_FLAG) != 0; };
+    // the upstream sites of column c around the node: at its height, one below, one above (an xy
+    // diagonal has the first only, the node's own column the other two)
+    auto column = [&](int64_t n, int c, uint32_t &at, uint32_t &below, uint32_t &above) {
+        at = COL.at[c] ? link(n, COL.at[c]) : (uint32_t)n;
+        below = COL.below[c] ? link(n, COL.below[c]) : BB_FLAG;
+        above = COL.above[c] ? link(n, COL.above[c]) : BB_FLAG;
+    };
+    // per node and column the rank (the number of pore voxels before the site at the node's
+    // height), from which the three sites' ids follow unless the column wraps round in z there
+    auto rank = [&](uint32_t at, uint32_t below, uint32_t above) {
+        return !none(at) ? at : !none(below) ? below + 1 : above;
+    };
 #pragma omp parallel for schedule(static)
     for (int64_t w = 0; w < W; ++w) {
         const int64_t n0 = w * 64, n1 = std::min(n0 + 64, N);
         uint32_t *h = &out.hdr[(size_t)(w * HDR_WORDS)];
+        auto set = [h](int at, int64_t lane) { h[at + (lane >> 5)] |= 1u << (lane & 31); };
+        auto solid = [&](uint32_t v, int q, int64_t lane) {
+            if (none(v) && q) set(HDR_MASK + 2 * (q - 1), lane);
+        };
         bool wide = false;
-        for (int q = 0; q < 18; ++q) {
-            uint32_t lo = 0xFFFFFFFFu, hi = 0;
+        for (int c = 0; c <= NCOL; ++c) {
+            uint32_t lo = 0xFFFFFFFFu, hi = 0, at, below, above;
             for (int64_t n = n0; n < n1; ++n) {
-                const uint32_t v = g.nbr[(size_t)(q * P + n)];
-                if (v & BB_FLAG) continue;
-                lo = std::min(lo, v);
-                hi = std::max(hi, v);
+                column(n, c, at, below, above);
+                solid(at, COL.at[c], n - n0);
+                solid(below, COL.below[c], n - n0);
+                solid(above, COL.above[c], n - n0);
+                if (none(at) && none(below) && none(above)) continue;
+                const uint32_t r = rank(at, below, above);
+                if ((!none(below) && below != r - 1) || (!none(above) && above != r + !none(at)))
+                    set(HDR_EDGE, n - n0);
+                lo = std::min(lo, r);
+                hi = std::max(hi, r);
             }
-            if (lo == 0xFFFFFFFFu) lo = hi = 0;   // no fluid upstream in this direction
-            h[q] = lo;
-            if (hi - lo >= (uint32_t)RES_BB) wide = true;
+            if (c == NCOL || lo == 0xFFFFFFFFu) continue;   // the own column needs no ranks
+            h[c] = lo;
+            wide |= hi - lo > 0xFFFFu;
         }
-        is_wide[(size_t)w] = wide;
+        h[HDR_WIDE] = wide ? 0u : HDR_COMPACT;
     }
-    int64_t nw = 0;
+    int64_t nw = 0, ne = 0;
     for (int64_t w = 0; w < W; ++w) {
         uint32_t *h = &out.hdr[(size_t)(w * HDR_WORDS)];
-        h[HDR_WIDE] = is_wide[(size_t)w] ? (uint32_t)nw++ : HDR_COMPACT;
-        h[HDR_WIDE + 1] = 0;
+        if (h[HDR_WIDE] != HDR_COMPACT) {
+            h[HDR_WIDE] = (uint32_t)nw++;
+            continue;
+        }
+        h[HDR_EDGE_BASE] = (uint32_t)ne;
+        ne += __builtin_popcount(h[HDR_EDGE]) + __builtin_popcount(h[HDR_EDGE + 1]);
     }
     out.n_wide = nw;
+    out.n_edge = ne;
     out.wide.assign((size_t)(nw * 18 * 64), 0u);
+    out.edge.assign((size_t)(ne * EDGE_WORDS), 0u);
 #pragma omp parallel for schedule(static)
     for (int64_t w = 0; w < W; ++w) {
         const int64_t n0 = w * 64, n1 = std::min(n0 + 64, N);
         const uint32_t *h = &out.hdr[(size_t)(w * HDR_WORDS)];
-        for (int q = 0; q < 18; ++q)
-            for (int64_t n = n0; n < n1; ++n) {
-                const uint32_t v = g.nbr[(size_t)(q * P + n)];
-                if (h[HDR_WIDE] != HDR_COMPACT)
-                    out.wide[(size_t)(((int64_t)h[HDR_WIDE] * 18 + q) * 64 + (n - n0))] = v;
-                else if (!(v & BB_FLAG))
-                    out.res[(size_t)(q * P + n)] = (uint16_t)(v - h[q]);
+        if (h[HDR_WIDE] != HDR_COMPACT) {
+            for (int q = 1; q < Q; ++q)
+                for (int64_t n = n0; n < n1; ++n)
+                    out.wide[(size_t)(((int64_t)h[HDR_WIDE] * 18 + q - 1) * 64 + (n - n0))] = link(n, q) & ~BB_FLAG;
+            continue;
+        }
+        uint32_t rec = h[HDR_EDGE_BASE];
+        for (int64_t n = n0; n < n1; ++n) {
+            for (int c = 0; c < NCOL; ++c) {
+                uint32_t at, below, above;
+                column(n, c, at, below, above);
+                if (none(at) && none(below) && none(above)) continue;
+                out.res[(size_t)(((c / 4) * P + n) * 4 + c % 4)] = (uint16_t)(rank(at, below, above) - h[c]);
             }
+            if (h[HDR_EDGE + ((n - n0) >> 5)] >> ((n - n0) & 31) & 1) {
+                for (int q = 1; q < Q; ++q)
+                    if (EZ[q] != 0) out.edge[(size_t)((int64_t)rec * EDGE_WORDS + COL.slot[q])] = link(n, q) & ~BB_FLAG;
+                ++rec;
+            }
+        }
     }
     // decode everything as the device does and compare
     int64_t bad = 0;
 #pragma omp parallel for schedule(static) reduction(+ : bad)
-    for (int64_t n = 0; n < N; ++n) {
-        const uint32_t *h = &out.hdr[(size_t)((n >> 6) * HDR_WORDS)];
-        for (int q = 0; q < 18; ++q) {
-            uint32_t v;
-            if (h[HDR_WIDE] == HDR_COMPACT) {
-                const uint16_t r = out.res[(size_t)(q * P + n)];
-                v = r == RES_BB ? ((uint32_t)n | BB_FLAG) : h[q] + r;
-            } else {
-                v = out.wide[(size_t)(((int64_t)h[HDR_WIDE] * 18 + q) * 64 + (n & 63))];
-            }
-            bad += v != g.nbr[(size_t)(q * P + n)];
-        }
-    }
+    for (int64_t n = 0; n < N; ++n)
+        for (int q = 1; q < Q; ++q) bad += unpack_link(out, P, n, q) != link(n, q);
     if (bad) {
         err = "neighbour table packing failed its decode check (" + std::to_string(bad) + " entries)";
         return LBM_ERR_STATE;
@@ -170,20 +241,17 @@ int pack_neighbours(const SparseGeometry &g, PackedNbr &out, std::string &err)
 hipError_t DeviceNbr::upload(const PackedNbr &p, int64_t P, hipStream_t s)
 {
     release();
-    n_wide = p.n_wide;
-    const size_t b_res = (size_t)18 * P * sizeof(uint16_t), b_hdr = p.hdr.size() * sizeof(uint32_t);
-    const size_t b_wide = std::max<size_t>(p.wide.size(), 1) * sizeof(uint32_t);
-    bytes = b_res + b_hdr + b_wide;
+    const size_t b_res = (size_t)NCOL * P * sizeof(uint16_t), b_hdr = p.hdr.size() * sizeof(uint32_t);
+    const size_t b_edge = p.edge.size() * sizeof(uint32_t), b_wide = p.wide.size() * sizeof(uint32_t);
     hipError_t e;
     if ((e = hipMalloc(&res, b_res)) != hipSuccess) return e;
     if ((e = hipMalloc(&hdr, b_hdr)) != hipSuccess) return e;
-    if ((e = hipMalloc(&wide, b_wide)) != hipSuccess) return e;
+    if ((e = hipMalloc(&edge, std::max<size_t>(b_edge, 16))) != hipSuccess) return e;
+    if ((e = hipMalloc(&wide, std::max<size_t>(b_wide, 16))) != hipSuccess) return e;
     if ((e = hipMemcpyAsync(res, p.res.data(), b_res, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
     if ((e = hipMemcpyAsync(hdr, p.hdr.data(), b_hdr, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
-    if (!p.wide.empty() &&
-        (e = hipMemcpyAsync(wide, p.wide.data(), p.wide.size() * sizeof(uint32_t), hipMemcpyHostToDevice, s)) !=
-            hipSuccess)
-        return e;
+    if (b_edge && (e = hipMemcpyAsync(edge, p.edge.data(), b_edge, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
+    if (b_wide && (e = hipMemcpyAsync(wide, p.wide.data(), b_wide, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
     return hipSuccess;
 }
 
@@ -191,9 +259,8 @@ void DeviceNbr::release()
 {
     if (res) (void)hipFree(res), res = nullptr;
     if (hdr) (void)hipFree(hdr), hdr = nullptr;
+    if (edge) (void)hipFree(edge), edge = nullptr;
     if (wide) (void)hipFree(wide), wide = nullptr;
-    n_wide = 0;
-    bytes = 0;
 }
 
 }  // namespace lbm

@@ -66,19 +66,24 @@ bool pores_wrap_along(const SparseGeometry &g, int axis);
 // Round up to a multiple of the block size so every direction row starts 256-byte aligned.
 inline int64_t padded_stride(int64_t n) { return ((n + 255) / 256) * 256; }
 
-// Device form of the neighbour lists (decoded by load_nbr in nbrpack.h): per wavefront of 64
-// node ids and direction, a 32-bit base and 16-bit residuals; waves whose spread does not fit
-// keep their full words in a side table.
-constexpr int HDR_WORDS = 20;                  // per wave: 18 bases, wide slot, pad
-constexpr int HDR_WIDE = 18;
-constexpr uint16_t RES_BB = 0xFFFF;            // residual of a bounce-back link
+// Device form of the neighbour lists (decoded by load_links in nbrpack.h): per wavefront of 64
+// node ids one header with a base per neighbour column and a solid mask per direction, and per
+// node and column one 16-bit rank.
+constexpr int NCOL = 8;                        // neighbour columns (x - ex, y - ey), own one apart
+constexpr int HDR_WORDS = 48;                  // 32-bit words per wave
+constexpr int HDR_MASK = 8;                    // after the NCOL bases: 18 64-bit solid masks
+constexpr int HDR_EDGE = 44;                   // 64-bit mask of the edge lanes
+constexpr int HDR_EDGE_BASE = 46;              // index of the wave's first edge record
+constexpr int HDR_WIDE = 47;                   // wide slot
 constexpr uint32_t HDR_COMPACT = 0xFFFFFFFFu;  // wide slot of a compact wave
+constexpr int EDGE_WORDS = 12;                 // an edge record: the 10 directions with e_z != 0, padded
 
 struct PackedNbr {
-    std::vector<uint16_t> res;    // 18 x P
+    std::vector<uint16_t> res;    // 2 x P x 4: ranks in columns 0-3 (axis) and 4-7 (xy diagonals)
     std::vector<uint32_t> hdr;    // (P / 64) x HDR_WORDS
+    std::vector<uint32_t> edge;   // n_edge x EDGE_WORDS
     std::vector<uint32_t> wide;   // n_wide x 18 x 64
-    int64_t n_wide = 0;
+    int64_t n_wide = 0, n_edge = 0;
 };
 
 // Pack g.nbr, then decode every entry and compare with the full table (LBM_ERR_STATE if any
@@ -86,21 +91,21 @@ struct PackedNbr {
 int pack_neighbours(const SparseGeometry &g, PackedNbr &out, std::string &err);
 
 struct NbrDev {
-    const uint16_t *__restrict__ res;   // 18 x P
+    const uint2 *__restrict__ res;      // 2 x P: four 16-bit ranks each
     const uint32_t *__restrict__ hdr;   // (P / 64) x HDR_WORDS
+    const uint4 *__restrict__ edge;     // n_edge x EDGE_WORDS / 4
     const uint32_t *__restrict__ wide;  // n_wide x 18 x 64
 };
 
 // Owner of the packed table in device memory.
 struct DeviceNbr {
-    uint16_t *res = nullptr;
+    uint2 *res = nullptr;
+    uint4 *edge = nullptr;
     uint32_t *hdr = nullptr, *wide = nullptr;
-    int64_t n_wide = 0;
-    size_t bytes = 0;
     // allocate and queue the copies on s; p must stay alive until s has been synchronised
     hipError_t upload(const PackedNbr &p, int64_t P, hipStream_t s);
     void release();
-    NbrDev view() const { return NbrDev{res, hdr, wide}; }
+    NbrDev view() const { return NbrDev{res, hdr, edge, wide}; }
 };
 
 // Face boundaries (lbm_sp_set_boundaries).  Every fluid node on an active face gets one

@@ -30,6 +30,30 @@ constexpr int opp(int q)
 constexpr int NPAIR = 9;
 constexpr int PA[NPAIR] = {1, 3, 5, 7, 8, 11, 12, 15, 16};
 
+// Neighbour columns: the upstream site x - e_q lies in the column of voxels at (x - ex, y - ey).
+// Columns 0-3 hold the axis links q = 1..4 and the xz / yz diagonals above and below them, columns
+// 4-7 the xy diagonals q = 7..10; column 8 is the node's own.
+constexpr int link_column(int q)
+{
+    for (int r = 1; r <= 10; ++r)
+        if (EZ[r] == 0 && EX[r] == EX[q] && EY[r] == EY[q]) return r <= 4 ? r - 1 : r - 3;
+    return 8;
+}
+// the direction of column c with z component ez (0 if the lattice has none)
+constexpr int column_link(int c, int ez = 0)
+{
+    for (int r = 1; r < 19; ++r)
+        if (EZ[r] == ez && link_column(r) == c) return r;
+    return 0;
+}
+// the place of a direction with e_z != 0 in an edge record (nbrpack.h): the own column first
+constexpr int edge_slot(int q)
+{
+    int s = 0;
+    for (int r = 5; r < q; ++r) s += EZ[r] != 0;
+    return s;
+}
+
 // lattice weight as a rational number: 1/3, 1/18, 1/36
 constexpr int e2_of(int q) { return EX[q] * EX[q] + EY[q] * EY[q] + EZ[q] * EZ[q]; }
 constexpr double weight(int q) { return e2_of(q) == 0 ? 1.0 / 3.0 : (e2_of(q) == 1 ? 1.0 / 18.0 : 1.0 / 36.0); }

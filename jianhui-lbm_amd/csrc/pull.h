@@ -2,10 +2,9 @@
 //
 // Population q of node n after streaming is the post-collision population q of the upstream
 // node n - e_q, or -- when that site is solid -- the post-collision population opp(q) of n
-// itself (halfway bounce-back).  The neighbour table gives, per moving direction q = 1..18
-// and node, the upstream node index with BB_FLAG set for the bounce-back case (decoded from
-// its packed device form by load_nbr), so each load is one select and one gather; the rest
-// population needs no index.
+// itself (halfway bounce-back).  The links of a node (load_links) give, per moving direction
+// q = 1..18, the upstream node and whether its site is solid, so each load is one select and
+// one gather; the rest population needs no link.
 #pragma once
 #include "collide.h"
 #include "lattice.h"
@@ -16,12 +15,34 @@ namespace lbm {
 
 enum KMode { K_INIT = 0, K_DIRECT = 1, K_PULL = 2 };
 
+// Element offset of population q of node n after streaming in rows of stride P.
+template <int K>
+__device__ __forceinline__ int64_t pull_offset(const Links<K> &l, int64_t P, int64_t n, int q)
+{
+    return (l.solid(q) ? (int64_t)opp(q) * P : (int64_t)q * P) + (l.solid(q) ? n : (int64_t)l.up[q - 1]);
+}
+
+// load(q) for the links of node n, the ones at the node's height first: an edge lane's others wait
+// for its record.
+template <int K, typename F>
+__device__ __forceinline__ void gather_links(const NbrDev &nbr, int64_t P, int64_t n, Links<K> &l, F &&load)
+{
+    level_links(nbr, P, n, l);
+#pragma unroll
+    for (int q = 1; q <= K; ++q)
+        if (EZ[q] == 0) load(q);
+    wrap_links(nbr, n, l);
+#pragma unroll
+    for (int q = 1; q <= K; ++q)
+        if (EZ[q] != 0) load(q);
+}
+
 // Gather the 19 pre-collision deviations of node n.  In K_DIRECT mode the buffer holds a
-// post-streaming state (a loaded checkpoint) and is read in place.  The 18 neighbour words
-// are returned in nb (K_PULL only) for callers that also need the neighbour sites.
+// post-streaming state (a loaded checkpoint) and is read in place.  The node's links are
+// returned in l (K_PULL only) for callers that also need the neighbour sites.
 template <typename ST, int MODE>
 __device__ __forceinline__ void gather_pops(const ST *__restrict__ src, const NbrDev &nbr, int64_t P, int64_t n,
-                                            float inv_scale, typename Store<ST>::C (&h)[Q], uint32_t (&nb)[Q - 1])
+                                            float inv_scale, typename Store<ST>::C (&h)[Q], Links<Q - 1> &l)
 {
     h[0] = Store<ST>::load(src[n], inv_scale);
     if (MODE == K_DIRECT) {
@@ -29,13 +50,7 @@ __device__ __forceinline__ void gather_pops(const ST *__restrict__ src, const Nb
         for (int q = 1; q < Q; ++q) h[q] = Store<ST>::load(src[(int64_t)q * P + n], inv_scale);
         return;
     }
-    load_nbr(nbr, P, n, nb);
-#pragma unroll
-    for (int q = 1; q < Q; ++q) {
-        const uint32_t v = nb[q - 1];
-        const int64_t row = (v & BB_FLAG) ? (int64_t)opp(q) : (int64_t)q;
-        h[q] = Store<ST>::load(src[row * P + (int64_t)(v & ~BB_FLAG)], inv_scale);
-    }
+    gather_links(nbr, P, n, l, [&](int q) { h[q] = Store<ST>::load(src[pull_offset(l, P, n, q)], inv_scale); });
 }
 
 }  // namespace lbm

@@ -9,8 +9,8 @@
 //
 // Data layout in HBM (structure of arrays, row stride P = N rounded up to 256):
 //   pops[2]  19 x P  storage type (double / float / half), deviations f - w*rho0
-//   nbr      packed upstream node of direction q = 1..18 or bounce back (nbrpack.h):
-//            18 x P uint16 residuals + per-wave 32-bit bases
+//   nbr      packed upstream node of direction q = 1..18 or bounce back (nbrpack.h): 8 x P
+//            uint16 column ranks + a header per wave
 //   u_aux     3 x P  compute type, u of the previous step (for the Error diagnostic)
 //   rho_aux   1 x P  compute type, density of a loaded checkpoint (first step only)
 #include <algorithm>
@@ -94,8 +94,8 @@ __device__ __forceinline__ void power_law_rates(const C (&h)[Q], const Macro<C> 
 template <typename ST, int MODE>
 __device__ __forceinline__ void gather(const SpArgs<ST> &a, int64_t n, typename Store<ST>::C (&h)[Q])
 {
-    uint32_t nb[Q - 1];
-    gather_pops<ST, MODE>(a.src, a.nbr, a.P, n, a.inv_scale, h, nb);
+    Links<Q - 1> l;
+    gather_pops<ST, MODE>(a.src, a.nbr, a.P, n, a.inv_scale, h, l);
 }
 
 template <typename ST, int MODE>
@@ -144,8 +144,8 @@ __global__ void __launch_bounds__(NB) sp_step_kernel(SpArgs<ST> a)
             bc_save(a.bc, n, h, mc.drho, mc.ux, mc.uy, mc.uz);
         }
     } else {
-        uint32_t nb[Q - 1];
-        gather_pops<ST, MODE>(a.src, a.nbr, a.P, n, a.inv_scale, h, nb);
+        Links<Q - 1> l;
+        gather_pops<ST, MODE>(a.src, a.nbr, a.P, n, a.inv_scale, h, l);
         if (BC && MODE == K_PULL) bc_patch(a.bc, n, a.rho0, h);
         moments_fwd(h, m);
         mc = node_macro<ST, MODE>(a, n, m);
@@ -154,11 +154,7 @@ __global__ void __launch_bounds__(NB) sp_step_kernel(SpArgs<ST> a)
             C g[7];
             g[0] = a.st.src[n];
 #pragma unroll
-            for (int q = 1; q < 7; ++q) {
-                const uint32_t v = nb[q - 1];
-                const int64_t row = (v & BB_FLAG) ? (int64_t)opp(q) : (int64_t)q;
-                g[q] = a.st.src[row * a.P + (int64_t)(v & ~BB_FLAG)];
-            }
+            for (int q = 1; q < 7; ++q) g[q] = a.st.src[pull_offset(l, a.P, n, q)];
             C c = g[0];
 #pragma unroll
             for (int q = 1; q < 7; ++q) c += g[q];
@@ -202,7 +198,7 @@ struct DiagBox {
 // Sums over the nodes n_lo <= n < n_hi (all nodes, or one reference rank's share of them for
 // Error over ranks); the Error terms skip the range's last node.  The launch covers the range
 // from the 64-aligned node below n_lo, so that every wavefront stays within one 64-node group of
-// the packed neighbour table (load_nbr); lanes before n_lo only add zeros.
+// the packed neighbour table (load_links); lanes before n_lo only add zeros.
 template <typename ST, int MODE>
 __global__ void __launch_bounds__(BLOCK) sp_diag_kernel(SpArgs<ST> a, const int32_t *__restrict__ supinv,
                                                         DiagBox box, int64_t n_lo, int64_t n_hi,
@@ -255,7 +251,7 @@ __global__ void __launch_bounds__(BLOCK) sp_diag_kernel(SpArgs<ST> a, const int3
 
 // Sums of u and node counts per cube of a cube grid (Comput_Grop_Perm, SP:4886-5090), one
 // workgroup per cube.  A cube's nodes are listed as entries (64-node group, lane mask); a wave
-// takes one entry at a time, so its active lanes always lie in one group (as load_nbr and
+// takes one entry at a time, so its active lanes always lie in one group (as load_links and
 // bc_patch require).  Each thread sums its nodes in a fixed order and the block reduction has a
 // fixed tree: the sums are the same on every call.
 template <typename ST, int MODE>

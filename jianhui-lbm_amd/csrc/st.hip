@@ -61,14 +61,8 @@ __device__ __forceinline__ void st_gather(const StArgs<C> &a, int64_t n, C (&g)[
         for (int q = 1; q < Q7; ++q) g[q] = a.src[(int64_t)q * a.P + n];
         return;
     }
-    uint32_t nb[6];
-    load_nbr_first<6>(a.nbr, a.P, n, nb);
-#pragma unroll
-    for (int q = 1; q < Q7; ++q) {
-        const uint32_t v = nb[q - 1];
-        const int64_t row = (v & BB_FLAG) ? (int64_t)opp(q) : (int64_t)q;
-        g[q] = a.src[row * a.P + (int64_t)(v & ~BB_FLAG)];
-    }
+    Links<6> l;
+    gather_links(a.nbr, a.P, n, l, [&](int q) { g[q] = a.src[pull_offset(l, a.P, n, q)]; });
 }
 
 template <typename C, int MODE, int NB = BLOCK>
@@ -106,7 +100,7 @@ template <typename C, int MODE>
 __global__ void __launch_bounds__(BLOCK) st_get_state_kernel(StArgs<C> a, int64_t n0, int64_t n1,
                                                              double *__restrict__ g_out, double *__restrict__ c_out)
 {
-    const int64_t n = group_floor(n0) + (int64_t)blockIdx.x * BLOCK + threadIdx.x;   // see load_nbr
+    const int64_t n = group_floor(n0) + (int64_t)blockIdx.x * BLOCK + threadIdx.x;   // see load_links
     if (n < n0 || n >= n1) return;
     const int64_t l = n - n0;
     C g[Q7];

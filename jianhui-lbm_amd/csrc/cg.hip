@@ -15,7 +15,8 @@
 //                     pull form sums the same terms without atomics, in a fixed order.
 //
 // Data layout (row stride P):
-//   pops[2] 19 x P  deviations f - w rho0, canonical (SP) velocity order
+//   pops[2] 19 x P  deviations f - w rho0, canonical (SP) velocity order, in blocks of 256 nodes
+//                   (pop_at, lattice.h)
 //   nbr     packed upstream node per direction or bounce back (nbrpack.h)
 //   col      2 x P  rho_r, rho_b after colour streaming (the reference's rho_r/rho_b): doubles in
 //                   the FP64 build, int32 fixed point (units of 2^-29) in the FP32 build
@@ -133,9 +134,9 @@ __device__ __forceinline__ void cg_node_state(const CgArgs<ST> &a, int64_t n, ty
         sp_eq_moments(mc, m);   // f = M^-1 meq(1, u0) = feq(1, u0) (CG:2644-2681)
         return;
     }
-    h[0] = Store<ST>::load(a.src[n], a.inv_scale);
+    h[0] = Store<ST>::load(a.src[pop_at<Q>(0, n)], a.inv_scale);
     gather_links(a.nbr, a.P, n, l, [&](int q) {
-        h[q] = Store<ST>::load(a.src[MODE == K_DIRECT ? (int64_t)q * a.P + n : pull_offset(l, a.P, n, q)], a.inv_scale);
+        h[q] = Store<ST>::load(a.src[MODE == K_DIRECT ? pop_at<Q>(q, n) : pull_offset<Q>(l, n, q)], a.inv_scale);
     });
     moments_fwd(h, m);
     if (MODE == K_DIRECT) {
@@ -219,7 +220,7 @@ __device__ __forceinline__ void cg_collide_node(const CgArgs<ST> &a, int64_t n, 
     }
     cg_relax(m, mc, gx, gy, gz, sv, a.cap_a * cc, nx, ny, nz, h);
 #pragma unroll
-    for (int q = 0; q < Q; ++q) Store<ST>::store_nt(&a.dst[(int64_t)q * a.P + n], h[q], a.scale);
+    for (int q = 0; q < Q; ++q) Store<ST>::store_nt(&a.dst[pop_at<Q>(q, n)], h[q], a.scale);
     const C st[6] = {mc.ux, mc.uy, mc.uz, nx, ny, nz};
     store_cs(a.cs, n, a.P, rr_raw, rb_raw, st);
 }
@@ -794,7 +795,7 @@ __global__ void __launch_bounds__(BLOCK) cg_load_state_kernel(CgArgs<ST> a, int6
 #pragma unroll
     for (int qc = 0; qc < Q; ++qc) {
         const int q = cg_to_canon(qc);
-        a.dst[(int64_t)q * a.P + n] = Store<ST>::put((C)(f[l * Q + qc] - weight(q) * (double)a.rho0), a.scale);
+        a.dst[pop_at<Q>(q, n)] = Store<ST>::put((C)(f[l * Q + qc] - weight(q) * (double)a.rho0), a.scale);
     }
     for (int c = 0; c < 3; ++c) a.u_aux[(int64_t)c * a.P + n] = (C)u[l * 3 + c];
     rho_aux[n] = (C)rho[l];

@@ -111,6 +111,21 @@ constexpr int cg_to_canon(int qc)
     return -1;
 }
 
+// Element offset of population q of node n in a buffer of NQ populations a node.  Nodes are stored
+// in blocks of POP_BLOCK, all NQ rows of a block together: a workgroup then reads and writes a
+// few stretches of 19 kB (FP32) each, where NQ rows of the whole box were 2 NQ streams far apart,
+// in as many DRAM pages and address translations.  A gather touches the same cache lines in
+// either layout.  Step on device with rows -> blocks of 64 / 256 / 512 nodes: 256^3 sphere pack FP32
+// 187.8 -> 176.2 / 175.9 / 175.4 us, 171 x 203 x 187 FP64 117.6 -> 109.9 / 109.9 / 109.7 us, 192^3
+// fibres with solute FP32 247.0 -> 220.9 / 219.6 / 220.9 us, colour gradient 192^3 FP32 224.3 ->
+// 217.9 / 217.0 / 219.7 us, 64^3 FP64 13.5 -> 13.2 / 13.1 / 13.3 us; 256 divides the padded node count.
+constexpr int POP_BLOCK = 256;
+template <int NQ>
+constexpr int64_t pop_at(int q, uint32_t n)
+{
+    return (int64_t)((uint64_t)(n / POP_BLOCK) * uint32_t((NQ - 1) * POP_BLOCK) + n + uint32_t(q * POP_BLOCK));
+}
+
 // upstream-index encoding: bit 31 set = the upstream site is solid, read the opposite
 // population of this node instead (halfway bounce-back)
 constexpr uint32_t BB_FLAG = 0x80000000u;

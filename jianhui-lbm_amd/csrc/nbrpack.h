@@ -67,13 +67,8 @@ __device__ __forceinline__ void level_links(const NbrDev &d, int64_t P, int64_t 
     for (int q = 1; q <= K; ++q) l.bb[q - 1] = reinterpret_cast<const uint64_t *>(h + HDR_MASK)[q - 1];
     l.edge = reinterpret_cast<const uint64_t *>(h + HDR_EDGE)[0];
     const uint32_t slot = h[HDR_WIDE];
-    if (slot != HDR_COMPACT) {
-        const uint32_t *__restrict__ wp = d.wide + (int64_t)slot * (18 * 64) + (n & 63);
-#pragma unroll
-        for (int q = 1; q <= K; ++q) l.up[q - 1] = wp[(q - 1) * 64];
-        l.edge = 0;
-        return;
-    }
+    // decoded whether the wave is compact or not: in an else branch, the rank loads would be
+    // issued only when the header has arrived
 #pragma unroll
     for (int q = 1; q <= K; ++q) {
         const int c = link_column(q);
@@ -83,6 +78,12 @@ __device__ __forceinline__ void level_links(const NbrDev &d, int64_t P, int64_t 
             const uint32_t at = h[c] + r[c];
             l.up[q - 1] = EZ[q] == 0 ? at : EZ[q] > 0 ? at - 1 : at + (l.solid(column_link(c)) ? 0u : 1u);
         }
+    }
+    if (slot != HDR_COMPACT) {
+        const uint32_t *__restrict__ wp = d.wide + (int64_t)slot * (18 * 64) + (n & 63);
+#pragma unroll
+        for (int q = 1; q <= K; ++q) l.up[q - 1] = wp[(q - 1) * 64];
+        l.edge = 0;
     }
 }
 

@@ -15,11 +15,14 @@ namespace lbm {
 
 enum KMode { K_INIT = 0, K_DIRECT = 1, K_PULL = 2 };
 
-// Element offset of population q of node n after streaming in rows of stride P.
-template <int K>
-__device__ __forceinline__ int64_t pull_offset(const Links<K> &l, int64_t P, int64_t n, int q)
+// Element offset of population q of node n after streaming, in a buffer of NQ a node: the node and
+// the row are selected, not the offsets, which the compiler would compute in divergent branches.
+template <int NQ, int K>
+__device__ __forceinline__ int64_t pull_offset(const Links<K> &l, int64_t n, int q)
 {
-    return (l.solid(q) ? (int64_t)opp(q) * P : (int64_t)q * P) + (l.solid(q) ? n : (int64_t)l.up[q - 1]);
+    const uint32_t at = l.solid(q) ? (uint32_t)n : l.up[q - 1];
+    const uint32_t row = l.solid(q) ? uint32_t(opp(q) * POP_BLOCK) : uint32_t(q * POP_BLOCK);
+    return (int64_t)((uint64_t)(at / POP_BLOCK) * uint32_t((NQ - 1) * POP_BLOCK) + (at + row));
 }
 
 // load(q) for the links of node n, the ones at the node's height first: an edge lane's others wait
@@ -44,13 +47,13 @@ template <typename ST, int MODE>
 __device__ __forceinline__ void gather_pops(const ST *__restrict__ src, const NbrDev &nbr, int64_t P, int64_t n,
                                             float inv_scale, typename Store<ST>::C (&h)[Q], Links<Q - 1> &l)
 {
-    h[0] = Store<ST>::load(src[n], inv_scale);
+    h[0] = Store<ST>::load(src[pop_at<Q>(0, n)], inv_scale);
     if (MODE == K_DIRECT) {
 #pragma unroll
-        for (int q = 1; q < Q; ++q) h[q] = Store<ST>::load(src[(int64_t)q * P + n], inv_scale);
+        for (int q = 1; q < Q; ++q) h[q] = Store<ST>::load(src[pop_at<Q>(q, n)], inv_scale);
         return;
     }
-    gather_links(nbr, P, n, l, [&](int q) { h[q] = Store<ST>::load(src[pull_offset(l, P, n, q)], inv_scale); });
+    gather_links(nbr, P, n, l, [&](int q) { h[q] = Store<ST>::load(src[pull_offset<Q>(l, n, q)], inv_scale); });
 }
 
 }  // namespace lbm

@@ -7,8 +7,9 @@
 // post-collision populations, coalesced, to the other buffer.  The stored state is therefore
 // post-collision; the reference's post-streaming state is the pull of it (get_state).
 //
-// Data layout in HBM (structure of arrays, row stride P = N rounded up to 256):
-//   pops[2]  19 x P  storage type (double / float / half), deviations f - w*rho0
+// Data layout in HBM (row stride P = N rounded up to 256):
+//   pops[2]  19 x P  storage type (double / float / half), deviations f - w*rho0, in blocks of
+//            256 nodes (pop_at, lattice.h)
 //   nbr      packed upstream node of direction q = 1..18 or bounce back (nbrpack.h): 8 x P
 //            uint16 column ranks + a header per wave
 //   u_aux     3 x P  compute type, u of the previous step (for the Error diagnostic)
@@ -152,19 +153,19 @@ __global__ void __launch_bounds__(NB) sp_step_kernel(SpArgs<ST> a)
         if (BC) bc_save(a.bc, n, h, mc.drho, mc.ux, mc.uy, mc.uz);
         if (FUSED && MODE == K_PULL) {
             C g[7];
-            g[0] = a.st.src[n];
+            g[0] = a.st.src[pop_at<7>(0, n)];
 #pragma unroll
-            for (int q = 1; q < 7; ++q) g[q] = a.st.src[pull_offset(l, a.P, n, q)];
+            for (int q = 1; q < 7; ++q) g[q] = a.st.src[pull_offset<7>(l, n, q)];
             C c = g[0];
 #pragma unroll
             for (int q = 1; q < 7; ++q) c += g[q];
             const C wc = a.st.wq * c;
-            __builtin_nontemporal_store(g[0] - a.st.omega * (g[0] - a.st.w0 * c), &a.st.dst[n]);
+            __builtin_nontemporal_store(g[0] - a.st.omega * (g[0] - a.st.w0 * c), &a.st.dst[pop_at<7>(0, n)]);
 #pragma unroll
             for (int q = 1; q < 7; ++q) {
                 const C eu = q == 1 ? mc.ux : q == 2 ? -mc.ux : q == 3 ? mc.uy : q == 4 ? -mc.uy : q == 5 ? mc.uz : -mc.uz;
                 const C eq = wc * (C(1) + eu * a.st.inv_cs2);
-                __builtin_nontemporal_store(g[q] - a.st.omega * (g[q] - eq), &a.st.dst[(int64_t)q * a.P + n]);
+                __builtin_nontemporal_store(g[q] - a.st.omega * (g[q] - eq), &a.st.dst[pop_at<7>(q, n)]);
             }
         }
     }
@@ -177,7 +178,7 @@ __global__ void __launch_bounds__(NB) sp_step_kernel(SpArgs<ST> a)
     if (PL && MODE == K_PULL) power_law_rates(h, mc, a.nu_vn, n, a.pl_m, a.pl_n, sv, sq);
     sp_relax(m, mc, a.gx, a.gy, a.gz, sv, sq, h);
 #pragma unroll
-    for (int q = 0; q < Q; ++q) Store<ST>::store_nt(&a.dst[(int64_t)q * a.P + n], h[q], a.scale);
+    for (int q = 0; q < Q; ++q) Store<ST>::store_nt(&a.dst[pop_at<Q>(q, n)], h[q], a.scale);
 }
 
 template <typename C>
@@ -342,7 +343,7 @@ __global__ void __launch_bounds__(BLOCK) sp_load_state_kernel(SpArgs<ST> a, int6
     const int64_t l = n - n0;
 #pragma unroll
     for (int q = 0; q < Q; ++q)
-        a.dst[(int64_t)q * a.P + n] = Store<ST>::put((typename Store<ST>::C)(f[l * Q + q] - weight(q) * (double)a.rho0),
+        a.dst[pop_at<Q>(q, n)] = Store<ST>::put((typename Store<ST>::C)(f[l * Q + q] - weight(q) * (double)a.rho0),
                                                     a.scale);
     for (int c = 0; c < 3; ++c) a.u_aux[(int64_t)c * a.P + n] = (typename Store<ST>::C)u[l * 3 + c];
     rho_aux[n] = (typename Store<ST>::C)rho[l];

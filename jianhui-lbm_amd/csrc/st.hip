@@ -12,7 +12,7 @@
 // the packed D3Q19 pull table are the D3Q7 links), relaxes and writes the post-collision
 // populations.  As in the flow kernels the stored state is post-collision; get_state pulls.
 //
-// Data layout (row stride P): pops[2] 7 x P, u 3 x P (the flow handle's when coupled),
+// Data layout (row stride P): pops[2] 7 x P in blocks of 256 nodes (pop_at), u 3 x P (the flow handle's when coupled),
 // c_init P (the concentration of an equilibrium start).
 #include <algorithm>
 #include <cmath>
@@ -55,14 +55,14 @@ __device__ __forceinline__ C axis_dot(int q, C ux, C uy, C uz)
 template <typename C, int MODE>
 __device__ __forceinline__ void st_gather(const StArgs<C> &a, int64_t n, C (&g)[Q7])
 {
-    g[0] = a.src[n];
+    g[0] = a.src[pop_at<Q7>(0, n)];
     if (MODE == K_DIRECT) {
 #pragma unroll
-        for (int q = 1; q < Q7; ++q) g[q] = a.src[(int64_t)q * a.P + n];
+        for (int q = 1; q < Q7; ++q) g[q] = a.src[pop_at<Q7>(q, n)];
         return;
     }
     Links<6> l;
-    gather_links(a.nbr, a.P, n, l, [&](int q) { g[q] = a.src[pull_offset(l, a.P, n, q)]; });
+    gather_links(a.nbr, a.P, n, l, [&](int q) { g[q] = a.src[pull_offset<Q7>(l, n, q)]; });
 }
 
 template <typename C, int MODE, int NB = BLOCK>
@@ -84,13 +84,13 @@ __global__ void __launch_bounds__(NB) st_step_kernel(StArgs<C> a, int32_t order)
     {
         const C eq = a.w0 * c;
         const C v = MODE == K_INIT ? eq : g[0] - a.omega * (g[0] - eq);
-        __builtin_nontemporal_store(v, &a.dst[n]);
+        __builtin_nontemporal_store(v, &a.dst[pop_at<Q7>(0, n)]);
     }
 #pragma unroll
     for (int q = 1; q < Q7; ++q) {
         const C eq = wc * (C(1) + axis_dot(q, ux, uy, uz) * a.inv_cs2);
         const C v = MODE == K_INIT ? eq : g[q] - a.omega * (g[q] - eq);
-        __builtin_nontemporal_store(v, &a.dst[(int64_t)q * a.P + n]);
+        __builtin_nontemporal_store(v, &a.dst[pop_at<Q7>(q, n)]);
     }
 }
 
@@ -129,7 +129,7 @@ __global__ void __launch_bounds__(BLOCK) st_load_state_kernel(StArgs<C> a, int64
     const int64_t n = n0 + (int64_t)blockIdx.x * BLOCK + threadIdx.x;
     if (n >= n1) return;
 #pragma unroll
-    for (int q = 0; q < Q7; ++q) a.dst[(int64_t)q * a.P + n] = (C)g_in[(n - n0) * Q7 + q];
+    for (int q = 0; q < Q7; ++q) a.dst[pop_at<Q7>(q, n)] = (C)g_in[(n - n0) * Q7 + q];
 }
 
 // mass, min, max, first and second moments, non-finite count (FP64, fixed reduction order)

@@ -1260,22 +1260,13 @@ int CgSolver::step(int nsteps, double *elapsed_ms)
 int CgSolver::get_state(double *f, double *u, double *rho, double *psi, double *rr, double *rb)
 {
     if (mode_ == STATE_EMPTY) return fail(LBM_ERR_STATE, "state not initialised");
-    double *outs[6] = {f, u, rho, psi, rr, rb};
-    const int width[6] = {Q, 3, 1, 1, 1, 1};
-    int per_node = 0;
-    for (int k = 0; k < 6; ++k) per_node += outs[k] ? width[k] : 0;
-    if (per_node == 0) return LBM_OK;
     LBM_HIP_TRY(hipSetDevice(device_));
     LBM_HIP_TRY(stage_.ensure());
-    const int64_t N = geo_.N, chunk = stage_chunk(STAGE_BYTES, per_node);
+    const int64_t N = geo_.N;
     const int mode = cg_kmode(mode_);
-    hipError_t e = hipSuccess;
-    for (int64_t n0 = 0; n0 < N && e == hipSuccess; n0 += chunk) {
-        const int64_t c = std::min(chunk, N - n0), n1 = n0 + c;
-        double *bufs[6] = {nullptr};
-        double *p = (double *)stage_.buf;
-        for (int k = 0; k < 6; ++k)
-            if (outs[k]) bufs[k] = p, p += c * width[k];
+    const ReadPart parts[6] = {{f, Q}, {u, 3}, {rho, 1}, {psi, 1}, {rr, 1}, {rb, 1}};
+    LBM_HIP_TRY(read_back(device_, stream_, N, parts, 6, stage_.buf, STAGE_BYTES, BLOCK,
+                          [&](int64_t n0, int64_t n1, double *const *bufs) {
         dim3 g((unsigned)((n1 - group_floor(n0) + BLOCK - 1) / BLOCK)), b(BLOCK);
         if (prm_.precision == LBM_FP64) {
             auto a = make_cg_args<double>(prm_, visc_, u_i_, pops_[cur_], nullptr, nbr_.view(), d_col_, d_psi_, d_cs_, d_u_,
@@ -1296,15 +1287,8 @@ int CgSolver::get_state(double *f, double *u, double *rho, double *psi, double *
             else
                 cg_get_state_kernel<float, K_PULL><<<g, b, 0, stream_>>>(a, n0, n1, bufs[0], bufs[1], bufs[2], bufs[3], bufs[4], bufs[5]);
         }
-        e = hipGetLastError();
-        for (int k = 0; k < 6 && e == hipSuccess; ++k)
-            if (outs[k])
-                e = hipMemcpyAsync(outs[k] + n0 * width[k], bufs[k], (size_t)c * width[k] * sizeof(double),
-                                   hipMemcpyDeviceToHost, stream_);
-    }
-    const hipError_t es = hipStreamSynchronize(stream_);
-    LBM_HIP_TRY(e);
-    LBM_HIP_TRY(es);
+        return hipGetLastError();
+    }));
     return LBM_OK;
 }
 

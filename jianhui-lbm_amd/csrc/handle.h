@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "lbm_mi355x.h"
+#include "readback.h"
 
 struct lbm_handle {
     enum Kind { SP = 1, CG = 2, SERVER = 3, ST = 4 };
@@ -159,6 +160,7 @@ constexpr int BLOCK_DEFAULT = 256;   // workgroup size of every launch the autot
 constexpr size_t STAGE_BYTES = size_t(16) << 20;
 struct Staging {
     void *buf = nullptr;
+    PinnedUser pinned;
     hipError_t ensure()
     {
         return buf ? hipSuccess : hipMalloc(&buf, STAGE_BYTES);
@@ -197,8 +199,6 @@ public:
     int load_state(const double *f, const double *u, const double *rho);
     int step(int nsteps, double *elapsed_ms);
     int get_state(double *f, double *u, double *rho);
-    // get_state through a caller-chosen device buffer of the given size (no allocation)
-    int get_state_via(double *f, double *u, double *rho, void *buf, size_t bytes);
     // get_state through the library's fixed device array (lbm_sp_get_state_noalloc)
     int get_state_noalloc(double *f, double *u, double *rho);
     int diagnostics(const int32_t *box, lbm_sp_diag *out);
@@ -245,6 +245,7 @@ private:
     void release_boundaries();
     BcDev bc_view(bool for_step) const;
     int reset_viscosity();
+    int get_state_via(double *f, double *u, double *rho, void *buf, size_t bytes);
     int reduce_range(const DiagBox &db, int64_t n_lo, int64_t n_hi);
     hipError_t state_to_device(int64_t n0, int64_t n1, const int32_t *supinv, int64_t v0, double *df, double *du,
                                double *dr);

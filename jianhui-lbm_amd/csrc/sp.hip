@@ -188,6 +188,13 @@ __global__ void __launch_bounds__(BLOCK) fill_kernel(C *__restrict__ p, C v, int
     if (i < n) p[i] = v;
 }
 
+template <typename C>
+__global__ void __launch_bounds__(BLOCK) widen_kernel(const C *__restrict__ p, double *__restrict__ out, int64_t n)
+{
+    const int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (i < n) out[i] = (double)p[i];
+}
+
 // ---------------------------------------------------------------- diagnostics
 constexpr int NDIAG = 8;   // Q0 Q1 Q2 err_num err_den speed_sum umax2 nan  (+ box count below)
 
@@ -801,15 +808,17 @@ int SpSolver::get_viscosity(double *nu)
         for (int64_t i = 0; i < N; ++i) nu[i] = prm_.nu;
         return LBM_OK;
     }
-    if (ct_bytes_ == 8) {
-        LBM_HIP_TRY(hipMemcpyAsync(nu, d_nu_vn_, (size_t)N * 8, hipMemcpyDeviceToHost, stream_));
-        LBM_HIP_TRY(hipStreamSynchronize(stream_));
-    } else {
-        std::vector<float> t((size_t)N);
-        LBM_HIP_TRY(hipMemcpyAsync(t.data(), d_nu_vn_, (size_t)N * 4, hipMemcpyDeviceToHost, stream_));
-        LBM_HIP_TRY(hipStreamSynchronize(stream_));
-        for (int64_t i = 0; i < N; ++i) nu[i] = t[(size_t)i];
-    }
+    LBM_HIP_TRY(stage_.ensure());
+    const ReadPart part{nu, 1};
+    LBM_HIP_TRY(read_back(device_, stream_, N, &part, 1, stage_.buf, STAGE_BYTES, BLOCK,
+                          [&](int64_t n0, int64_t n1, double *const *p) {
+        const dim3 g((unsigned)((n1 - n0 + BLOCK - 1) / BLOCK)), b(BLOCK);
+        if (ct_bytes_ == 8)
+            widen_kernel<double><<<g, b, 0, stream_>>>((const double *)d_nu_vn_ + n0, p[0], n1 - n0);
+        else
+            widen_kernel<float><<<g, b, 0, stream_>>>((const float *)d_nu_vn_ + n0, p[0], n1 - n0);
+        return hipGetLastError();
+    }));
     return LBM_OK;
 }
 
@@ -874,10 +883,15 @@ int SpSolver::get_state(double *f, double *u, double *rho)
     if (mode_ == STATE_EMPTY) return fail(LBM_ERR_STATE, "state not initialised");
     LBM_HIP_TRY(hipSetDevice(device_));
     LBM_HIP_TRY(stage_.ensure());
-    return get_state_via(f, u, rho, stage_.buf, STAGE_BYTES);
+    const ReadPart parts[3] = {{f, Q}, {u, 3}, {rho, 1}};
+    LBM_HIP_TRY(read_back(device_, stream_, geo_.N, parts, 3, stage_.buf, STAGE_BYTES, BLOCK,
+                          [&](int64_t n0, int64_t n1, double *const *p) {
+                              return state_to_device(n0, n1, nullptr, 0, p[0], p[1], p[2]);
+                          }));
+    return LBM_OK;
 }
 
-// the state crosses through buf in chunks of whole blocks of nodes; each chunk's copies are
+// for a caller that must not allocate: the state crosses through buf in chunks of whole blocks of nodes; each chunk's copies are
 // ordered on the stream before the next chunk's kernel overwrites buf
 int SpSolver::get_state_via(double *f, double *u, double *rho, void *buf, size_t bytes)
 {
@@ -912,34 +926,21 @@ int SpSolver::get_dense(double *u_ijk, double *rho_ijk)
     // the box in chunks of consecutive voxels; the fluid nodes of a voxel range are a range of
     // node ids, since the numbering is i-major like the voxel index
     const int64_t N = geo_.N, V = (int64_t)geo_.nx * geo_.ny * geo_.nz;
-    const int64_t chunk = stage_chunk(STAGE_BYTES, (u_ijk ? 3 : 0) + (rho_ijk ? 1 : 0));
     const std::vector<int32_t> &sup = geo_.supinv;
-    hipError_t e = hipSuccess;
-    for (int64_t v0 = 0; v0 < V && e == hipSuccess; v0 += chunk) {
-        const int64_t c = std::min(chunk, V - v0);
-        double *gu = u_ijk ? (double *)stage_.buf : nullptr;
-        double *gr = rho_ijk ? (double *)stage_.buf + (u_ijk ? c * 3 : 0) : nullptr;
+    const ReadPart parts[2] = {{u_ijk, 3}, {rho_ijk, 1}};
+    LBM_HIP_TRY(read_back(device_, stream_, V, parts, 2, stage_.buf, STAGE_BYTES, BLOCK,
+                          [&](int64_t v0, int64_t v1, double *const *p) {
+        const int64_t c = v1 - v0;
         // solid voxels keep the values the reference's writers put there: u = 0, rho = 1
         const dim3 b(BLOCK);
-        if (gu) {
-            fill_kernel<double><<<dim3((unsigned)((c * 3 + BLOCK - 1) / BLOCK)), b, 0, stream_>>>(gu, 0.0, c * 3);
-            e = hipGetLastError();
-        }
-        if (e == hipSuccess && gr) {
-            fill_kernel<double><<<dim3((unsigned)((c + BLOCK - 1) / BLOCK)), b, 0, stream_>>>(gr, 1.0, c);
-            e = hipGetLastError();
-        }
+        if (p[0]) fill_kernel<double><<<dim3((unsigned)((c * 3 + BLOCK - 1) / BLOCK)), b, 0, stream_>>>(p[0], 0.0, c * 3);
+        if (p[1]) fill_kernel<double><<<dim3((unsigned)((c + BLOCK - 1) / BLOCK)), b, 0, stream_>>>(p[1], 1.0, c);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
         const int64_t n0 = std::lower_bound(sup.begin(), sup.end(), v0) - sup.begin();
-        const int64_t n1 = std::lower_bound(sup.begin(), sup.end(), (int64_t)(v0 + c)) - sup.begin();
-        if (e == hipSuccess) e = state_to_device(n0, std::min(n1, N), d_supinv_, v0, nullptr, gu, gr);
-        if (e == hipSuccess && gu)
-            e = hipMemcpyAsync(u_ijk + v0 * 3, gu, (size_t)c * 3 * sizeof(double), hipMemcpyDeviceToHost, stream_);
-        if (e == hipSuccess && gr)
-            e = hipMemcpyAsync(rho_ijk + v0, gr, (size_t)c * sizeof(double), hipMemcpyDeviceToHost, stream_);
-    }
-    const hipError_t es = hipStreamSynchronize(stream_);
-    LBM_HIP_TRY(e);
-    LBM_HIP_TRY(es);
+        const int64_t n1 = std::lower_bound(sup.begin(), sup.end(), v1) - sup.begin();
+        return state_to_device(n0, std::min(n1, N), d_supinv_, v0, nullptr, p[0], p[1]);
+    }));
     return LBM_OK;
 }
 

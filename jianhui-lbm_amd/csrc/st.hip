@@ -531,13 +531,10 @@ int StSolver::get_state(double *g, double *conc)
     LBM_HIP_TRY(stage_.ensure());
     const void *u = velocity();
     const int mode = st_kmode(mode_);
-    const int64_t chunk = stage_chunk(STAGE_BYTES, (g ? Q7 : 0) + (conc ? 1 : 0));
-    hipError_t e = hipSuccess;
-    for (int64_t n0 = 0; n0 < N_ && e == hipSuccess; n0 += chunk) {
-        const int64_t c = std::min(chunk, N_ - n0);
-        double *dg = g ? (double *)stage_.buf : nullptr;
-        double *dc = conc ? (double *)stage_.buf + (g ? c * Q7 : 0) : nullptr;
-        const int64_t n1 = n0 + c;
+    const ReadPart parts[2] = {{g, Q7}, {conc, 1}};
+    LBM_HIP_TRY(read_back(device_, stream_, N_, parts, 2, stage_.buf, STAGE_BYTES, BLOCK,
+                          [&](int64_t n0, int64_t n1, double *const *p) {
+        double *dg = p[0], *dc = p[1];
         dim3 gr((unsigned)((n1 - group_floor(n0) + BLOCK - 1) / BLOCK)), b(BLOCK);
         if (st_bytes_ == 8) {
             auto a = make_st_args<double>(pops_[cur_], nullptr, nbr_, u, d_cinit_, N_, P_, prm_);
@@ -550,15 +547,8 @@ int StSolver::get_state(double *g, double *conc)
             else if (mode == K_DIRECT) st_get_state_kernel<float, K_DIRECT><<<gr, b, 0, stream_>>>(a, n0, n1, dg, dc);
             else st_get_state_kernel<float, K_PULL><<<gr, b, 0, stream_>>>(a, n0, n1, dg, dc);
         }
-        e = hipGetLastError();
-        if (e == hipSuccess && g)
-            e = hipMemcpyAsync(g + n0 * Q7, dg, (size_t)c * Q7 * sizeof(double), hipMemcpyDeviceToHost, stream_);
-        if (e == hipSuccess && conc)
-            e = hipMemcpyAsync(conc + n0, dc, (size_t)c * sizeof(double), hipMemcpyDeviceToHost, stream_);
-    }
-    const hipError_t es = hipStreamSynchronize(stream_);
-    LBM_HIP_TRY(e);
-    LBM_HIP_TRY(es);
+        return hipGetLastError();
+    }));
     return LBM_OK;
 }
 

@@ -152,9 +152,9 @@ __device__ __forceinline__ void cg_node_state(const CgArgs<ST> &a, int64_t n, ty
 
 // One node of the collide kernel.  SLOTS > 0 and FAST: the phase field of the block's
 // neighbourhood is in LDS (lpsi, at the slots of ColourWin w); otherwise it is read from global
-// memory.
+// memory.  A lane that is not live stores nothing.
 template <typename ST, int MODE, bool STORE_U, int SLOTS, bool FAST>
-__device__ __forceinline__ void cg_collide_node(const CgArgs<ST> &a, int64_t n, const typename Store<ST>::C *lpsi,
+__device__ __forceinline__ void cg_collide_node(const CgArgs<ST> &a, int64_t n, bool live, const typename Store<ST>::C *lpsi,
                                                 const ColourWin &w)
 {
     using C = typename Store<ST>::C;
@@ -213,6 +213,7 @@ __device__ __forceinline__ void cg_collide_node(const CgArgs<ST> &a, int64_t n, 
     else
         sv = ps < -a.delta ? a.wg : a.lg0 + a.g1 * ps + a.g2 * ps * ps;
 
+    if (!live) return;
     if (STORE_U && MODE != K_DIRECT) {
         a.u_aux[n] = mc.ux;
         a.u_aux[a.P + n] = mc.uy;
@@ -234,7 +235,9 @@ __global__ void __launch_bounds__(NB) cg_collide_kernel(CgArgs<ST> a)
 {
     using C = typename Store<ST>::C;
     const int64_t b = tile_of(a.order, blockIdx.x, gridDim.x);
-    const int64_t n = b * NB + threadIdx.x;
+    const int64_t n_own = b * NB + threadIdx.x;
+    const bool live = n_own < a.N;
+    const int64_t n = lane_row(n_own, a.P);
     __shared__ C lpsi[SLOTS > 0 ? SLOTS : 1];
     ColourWin w{};
     if (SLOTS > 0) w = a.wins[b];
@@ -249,11 +252,11 @@ __global__ void __launch_bounds__(NB) cg_collide_kernel(CgArgs<ST> a)
         for (int i = 0; i < NS; ++i) lpsi[threadIdx.x + i * NB] = v[i];
         __syncthreads();
     }
-    if (n >= a.N) return;
+    if (SLOTS > 0 && !live) return;   // its slots may lie past the block's
     if (SLOTS > 0 && w.fast == CW_ALL)
-        cg_collide_node<ST, MODE, STORE_U, SLOTS, true>(a, n, lpsi, w);
+        cg_collide_node<ST, MODE, STORE_U, SLOTS, true>(a, n, live, lpsi, w);
     else
-        cg_collide_node<ST, MODE, STORE_U, SLOTS, false>(a, n, lpsi, w);
+        cg_collide_node<ST, MODE, STORE_U, SLOTS, false>(a, n, live, lpsi, w);
 }
 
 // e_q . (x, y, z) with the zero components left out (0 * v is not folded away in IEEE arithmetic)
@@ -288,23 +291,25 @@ __device__ __forceinline__ void static_for(F &&f)
 // g_r, g_b leaving a node with colour state v in direction e_q, or -e_q when bb (the opposite
 // direction, used for the bounce-back term of the pull): the equilibrium split
 // g_c = w rho_c phi_q, phi_q = 1 + 3 e.u + 4.5 (e.u)^2 - 1.5 u.u (CG:3477-3485), then the
-// recolouring g_r += d, g_b -= d, d = min(g_r,q, g_r,opp, g_b,q, g_b,opp) e.C/|C| (CG:3493-3508)
+// recolouring g_r += d, g_b -= d, d = min(g_r,q, g_r,opp, g_b,q, g_b,opp) e.C/|C| (CG:3493-3508).
+// Here and in ColourSums the fused multiply-adds are written out: left to the compiler, the gather
+// and the staged kernels were contracted alike or not as the code around them changed.
 template <int q, typename C>
 __device__ __forceinline__ void colour_pull_term(const C (&v)[8], bool bb, C &gr, C &gb)
 {
+#pragma clang fp contract(off)
     const C rr = v[0], rb = v[1], ux = v[2], uy = v[3], uz = v[4];
-    const C uu = ux * ux + uy * uy + uz * uz;
+    const C uu = fma(uz, uz, fma(ux, ux, uy * uy));
     const C du = e_dot<q>(ux, uy, uz), eu = bb ? -du : du;
-    const C base = C(1) - C(1.5) * uu + C(4.5) * eu * eu;
-    const C phq = base + C(3) * eu, php = base - C(3) * eu;
+    const C base = fma(C(4.5) * eu, eu, fma(C(-1.5), uu, C(1)));
+    const C phq = fma(C(3), eu, base), php = fma(C(-3), eu, base);
     const C w = C(weight(q));
     const C wr = w * rr, wb = w * rb;
-    gr = wr * phq;
-    gb = wb * phq;
-    const C mn = fmin(fmin(fmin(gr, wr * php), gb), wb * php);
+    const C mn = fmin(fmin(fmin(wr * phq, wr * php), wb * phq), wb * php);
     const C dn = e_dot<q>(v[5], v[6], v[7]), en = bb ? -dn : dn;
-    gr += mn * en;
-    gb -= mn * en;
+    const C moved = mn * en;
+    gr = fma(wr, phq, moved);
+    gb = fma(wb, phq, -moved);
 }
 
 // The FP64 build's colour sums of one node, direction by direction: begin() with the node's own
@@ -313,21 +318,21 @@ __device__ __forceinline__ void colour_pull_term(const C (&v)[8], bool bb, C &gr
 // is the node's own state, whose opposite term comes back), then store().  The gather and the
 // staged kernel add the same terms in the same order, so they give the same bits.
 struct ColourSums64 {
-    double rr, rb;
+    double rr, rb, w0;
     __device__ __forceinline__ void begin(const double (&own)[8])
     {
-        const double uu = own[2] * own[2] + own[3] * own[3] + own[4] * own[4];
-        const double w0 = weight(0) * (1.0 - 1.5 * uu);
-        rr = w0 * own[0];
-        rb = w0 * own[1];
+        const double uu = fma(own[4], own[4], fma(own[2], own[2], own[3] * own[3]));
+        w0 = weight(0) * fma(-1.5, uu, 1.0);
+        rr = own[0];
+        rb = own[1];
     }
     template <int q>
     __device__ __forceinline__ void add(bool bb, const double (&v)[8])
     {
         double gr, gb;
         colour_pull_term<q>(v, bb, gr, gb);
-        rr += gr;
-        rb += gb;
+        rr = q == 1 ? fma(w0, rr, gr) : rr + gr;   // the rest population with the first term
+        rb = q == 1 ? fma(w0, rb, gb) : rb + gb;
     }
     __device__ __forceinline__ void store(int64_t n, int64_t P, double *__restrict__ col, double *__restrict__ psi) const
     {
@@ -403,22 +408,23 @@ struct ColourSums {
     static constexpr float UNIT = (float)(1.0 / ColourStore<float>::ONE);   // 2^-29, exact
     static constexpr float ONE = (float)ColourStore<float>::ONE;
     int32_t sr, sb;
-    float tr, tb;
+    float tr, tb, c0;
     __device__ __forceinline__ void begin(const float (&own)[8])
     {
         const int32_t R0 = __float_as_int(own[0]), B0 = __float_as_int(own[1]);
         // rest population: the remainder of the bulk, and w0 rho (phi_0 - 1) = -1.5 w0 rho u.u
         sr = R0 - 6 * colour_share(true, R0) - 12 * colour_share(false, R0);
         sb = B0 - 6 * colour_share(true, B0) - 12 * colour_share(false, B0);
-        const float uu0 = own[2] * own[2] + own[3] * own[3] + own[4] * own[4];
-        const float c0 = (float)weight(0) * -1.5f * uu0;
-        tr = c0 * ((float)R0 * UNIT);
-        tb = c0 * ((float)B0 * UNIT);
+        const float uu0 = fmaf(own[4], own[4], fmaf(own[2], own[2], own[3] * own[3]));
+        c0 = (float)weight(0) * -1.5f * uu0;
+        tr = (float)R0 * UNIT;
+        tb = (float)B0 * UNIT;
     }
     // bb: the upstream site is solid
     template <int q>
     __device__ __forceinline__ void add(bool bb, const float (&vs)[8])
     {
+#pragma clang fp contract(off)
         constexpr bool axis = e2_of(q) == 1;
         const int32_t R = __float_as_int(vs[0]), B = __float_as_int(vs[1]);
         sr += colour_share(axis, R);
@@ -427,18 +433,20 @@ struct ColourSums {
         constexpr float WU = (float)weight(q) * UNIT;
         const float wr = (float)R * WU, wb = (float)B * WU;
         const float ux = vs[2], uy = vs[3], uz = vs[4];
-        const float uu = ux * ux + uy * uy + uz * uz;
+        const float uu = fmaf(uz, uz, fmaf(ux, ux, uy * uy));
         // a solid upstream site sends back this node's own opposite share: e_q negated
         const float du = e_dot<q>(ux, uy, uz), eu = bb ? -du : du;
         // phi_q - 1 formed from the small terms alone: rounding 1 + small and taking 1 off again
         // would be biased, and would drift the colour totals
-        const float s2 = 4.5f * eu * eu - 1.5f * uu;
-        const float eps = s2 + 3.0f * eu;
-        const float phq = 1.0f + eps, php = 1.0f + (s2 - 3.0f * eu);
+        const float s2 = fmaf(eu, 4.5f * eu, -(1.5f * uu));
+        const float eps = fmaf(3.0f, eu, s2);
+        const float phq = 1.0f + eps, php = 1.0f + fmaf(-3.0f, eu, s2);
         const float mn = fminf(fminf(fminf(wr * phq, wr * php), wb * phq), wb * php);
         const float dn = e_dot<q>(vs[5], vs[6], vs[7]), en = bb ? -dn : dn;
-        tr += wr * eps + mn * en;
-        tb += wb * eps - mn * en;
+        const float moved = mn * en;
+        const float gr = fmaf(wr, eps, moved), gb = fmaf(wb, eps, -moved);
+        tr = q == 1 ? fmaf(c0, tr, gr) : tr + gr;   // the rest population with the first term
+        tb = q == 1 ? fmaf(c0, tb, gb) : tb + gb;
     }
     __device__ __forceinline__ void store(int64_t n, int64_t P, int32_t *__restrict__ col, float *__restrict__ psi) const
     {
@@ -544,11 +552,11 @@ __global__ void __launch_bounds__(CW_BLOCK) cg_colour_kernel_win(NbrDev nbr, con
     const int64_t b = tile_of(order, blockIdx.x, gridDim.x);
     const ColourWin w = wins[b];
     const f4 *__restrict__ cs4 = reinterpret_cast<const f4 *>(cs);
-    const int64_t n = b * CW_BLOCK + threadIdx.x;
-    // the neighbour table first, in flight during the staging (the table has P >= N rows, P a
-    // multiple of 256, so a 512-node block can reach past its end: lanes past N load nothing)
+    const int64_t n_own = b * CW_BLOCK + threadIdx.x;
+    const int64_t n = lane_row(n_own, P);   // lanes past the last node store nothing
+    // the neighbour table first, in flight during the staging
     Links<Q - 1> src;
-    if (n < N) load_links(nbr, P, n, src);
+    load_links(nbr, P, n, src);
     if (w.fast == CW_ALL) {   // the same for the whole block
         // slots threadIdx.x + i CW_BLOCK: all loads in flight before the first LDS write
         constexpr int NS = SLOTS / CW_BLOCK;
@@ -567,7 +575,7 @@ __global__ void __launch_bounds__(CW_BLOCK) cg_colour_kernel_win(NbrDev nbr, con
         }
         __syncthreads();
     }
-    if (n >= N) return;
+    if (n_own >= N) return;
     auto lds_state = [&](int32_t slot, float (&v)[8]) {
         const f4 a = lds[slot], c = lds[SLOTS + slot];
         v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
@@ -617,9 +625,10 @@ __global__ void __launch_bounds__(CW_BLOCK) cg_colour_kernel_win64(NbrDev nbr, c
     const int64_t b = tile_of(order, blockIdx.x, gridDim.x);
     const ColourWin w = wins[b];
     const d2 *__restrict__ cs2 = reinterpret_cast<const d2 *>(cs);   // node m: cs2[4 m .. 4 m + 3]
-    const int64_t n = b * CW_BLOCK + threadIdx.x;
+    const int64_t n_own = b * CW_BLOCK + threadIdx.x;
+    const int64_t n = lane_row(n_own, P);   // lanes past the last node store nothing
     Links<Q - 1> src;
-    if (n < N) load_links(nbr, P, n, src);   // lanes past N load nothing (see cg_colour_kernel_win)
+    load_links(nbr, P, n, src);
     if (w.fast == CW_ALL) {   // the same for the whole block
         constexpr int NS = SLOTS / CW_BLOCK;
         static_assert(SLOTS % CW_BLOCK == 0, "whole slots per lane");
@@ -636,7 +645,7 @@ __global__ void __launch_bounds__(CW_BLOCK) cg_colour_kernel_win64(NbrDev nbr, c
             for (int c = 0; c < 4; ++c) lds[c * SLOTS + threadIdx.x + i * CW_BLOCK] = r[i][c];
         __syncthreads();
     }
-    if (n >= N) return;
+    if (n_own >= N) return;
     auto lds_state = [&](int32_t slot, double (&v)[8]) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {

@@ -36,28 +36,28 @@ __device__ __forceinline__ int64_t rr_tile(int64_t b) { return b; }
 // neighbouring x-planes, which gather each other's data, meet in one L2.  For the colour
 // streaming kernel (18 gathers of a 32-byte colour state per node) it cut the L2 misses 3x
 // (340 to 116 MiB per launch on a 192^3 pack) and the time by 6-13 %.
-__device__ __forceinline__ int64_t stream_tile(int64_t b, int64_t grid)
+__device__ __forceinline__ uint32_t stream_tile(uint32_t b, uint32_t grid)
 {
-    constexpr int64_t RUN = 8;
-    const int64_t full = grid / (NUM_XCD * RUN) * (NUM_XCD * RUN);
-    if (b >= full) return b;
-    const int64_t x = b % NUM_XCD, i = b / NUM_XCD;   // the i-th workgroup dealt to XCD x
-    return ((i / RUN) * NUM_XCD + x) * RUN + (i % RUN);
+    constexpr uint32_t RUN = 8;
+    const uint32_t full = grid / (NUM_XCD * RUN) * (NUM_XCD * RUN);
+    const uint32_t x = b % NUM_XCD, i = b / NUM_XCD;   // the i-th workgroup dealt to XCD x
+    return b >= full ? b : ((i / RUN) * NUM_XCD + x) * RUN + (i % RUN);
 }
 
-__device__ __forceinline__ int64_t xcd_slab_tile(int64_t b, int64_t grid)
+__device__ __forceinline__ uint32_t xcd_slab_tile(uint32_t b, uint32_t grid)
 {
-    const int64_t x = b % NUM_XCD, slot = b / NUM_XCD;
-    const int64_t per = grid / NUM_XCD, rem = grid % NUM_XCD;
+    const uint32_t x = b % NUM_XCD, slot = b / NUM_XCD;
+    const uint32_t per = grid / NUM_XCD, rem = grid % NUM_XCD;
     return x * per + (x < rem ? x : rem) + slot;
 }
 
 // Tile orders a launch can use (chosen per kernel and geometry by the autotuner, or set through
 // lbm_set_launch): the hardware order, runs of 8 tiles per XCD, or one slab per XCD.
 enum TileOrder : int32_t { ORDER_HW = 0, ORDER_RUNS8 = 1, ORDER_SLAB = 2 };
-__device__ __forceinline__ int64_t tile_of(int32_t order, int64_t b, int64_t grid)
+__device__ __forceinline__ int64_t tile_of(int32_t order, uint32_t b, uint32_t grid)
 {
-    return order == ORDER_RUNS8 ? stream_tile(b, grid) : (order == ORDER_SLAB ? xcd_slab_tile(b, grid) : b);
+    const uint32_t runs = stream_tile(b, grid), slab = xcd_slab_tile(b, grid);
+    return order == ORDER_RUNS8 ? runs : (order == ORDER_SLAB ? slab : b);
 }
 
 template <typename T>

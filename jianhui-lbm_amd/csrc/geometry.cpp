@@ -186,6 +186,9 @@ int pack_neighbours(const SparseGeometry &g, PackedNbr &out, std::string &err)
             wide |= hi - lo > 0xFFFFu;
         }
         h[HDR_WIDE] = wide ? 0u : HDR_COMPACT;
+        // lanes past the last node: solid all round, so that following their links stays in place
+        for (int64_t n = std::max(n0, n1); n < n0 + 64; ++n)
+            for (int q = 1; q < Q; ++q) set(HDR_MASK + 2 * (q - 1), n - n0);
     }
     int64_t nw = 0, ne = 0;
     for (int64_t w = 0; w < W; ++w) {

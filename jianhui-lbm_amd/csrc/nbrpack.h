@@ -34,9 +34,17 @@
 
 namespace lbm {
 
+constexpr int64_t WAVE_NODES = 64;
+
 // The first node of n's 64-node group: launches over a node range that does not start on a
 // group boundary start their threads here (and idle the lanes before the range).
 __host__ __device__ __forceinline__ int64_t group_floor(int64_t n) { return n & ~int64_t(63); }
+
+// The row a lane reads: its own node's, also past the last node (the arrays have P rows, and the
+// links of a row past the last node stay in place), or past the last row the one of the same lane in
+// the last wave.  A lane always reads the row of its own place in a wave: the header's masks go by
+// lane.
+__device__ __forceinline__ int64_t lane_row(int64_t n, int64_t P) { return n < P ? n : P - WAVE_NODES + (n & (WAVE_NODES - 1)); }
 
 // Where a node's K first populations come from (K = 6: the axis directions, all a D3Q7 pull
 // needs): population q from node up[q - 1], or from the node itself where solid(q).
@@ -48,10 +56,11 @@ struct Links {
     __device__ __forceinline__ bool solid(int q) const { return __builtin_amdgcn_inverse_ballot_w64(bb[q - 1]); }
 };
 
-// The links of node n, but for those of an edge lane with e_z != 0, which wrap_links adds: the
-// others can be followed while the edge records are on their way.  Every active lane of the
-// calling wave must lie in the same group of 64 node ids, which holds for launches whose
-// workgroups are whole wavefronts over consecutive, 64-aligned node ranges.
+// The links of row n < P, but for those of an edge lane with e_z != 0, which wrap_links adds: the
+// others can be followed while the edge records are on their way.  Lane k of the calling wave must
+// hold row k of one group of 64 (n & 63 == k for every active lane, n >> 6 the same for all),
+// which holds for launches whose workgroups are whole wavefronts over consecutive, 64-aligned
+// row ranges.
 template <int K>
 __device__ __forceinline__ void level_links(const NbrDev &d, int64_t P, int64_t n, Links<K> &l)
 {

@@ -68,8 +68,9 @@ __device__ __forceinline__ void st_gather(const StArgs<C> &a, int64_t n, C (&g)[
 template <typename C, int MODE, int NB = BLOCK>
 __global__ void __launch_bounds__(NB) st_step_kernel(StArgs<C> a, int32_t order)
 {
-    const int64_t n = tile_of(order, blockIdx.x, gridDim.x) * NB + threadIdx.x;
-    if (n >= a.N) return;
+    // lanes past the last node leave before the stores (see sp_step_kernel)
+    const int64_t n_own = tile_of(order, blockIdx.x, gridDim.x) * NB + threadIdx.x;
+    const int64_t n = lane_row(n_own, a.P);
     const C ux = a.u[n], uy = a.u[a.P + n], uz = a.u[2 * a.P + n];
     C g[Q7], c;
     if (MODE == K_INIT) {
@@ -80,6 +81,7 @@ __global__ void __launch_bounds__(NB) st_step_kernel(StArgs<C> a, int32_t order)
 #pragma unroll
         for (int q = 1; q < Q7; ++q) c += g[q];
     }
+    if (n_own >= a.N) return;
     const C wc = a.wq * c;
     {
         const C eq = a.w0 * c;

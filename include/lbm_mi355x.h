@@ -328,7 +328,7 @@ double lbm_srv_clock(const lbm_handle *h);
  * for the colour streaming, the variant.  No counterpart in the reference (a CPU program).  By
  * default a handle chooses them itself: at create, on its own geometry, it times every candidate
  * and keeps the fastest (the autotuner; choices are cached per kernel, precision and size class
- * for the life of the process, and boxes under 2^20 fluid nodes keep the defaults).
+ * for the life of the process; boxes under 2^20 fluid nodes take settings by their size).
  * lbm_set_launch fixes a setting, e.g. to compare two; results are identical for every setting. */
 #define LBM_KERNEL_SP_STEP 1      /* single-phase step (sp_step_kernel) */
 #define LBM_KERNEL_CG_COLLIDE 2   /* colour-gradient collide (cg_collide_kernel) */

@@ -1157,7 +1157,13 @@ int CgSolver::launch_step(bool store_u)
 // yet at create, and init or load_state sets every field the timing launches touch.
 int CgSolver::autotune()
 {
-    if (geo_.N < TUNE_MIN_NODES) return LBM_OK;
+    if (geo_.N < TUNE_MIN_NODES) {   // by size (tune.h)
+        const bool staged = geo_.N >= CG_STAGED_NODES && cwin_fast_ >= CG_STAGED_FAST;
+        const int32_t block = staged ? CW_BLOCK : BLOCK, variant = staged ? LBM_VARIANT_STAGED : LBM_VARIANT_GATHER;
+        launch_collide_ = lbm_launch{geo_.N < CG_SMALL_NODES ? 128 : block, ORDER_SLAB, variant, 0, 0.0};
+        launch_colour_ = lbm_launch{block, ORDER_SLAB, variant, 0, 0.0};
+        return LBM_OK;
+    }
     lbm_launch c1, c2;
     if (tune_cache_get(LBM_KERNEL_CG_COLLIDE, prm_.precision, geo_.N, c1) &&
         tune_cache_get(LBM_KERNEL_CG_COLOUR, prm_.precision, geo_.N, c2)) {
@@ -1198,6 +1204,7 @@ int CgSolver::autotune()
     LBM_HIP_TRY(tune_launch(stream_, cc,
                             [&](const lbm_launch &ls) {
                                 hipError_t e = launch_collide(K_PULL, false, ls, a, b);
+                                std::swap(a, b);   // back and forth, as a run steps
                                 return e == hipSuccess ? launch_colour(launch_colour_) : e;
                             },
                             best));
@@ -1208,6 +1215,7 @@ int CgSolver::autotune()
     LBM_HIP_TRY(tune_launch(stream_, cv,
                             [&](const lbm_launch &ls) {
                                 hipError_t e = launch_collide(K_PULL, false, launch_collide_, a, b);
+                                std::swap(a, b);
                                 return e == hipSuccess ? launch_colour(ls) : e;
                             },
                             best));

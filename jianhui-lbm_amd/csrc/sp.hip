@@ -598,10 +598,12 @@ int SpSolver::create(const lbm_sp_params &p, const int32_t *solid)
     return LBM_OK;
 }
 
-// Time the pull step's block sizes and tile orders on this geometry (on the post-collision state
-// of one init launch written to the spare buffer; the handle's state is left as it was).
+// Launch settings of a small box by its size; else time the pull step's block sizes and tile orders
+// on this geometry (on the post-collision state of one init launch, back and forth between the
+// buffers, which hold no state yet).
 int SpSolver::autotune()
 {
+    if (geo_.N < SP_SLAB_NODES) launch_ = lbm_launch{128, ORDER_SLAB, 0, 0, 0.0};
     if (geo_.N < TUNE_MIN_NODES) return LBM_OK;
     lbm_launch c;
     if (tune_cache_get(LBM_KERNEL_SP_STEP, prm_.precision, geo_.N, c)) {
@@ -612,8 +614,14 @@ int SpSolver::autotune()
     LBM_HIP_TRY(launch_kernel(K_INIT, false, nullptr, launch_, state, spare, true));
     const auto cands = tune_candidates(launch_, {128, 256, 512}, {ORDER_HW, ORDER_RUNS8, ORDER_SLAB}, {0});
     lbm_launch best;
+    // back and forth, as a run steps: always from the same buffer, a box of a few million nodes
+    // finds its source in the memory-side cache (3.9 M nodes FP16: 512-node slabs were picked, 78.6 us
+    // a step in a run, before 256-node runs, 75.2 us)
     LBM_HIP_TRY(tune_launch(stream_, cands,
-                            [&](const lbm_launch &ls) { return launch_kernel(K_PULL, false, nullptr, ls, spare, state, true); },
+                            [&](const lbm_launch &ls) {
+                                std::swap(state, spare);
+                                return launch_kernel(K_PULL, false, nullptr, ls, state, spare, true);
+                            },
                             best));
     launch_ = best;
     tune_cache_put(LBM_KERNEL_SP_STEP, prm_.precision, geo_.N, best);

@@ -227,6 +227,7 @@ int st_kmode(StateMode m) { return m == STATE_INIT ? K_INIT : (m == STATE_DIRECT
 // the flow's state, writing only both handles' spare buffers, so neither state changes.
 int StSolver::autotune()
 {
+    if (N_ < ST_SLAB_NODES) launch_ = launch_own_ = lbm_launch{128, ORDER_SLAB, 0, 0, 0.0};
     if (N_ < TUNE_MIN_NODES) return LBM_OK;
     const int kind = flow_ ? -LBM_KERNEL_ST_STEP : LBM_KERNEL_ST_STEP;   // separate cache entries
     lbm_launch c;
@@ -251,11 +252,13 @@ int StSolver::autotune()
     } else {
         const void *u = d_u_own_;
         const auto cands = tune_candidates(launch_own_, {128, 256, 512}, {ORDER_HW, ORDER_RUNS8, ORDER_SLAB}, {0});
-        auto run = [&](const lbm_launch &ls) {
+        int from = 0;
+        auto run = [&](const lbm_launch &ls) {   // back and forth, as a run steps (see SpSolver::autotune)
+            from ^= 1;
             return st_bytes_ == 8
-                       ? launch_st_t(make_st_args<double>(pops_[0], pops_[1], nbr_, u, d_cinit_, N_, P_, prm_), K_PULL,
+                       ? launch_st_t(make_st_args<double>(pops_[from], pops_[from ^ 1], nbr_, u, d_cinit_, N_, P_, prm_), K_PULL,
                                      grid_, ls, stream_)
-                       : launch_st_t(make_st_args<float>(pops_[0], pops_[1], nbr_, u, d_cinit_, N_, P_, prm_), K_PULL,
+                       : launch_st_t(make_st_args<float>(pops_[from], pops_[from ^ 1], nbr_, u, d_cinit_, N_, P_, prm_), K_PULL,
                                      grid_, ls, stream_);
         };
         LBM_HIP_TRY(tune_launch(stream_, cands, run, best));

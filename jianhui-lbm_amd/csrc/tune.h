@@ -11,9 +11,26 @@
 
 namespace lbm {
 
-// boxes with fewer fluid nodes keep the default settings: their launches are too short for the
-// choice to matter, and too short to time
+// boxes with fewer fluid nodes are not tuned: their launches are too short to time
 constexpr int64_t TUNE_MIN_NODES = int64_t(1) << 20;
+// Their settings go by size.  Where both buffers fit the eight L2s (32 MB), a slab of tiles for
+// each XCD serves a step: a tile is read where the launch before wrote it.  Workgroups of 128 nodes
+// fill the CUs of such a box better.  Step, default -> 128-node tiles in slabs: single phase 4,224
+// nodes FP64 4.71 -> 4.27 us, 28,800 FP32 4.52 -> 4.08, 117,964 FP32 6.27 -> 5.42, FP16 5.51 -> 5.14
+// (398,131 FP32 16.2 -> 15.8, FP64 27.0 -> 26.7, above the line: no gain worth a setting); solute
+// 26,214 nodes 3.07 -> 2.75, 209,715 4.22 -> 3.90, with the flow 5.36 -> 4.71 and 12.6 -> 11.6 us
+// (707,788: 11.7 -> 11.7 and 31.3 -> 32.5).
+constexpr int64_t SP_SLAB_NODES = int64_t(1) << 17;
+constexpr int64_t ST_SLAB_NODES = int64_t(1) << 18;
+// Colour gradient, both launches in slabs (one gathers what the other has just written), collide
+// and colour gathering below the line, staged above it where most blocks read from their runs.
+// Step FP32 / FP64, runs of 8 and gathers -> slabs and gathers | slabs and staged: 55,296 nodes 11.2 /
+// 16.2 -> 10.5 / 14.3 | 13.9 / 21.7 us, 131,072 16.4 / 26.8 -> 13.7 / 24.9 | 14.0 / 25.9, 184,320 22.3 /
+// 38.4 -> 20.1 / 37.8 | 23.4 / 44.9, 240,000 27.4 / 48.5 -> 26.4 / 48.3 | 24.2 / 47.6, 649,605 56.7 /
+// 109.2 -> 57.4 / 110.5 | 50.4 / 99.3, 921,600 77.3 / 153.9 -> 79.1 / 157.4 | 66.2 / 135.1.
+constexpr int64_t CG_STAGED_NODES = 215000;
+constexpr double CG_STAGED_FAST = 0.85;
+constexpr int64_t CG_SMALL_NODES = int64_t(1) << 15;   // 128-node collide tiles: 16,384 nodes 9.8 -> 9.3 us, 55,296 10.5 -> 10.9
 // an alternative replaces the default only when it is faster by this fraction
 constexpr double TUNE_MARGIN = 0.01;
 

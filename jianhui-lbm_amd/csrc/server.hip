@@ -12,7 +12,9 @@
 //                                 then per-sample FP64 flux reductions; retire converged
 //                                 samples, free their segments, admit more.
 //
-// Arena layout (row stride CAP nodes, a sample owns rows [base, base + npad)):
+// Arena layout (CAP nodes, a sample owns nodes [base, base + npad), both multiples of 256; the rows
+// of each block of 256 nodes lie together (pop_at), so a sample is one contiguous piece of each
+// array and a small one covers few pages):
 //   pops[2]  19 x CAP  populations (deviation form, FP32 or FP64)
 //   nbr      18 x CAP  int16 upstream delta: upstream - node in sample-local indices, taken
 //                      modulo the sample's node count (so the periodic wraps are short too);
@@ -81,11 +83,10 @@ struct TileDev {
     int64_t base;         // the sample's first arena node (local index origin)
 };
 
-// Addresses: a tile's rows start at the uniform pointer src + base (its sample's first node), and
-// each lane adds a 32-bit BYTE offset, (row * CAP + sample-local node) * sizeof(value), which
-// fits because the arena holds fewer than 2^32 / (19 * sizeof(value)) nodes.  A uniform base plus
-// a 32-bit unsigned offset is the load's own addressing form: one VGPR per address, no 64-bit
-// arithmetic.
+// Addresses: a sample's rows start at the uniform pointer src + 19 * base (its first node), and each
+// lane adds a 32-bit BYTE offset, pop_at(row, sample-local node) * sizeof(value), which fits because
+// the arena holds fewer than 2^32 / (19 * sizeof(value)) nodes.  A uniform base plus a 32-bit
+// unsigned offset is the load's own addressing form: one VGPR per address, no 64-bit arithmetic.
 template <typename T>
 __device__ __forceinline__ T *byte_at(T *base, uint32_t off)
 {
@@ -97,14 +98,25 @@ __device__ __forceinline__ const T *byte_at(const T *base, uint32_t off)
     return reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + off);
 }
 
+constexpr uint32_t row_bytes(int row, uint32_t size) { return (uint32_t)row * POP_BLOCK * size; }
+
+// The step, bounded by memory: 188 bytes a node in FP32, 340 in FP64 (two round trips in a row, the
+// deltas and the gathers, for the few tiles of a small sample).
 // WIDE: the launch covers the tiles of wide samples only (tiles tile0 .. tile0 + gridDim.x - 1;
 // the tile table lists narrow samples' tiles first), so a launch over narrow samples carries no
 // code or registers for the high halves.
-template <typename ST, int BLK, bool WIDE>
+// FIRST: a launch in which a sample may take its first step, from equilibrium.  The other launches
+// have no branch between the deltas and the gathers, so that all gathers are asked for together
+// (behind the branch the compiler asked for them in three batches).
+// Sixteen samples of edges 32 to 88, rows of CAP nodes and the branch -> blocks of 256 and no branch:
+// 27,900 -> 29,300 million node updates a second in FP32, 15,900 -> 17,100 in FP64; one sample of
+// 8,753 nodes 4.0 -> 3.8 us a step.  (Blocks with the branch: 28,300 and 16,900.  A slab of tiles for
+// each XCD gains nothing here: 3.8 us as well.)
+template <typename ST, int BLK, bool WIDE, bool FIRST>
 __global__ void __launch_bounds__(BLK) srv_step_kernel(const TileDev *__restrict__ tiles, const SlotDev *__restrict__ slots,
                                                        const ST *__restrict__ src, ST *__restrict__ dst,
                                                        const int16_t *__restrict__ nbr,
-                                                       const int16_t *__restrict__ nbr_hi, int64_t CAP, int64_t step,
+                                                       const int16_t *__restrict__ nbr_hi, int64_t step,
                                                        int64_t tile0)
 {
     using C = typename Store<ST>::C;
@@ -114,98 +126,54 @@ __global__ void __launch_bounds__(BLK) srv_step_kernel(const TileDev *__restrict
     if (n >= t.end) return;
     const SlotDev sl = slots[t.slot];
     const C gx = (C)sl.gx, gy = (C)sl.gy, gz = (C)sl.gz, rho0 = (C)sl.rho0;
-    const uint32_t cap = (uint32_t)CAP, ln = (uint32_t)(n - t.base);
-    const ST *__restrict__ S = src + t.base;
+    const uint32_t ln = (uint32_t)(n - t.base), own = pop_at<Q>(0, ln) * SZ;
+    const ST *__restrict__ S = src + t.base * Q;
     C h[Q], m[Q];
     Macro<C> mc;
-    if (step == sl.first_step) {   // f = feq(1, 0): the reference's init (SP:1343-1376)
+    const uint32_t link = pop_at<Q - 1>(0, ln) * 2u;
+    const int16_t *__restrict__ NB = nbr + t.base * (Q - 1);
+    constexpr int32_t bbv = WIDE ? SRV_BB32 : (int32_t)SRV_BB;
+    int32_t d[Q - 1];
+#pragma unroll
+    for (int q = 1; q < Q; ++q) d[q - 1] = *byte_at(NB, link + row_bytes(q - 1, 2));
+    if (WIDE) {
+        const int16_t *__restrict__ NH = nbr_hi + t.base * (Q - 1);
+#pragma unroll
+        for (int q = 1; q < Q; ++q)
+            d[q - 1] = srv_delta((int16_t)d[q - 1], *byte_at(NH, link + row_bytes(q - 1, 2)), true);
+    }
+    h[0] = Store<ST>::load(*byte_at(S, own), 1.0f);
+    if (FIRST && step == sl.first_step) {   // f = feq(1, 0): the reference's init (SP:1343-1376)
         mc.rho = C(1);
         mc.drho = C(1) - rho0;
         mc.ux = mc.uy = mc.uz = C(0);
         sp_eq_moments(mc, m);
     } else {
-        const int16_t *__restrict__ NB = nbr + t.base;
         const int32_t cnt = (int32_t)sl.count;
-        constexpr int32_t bbv = WIDE ? SRV_BB32 : (int32_t)SRV_BB;
-        h[0] = Store<ST>::load(*byte_at(S, ln * SZ), 1.0f);
-        int32_t d[Q - 1];
-#pragma unroll
-        for (int q = 1; q < Q; ++q) d[q - 1] = *byte_at(NB, ((uint32_t)(q - 1) * cap + ln) * 2u);
-        if (WIDE) {
-            const int16_t *__restrict__ NH = nbr_hi + t.base;
-#pragma unroll
-            for (int q = 1; q < Q; ++q)
-                d[q - 1] = srv_delta((int16_t)d[q - 1], *byte_at(NH, ((uint32_t)(q - 1) * cap + ln) * 2u), true);
-        }
 #pragma unroll
         for (int q = 1; q < Q; ++q) {
             // upstream node, sample-local: ln + d reduced modulo the node count (|d| <= count/2)
             int32_t u = (int32_t)ln + d[q - 1];
             u += u < 0 ? cnt : 0;
             u -= u >= cnt ? cnt : 0;
-            const uint32_t e = d[q - 1] == bbv ? (uint32_t)opp(q) * cap + ln : (uint32_t)q * cap + (uint32_t)u;
-            h[q] = Store<ST>::load(*byte_at(S, e * SZ), 1.0f);
-        }
-        moments_fwd(h, m);
-        mc = macro_from_moments(m, rho0, gx, gy, gz);
-    }
-    sp_relax(m, mc, gx, gy, gz, (C)sl.sv, (C)sl.sq, h);
-    ST *__restrict__ D = dst + t.base;
-#pragma unroll
-    for (int q = 0; q < Q; ++q) Store<ST>::store_nt(byte_at(D, ((uint32_t)q * cap + ln) * SZ), h[q], 1.0f);
-}
-
-// FP64 arena: 64-bit element indices, which keep this kernel at 70 VGPRs (7 waves per SIMD)
-// where the byte-offset form below needs 84 (5 waves)
-template <typename ST, int BLK, bool WIDE>
-__global__ void __launch_bounds__(BLK) srv_step_kernel_wide(const TileDev *__restrict__ tiles, const SlotDev *__restrict__ slots,
-                                                       const ST *__restrict__ src, ST *__restrict__ dst,
-                                                       const int16_t *__restrict__ nbr,
-                                                       const int16_t *__restrict__ nbr_hi, int64_t CAP, int64_t step,
-                                                       int64_t tile0)
-{
-    using C = typename Store<ST>::C;
-    const TileDev t = tiles[tile0 + stream_tile(blockIdx.x, gridDim.x)];
-    const int64_t n = t.begin + threadIdx.x;
-    if (n >= t.end) return;
-    const SlotDev sl = slots[t.slot];
-    const C gx = (C)sl.gx, gy = (C)sl.gy, gz = (C)sl.gz, rho0 = (C)sl.rho0;
-    C h[Q], m[Q];
-    Macro<C> mc;
-    if (step == sl.first_step) {   // f = feq(1, 0): the reference's init (SP:1343-1376)
-        mc.rho = C(1);
-        mc.drho = C(1) - rho0;
-        mc.ux = mc.uy = mc.uz = C(0);
-        sp_eq_moments(mc, m);
-    } else {
-        h[0] = Store<ST>::load(src[n], 1.0f);
-        constexpr int32_t bbv = WIDE ? SRV_BB32 : (int32_t)SRV_BB;
-        int32_t d[Q - 1];
-#pragma unroll
-        for (int q = 1; q < Q; ++q) d[q - 1] = nbr[(int64_t)(q - 1) * CAP + n];
-        if (WIDE) {
-#pragma unroll
-            for (int q = 1; q < Q; ++q) d[q - 1] = srv_delta((int16_t)d[q - 1], nbr_hi[(int64_t)(q - 1) * CAP + n], true);
-        }
-#pragma unroll
-        for (int q = 1; q < Q; ++q) {
             const bool bb = d[q - 1] == bbv;
-            const int64_t up = srv_upstream(d[q - 1], n, t.base, sl.count);
-            h[q] = Store<ST>::load(src[(bb ? (int64_t)opp(q) : (int64_t)q) * CAP + (bb ? n : up)], 1.0f);
+            const uint32_t at = bb ? ln : (uint32_t)u, row = bb ? row_bytes(opp(q), SZ) : row_bytes(q, SZ);
+            h[q] = Store<ST>::load(*byte_at(S, (uint32_t)pop_at<Q>(0, at) * SZ + row), 1.0f);
         }
         moments_fwd(h, m);
         mc = macro_from_moments(m, rho0, gx, gy, gz);
     }
     sp_relax(m, mc, gx, gy, gz, (C)sl.sv, (C)sl.sq, h);
+    ST *__restrict__ D = dst + t.base * Q;
 #pragma unroll
-    for (int q = 0; q < Q; ++q) Store<ST>::store_nt(&dst[(int64_t)q * CAP + n], h[q], 1.0f);
+    for (int q = 0; q < Q; ++q) Store<ST>::store_nt(byte_at(D, own + row_bytes(q, SZ)), h[q], 1.0f);
 }
 
 // per-tile flux partials Q[3] and a non-finite flag, from the current (pulled) state
 template <typename ST, int BLK>
 __global__ void __launch_bounds__(BLK) srv_flux_kernel(const TileDev *__restrict__ tiles, const SlotDev *__restrict__ slots,
                                                        const ST *__restrict__ src, const int16_t *__restrict__ nbr,
-                                                       const int16_t *__restrict__ nbr_hi, int64_t CAP,
+                                                       const int16_t *__restrict__ nbr_hi,
                                                        double *__restrict__ partial)
 {
     using C = typename Store<ST>::C;
@@ -215,15 +183,15 @@ __global__ void __launch_bounds__(BLK) srv_flux_kernel(const TileDev *__restrict
     if (n < t.end) {
         const SlotDev sl = slots[t.slot];
         C h[Q], m[Q];
-        h[0] = Store<ST>::load(src[n], 1.0f);
+        h[0] = Store<ST>::load(src[pop_at<Q>(0, n)], 1.0f);
         const bool wide = sl.wide != 0;
 #pragma unroll
         for (int q = 1; q < Q; ++q) {
-            const int64_t i = (int64_t)(q - 1) * CAP + n;
+            const int64_t i = pop_at<Q - 1>(q - 1, n);
             const int32_t d = srv_delta(nbr[i], wide ? nbr_hi[i] : (int16_t)0, wide);
             const bool bb = d == (wide ? SRV_BB32 : (int32_t)SRV_BB);
             const int64_t up = srv_upstream(d, n, t.base, sl.count);
-            h[q] = Store<ST>::load(src[(bb ? (int64_t)opp(q) : (int64_t)q) * CAP + (bb ? n : up)], 1.0f);
+            h[q] = Store<ST>::load(src[pop_at<Q>(bb ? opp(q) : q, bb ? n : up)], 1.0f);
         }
         moments_fwd(h, m);
         const Macro<C> mc = macro_from_moments(m, (C)sl.rho0, (C)sl.gx, (C)sl.gy, (C)sl.gz);
@@ -311,6 +279,22 @@ __device__ __forceinline__ void tile_reduce(double (&v)[K], double *out)
     }
 }
 
+// Both kernels below are bounded by memory for large batches, up to 16 (resid) and 11 (update) values
+// per population, and by round trips for small ones.  body(rows, q) takes the 19 rows AA_ROWS at a
+// time: their loads are asked for together, ahead of the stores that they could not be moved across,
+// and for all AA_MAX histories (past count: an address asked for anyway, the value not used) rather
+// than one behind each test of count.  One row and one history at a time -> this, FP32, 16 samples
+// with 1.27 M nodes at first: resid 315 -> 196 us, update 187 -> 137 (medians; the nodes left go down),
+// at 0.2 M nodes 114 -> 71 us.  6 rows take 214 registers in FP64.
+constexpr int AA_ROWS = 3;
+template <typename F>
+__device__ __forceinline__ void aa_rows(const F &body)
+{
+    body(std::integral_constant<int, Q % AA_ROWS>{}, 0);
+#pragma unroll 1
+    for (int q = Q % AA_ROWS; q < Q; q += AA_ROWS) body(std::integral_constant<int, AA_ROWS>{}, q);
+}
+
 template <typename ST, int BLK>
 __global__ void __launch_bounds__(BLK) srv_aa_resid_kernel(const TileDev *__restrict__ tiles,
                                                            const AaDev *__restrict__ aa, const ST *__restrict__ pops,
@@ -326,35 +310,49 @@ __global__ void __launch_bounds__(BLK) srv_aa_resid_kernel(const TileDev *__rest
     double acc[AA_NV];
 #pragma unroll
     for (int k = 0; k < AA_NV; ++k) acc[k] = 0.0;
-    if (a.mode != AA_NONE && n < t.end) {
+    if (a.mode == AA_SAVE && n < t.end) {
+        for (int q = 0; q < Q; ++q) X[pop_at<Q>(q, n)] = pops[pop_at<Q>(q, n)];
+    } else if (a.mode == AA_FIRST && n < t.end) {
         for (int q = 0; q < Q; ++q) {
-            const int64_t i = (int64_t)q * CAP + n;
-            const ST gs = pops[i];
-            if (a.mode == AA_SAVE) {
-                X[i] = gs;
-                continue;
+            const int64_t i = pop_at<Q>(q, n);
+            const ST g = pops[i];
+            RP[i] = (ST)((C)g - (C)X[i]);
+            GP[i] = g;
+            X[i] = g;   // the next iterate is g itself
+        }
+    } else if (a.mode == AA_RESID && n < t.end) {
+        aa_rows([&](auto rows, int q0) {
+            constexpr int G = decltype(rows)::value;
+            ST gs[G], xs[G], rp[G], gp[G], old[G][AA_MAX];
+#pragma unroll
+            for (int k = 0; k < G; ++k) {
+                const int64_t i = pop_at<Q>(q0 + k, n);
+                gs[k] = pops[i];
+                xs[k] = X[i];
+                rp[k] = RP[i];
+                gp[k] = GP[i];
+#pragma unroll
+                for (int h = 0; h < AA_MAX; ++h) old[k][h] = DR[min(h, a.count - 1) * V + i];
             }
-            const C g = (C)gs, r = g - (C)X[i];
-            if (a.mode == AA_RESID) {
-                const C dr = r - (C)RP[i], dg = g - (C)GP[i];
+#pragma unroll
+            for (int k = 0; k < G; ++k) {
+                const int64_t i = pop_at<Q>(q0 + k, n);
+                const C g = (C)gs[k], r = g - (C)xs[k];
+                const C dr = r - (C)rp[k], dg = g - (C)gp[k];
                 DR[a.head * V + i] = (ST)dr;
                 DG[a.head * V + i] = (ST)dg;
+                RP[i] = (ST)r;
+                GP[i] = gs[k];
                 const double drs = (double)(ST)dr;
 #pragma unroll
                 for (int h = 0; h < AA_MAX; ++h) {
-                    if (h < a.count) {
-                        const double v = h == a.head ? drs : (double)DR[h * V + i];
-                        acc[h] += v * drs;
-                        acc[AA_MAX + h] += v * (double)r;
-                    }
+                    const double v = h == a.head ? drs : (double)old[k][h];   // past count: sums that no one reads
+                    acc[h] += v * drs;
+                    acc[AA_MAX + h] += v * (double)r;
                 }
                 acc[2 * AA_MAX] += (double)r * (double)r;
-            } else {
-                X[i] = gs;   // FIRST: the next iterate is g itself
             }
-            RP[i] = (ST)r;
-            GP[i] = gs;
-        }
+        });
     }
     tile_reduce<BLK, AA_NV>(acc, partial + (int64_t)blockIdx.x * AA_NV);
 }
@@ -369,15 +367,27 @@ __global__ void __launch_bounds__(BLK) srv_aa_update_kernel(const TileDev *__res
     const int64_t n = t.begin + threadIdx.x;
     if (a.mode != AA_RESID || n >= t.end) return;
     const int64_t V = (int64_t)Q * CAP;
-    for (int q = 0; q < Q; ++q) {
-        const int64_t i = (int64_t)q * CAP + n;
-        double x = (double)pops[i];
+    aa_rows([&](auto rows, int q0) {
+        constexpr int G = decltype(rows)::value;
+        ST p[G], d[G][AA_MAX];
 #pragma unroll
-        for (int h = 0; h < AA_MAX; ++h)
-            if (h < a.count) x -= a.gamma[h] * (double)DG[h * V + i];
-        pops[i] = (ST)x;
-        X[i] = (ST)x;
-    }
+        for (int k = 0; k < G; ++k) {
+            const int64_t i = pop_at<Q>(q0 + k, n);
+            p[k] = pops[i];
+#pragma unroll
+            for (int h = 0; h < AA_MAX; ++h) d[k][h] = DG[min(h, a.count - 1) * V + i];
+        }
+#pragma unroll
+        for (int k = 0; k < G; ++k) {
+            const int64_t i = pop_at<Q>(q0 + k, n);
+            double x = (double)p[k];
+#pragma unroll
+            for (int h = 0; h < AA_MAX; ++h)
+                if (h < a.count) x -= a.gamma[h] * (double)d[k][h];
+            pops[i] = (ST)x;
+            X[i] = (ST)x;
+        }
+    });
 }
 
 // ---------------------------------------------------------------------------- sample preparation
@@ -466,7 +476,7 @@ __global__ void __launch_bounds__(256) srv_prep_number_kernel(const uint8_t *__r
 template <bool WIDE>
 __global__ void __launch_bounds__(256) srv_prep_links_kernel(const int32_t *__restrict__ idx, int32_t nx, int32_t ny,
                                                              int32_t nz, int64_t N, int16_t *__restrict__ nbr,
-                                                             int16_t *__restrict__ nbr_hi, int64_t CAP, int64_t base,
+                                                             int16_t *__restrict__ nbr_hi, int64_t base,
                                                              int32_t *__restrict__ flag)
 {
     const int64_t nyz = (int64_t)ny * nz, V = (int64_t)nx * nyz;
@@ -491,7 +501,7 @@ __global__ void __launch_bounds__(256) srv_prep_links_kernel(const int32_t *__re
             if (llabs(dd + N) < llabs(best)) best = dd + N;
             d = (int32_t)best;
         }
-        const int64_t e = (int64_t)(q - 1) * CAP + base + n;
+        const int64_t e = pop_at<Q - 1>(q - 1, (uint32_t)(base + n));
         if (WIDE) {
             nbr[e] = (int16_t)(uint16_t)((uint32_t)d & 0xFFFFu);
             nbr_hi[e] = (int16_t)(uint16_t)((uint32_t)d >> 16);
@@ -683,7 +693,7 @@ bool build_deltas(int nx, int ny, int nz, const uint8_t *pore, int64_t &N, int64
                         else
                             w = (int16_t)d;
                     }
-                    o[(size_t)((q - 1) * P + n)] = w;
+                    o[pop_at<Q - 1>(q - 1, (uint32_t)n)] = w;
                 }
             }
     if (bad) {
@@ -698,18 +708,18 @@ bool build_deltas(int nx, int ny, int nz, const uint8_t *pore, int64_t &N, int64
                     if (n < 0) continue;
                     for (int q = 1; q < Q; ++q) {
                         const uint32_t d = (uint32_t)link(i, j, k, n, q);
-                        o[(size_t)((q - 1) * P + n)] = (int16_t)(uint16_t)(d & 0xFFFFu);
-                        oh[(size_t)((q - 1) * P + n)] = (int16_t)(uint16_t)(d >> 16);
+                        o[pop_at<Q - 1>(q - 1, (uint32_t)n)] = (int16_t)(uint16_t)(d & 0xFFFFu);
+                        oh[pop_at<Q - 1>(q - 1, (uint32_t)n)] = (int16_t)(uint16_t)(d >> 16);
                     }
                 }
         for (int q = 0; q < 18; ++q)
             for (int64_t n = N; n < P; ++n) {
-                o[(size_t)(q * P + n)] = 0;
-                oh[(size_t)(q * P + n)] = (int16_t)(uint16_t)((uint32_t)SRV_BB32 >> 16);
+                o[pop_at<Q - 1>(q, (uint32_t)n)] = 0;
+                oh[pop_at<Q - 1>(q, (uint32_t)n)] = (int16_t)(uint16_t)((uint32_t)SRV_BB32 >> 16);
             }
     } else {
         for (int q = 0; q < 18; ++q)
-            for (int64_t n = N; n < P; ++n) o[(size_t)(q * P + n)] = SRV_BB;
+            for (int64_t n = N; n < P; ++n) o[pop_at<Q - 1>(q, (uint32_t)n)] = SRV_BB;
     }
     return true;
 }
@@ -746,6 +756,8 @@ private:
     template <int BLK>
     hipError_t launch_steps(int nsteps);
     hipError_t launch_steps_dispatch(int nsteps);
+    template <typename ST, int BLK, bool FIRST>
+    void launch_step();
     template <int BLK>
     hipError_t launch_flux();
     template <int BLK>
@@ -775,11 +787,12 @@ private:
     void *d_aa_vec_ = nullptr;
     AaDev *d_aa_ = nullptr, *h_aa_ = nullptr;   // h_aa_: two pinned halves, alternating by chunk
     int aa_half_ = 0;
-    double *d_aa_partial_ = nullptr, *d_aa_sums_ = nullptr, *h_aa_sums_ = nullptr;
+    double *d_aa_partial_ = nullptr, *h_aa_sums_ = nullptr;
     SlotDev *d_slots_ = nullptr;
     TileDev *d_tiles_ = nullptr;
     int32_t *d_tlo_ = nullptr, *d_thi_ = nullptr;
-    double *d_partial_ = nullptr, *d_sums_ = nullptr, *h_sums_ = nullptr;
+    double *d_partial_ = nullptr;
+    double *h_sums_ = nullptr;   // page-locked, as h_aa_sums_: the kernels write their results there
     int64_t max_slots_ = 0, max_tiles_ = 0;
     int64_t ntiles_ = 0;
     int64_t ntiles_narrow_ = 0;   // tiles 0 .. ntiles_narrow_ - 1 belong to narrow samples
@@ -848,23 +861,20 @@ bool Server::escalate_locked(Active &a, bool restart)
     if (!fallback_ && !make_fallback(a.req.npad)) return false;
     if (!fallback_->fits(a.req.npad)) return false;
     a.req.nbr = std::shared_ptr<int16_t[]>(new int16_t[(size_t)18 * a.req.npad]);
-    hipError_t e = hipMemcpy2DAsync(a.req.nbr.get(), (size_t)a.req.npad * sizeof(int16_t), d_nbr_ + a.base,
-                                    (size_t)cap_ * sizeof(int16_t), (size_t)a.req.npad * sizeof(int16_t), 18,
-                                    hipMemcpyDeviceToHost, stream_);
+    hipError_t e = hipMemcpyAsync(a.req.nbr.get(), d_nbr_ + 18 * a.base, (size_t)18 * a.req.npad * sizeof(int16_t),
+                                  hipMemcpyDeviceToHost, stream_);
     if (a.req.wide && e == hipSuccess) {
         a.req.nbr_hi = std::shared_ptr<int16_t[]>(new int16_t[(size_t)18 * a.req.npad]);
-        e = hipMemcpy2DAsync(a.req.nbr_hi.get(), (size_t)a.req.npad * sizeof(int16_t), d_nbr_hi_ + a.base,
-                             (size_t)cap_ * sizeof(int16_t), (size_t)a.req.npad * sizeof(int16_t), 18,
-                             hipMemcpyDeviceToHost, stream_);
+        e = hipMemcpyAsync(a.req.nbr_hi.get(), d_nbr_hi_ + 18 * a.base, (size_t)18 * a.req.npad * sizeof(int16_t),
+                           hipMemcpyDeviceToHost, stream_);
     }
     // otherwise the FP64 solve continues from the FP32 state rather than from rest: the
     // transient so far (the pressure build-up of the slow mode) is kept
     if (!restart) {
         a.req.carried.resize((size_t)Q * a.req.npad);
         if (e == hipSuccess)
-            e = hipMemcpy2DAsync(a.req.carried.data(), (size_t)a.req.npad * sizeof(float),
-                                 (const float *)pops_[cur_] + a.base, (size_t)cap_ * sizeof(float),
-                                 (size_t)a.req.npad * sizeof(float), Q, hipMemcpyDeviceToHost, stream_);
+            e = hipMemcpyAsync(a.req.carried.data(), (const float *)pops_[cur_] + Q * a.base,
+                               (size_t)Q * a.req.npad * sizeof(float), hipMemcpyDeviceToHost, stream_);
     }
     if (e == hipSuccess) e = hipStreamSynchronize(stream_);
     if (e != hipSuccess) return false;
@@ -954,14 +964,12 @@ int Server::create(const lbm_srv_params &p)
     LBM_HIP_TRY(hipMalloc(&d_tlo_, (size_t)max_slots_ * sizeof(int32_t)));
     LBM_HIP_TRY(hipMalloc(&d_thi_, (size_t)max_slots_ * sizeof(int32_t)));
     LBM_HIP_TRY(hipMalloc(&d_partial_, (size_t)max_tiles_ * 4 * sizeof(double)));
-    LBM_HIP_TRY(hipMalloc(&d_sums_, (size_t)max_slots_ * 4 * sizeof(double)));
     LBM_HIP_TRY(hipHostMalloc((void **)&h_sums_, (size_t)max_slots_ * 4 * sizeof(double), hipHostMallocDefault));
     if (aa_m_ > 0) {
         LBM_HIP_TRY(hipMalloc(&d_aa_vec_, (size_t)(3 + 2 * aa_m_) * Q * cap_ * st_));
         LBM_HIP_TRY(hipMalloc(&d_aa_, (size_t)max_slots_ * sizeof(AaDev)));
         LBM_HIP_TRY(hipHostMalloc((void **)&h_aa_, (size_t)2 * max_slots_ * sizeof(AaDev), hipHostMallocDefault));
         LBM_HIP_TRY(hipMalloc(&d_aa_partial_, (size_t)max_tiles_ * AA_NV * sizeof(double)));
-        LBM_HIP_TRY(hipMalloc(&d_aa_sums_, (size_t)max_slots_ * AA_NV * sizeof(double)));
         LBM_HIP_TRY(hipHostMalloc((void **)&h_aa_sums_, (size_t)max_slots_ * AA_NV * sizeof(double), hipHostMallocDefault));
     }
     free_.push_back({0, cap_});
@@ -997,8 +1005,7 @@ void Server::shutdown()
     for (void *&b : pops_)
         if (b) (void)hipFree(b), b = nullptr;
     void **bufs[] = {(void **)&d_nbr_, (void **)&d_nbr_hi_, (void **)&d_slots_, (void **)&d_tiles_, (void **)&d_tlo_, (void **)&d_thi_,
-                     (void **)&d_partial_, (void **)&d_sums_, &d_aa_vec_, (void **)&d_aa_, (void **)&d_aa_partial_,
-                     (void **)&d_aa_sums_};
+                     (void **)&d_partial_, &d_aa_vec_, (void **)&d_aa_, (void **)&d_aa_partial_};
     for (void **b : bufs)
         if (*b) (void)hipFree(*b), *b = nullptr;
     for (void *b : {(void *)d_prep_pore_, (void *)d_prep_idx_, (void *)d_prep_tile_, (void *)d_prep_flag_})
@@ -1215,21 +1222,18 @@ bool Server::try_admit_locked()
             e = prepare_on_device(a);
         } else {
             // a handed-over sample: its neighbour rows go straight into the arena rows
-            e = hipMemcpy2DAsync(d_nbr_ + base, (size_t)cap_ * sizeof(int16_t), a.req.nbr.get(),
-                                 (size_t)a.req.npad * sizeof(int16_t), (size_t)a.req.npad * sizeof(int16_t), 18,
-                                 hipMemcpyHostToDevice, stream_);
+            e = hipMemcpyAsync(d_nbr_ + 18 * base, a.req.nbr.get(), (size_t)18 * a.req.npad * sizeof(int16_t),
+                               hipMemcpyHostToDevice, stream_);
             if (e == hipSuccess && a.req.wide)
-                e = hipMemcpy2DAsync(d_nbr_hi_ + base, (size_t)cap_ * sizeof(int16_t), a.req.nbr_hi.get(),
-                                     (size_t)a.req.npad * sizeof(int16_t), (size_t)a.req.npad * sizeof(int16_t), 18,
-                                     hipMemcpyHostToDevice, stream_);
+                e = hipMemcpyAsync(d_nbr_hi_ + 18 * base, a.req.nbr_hi.get(), (size_t)18 * a.req.npad * sizeof(int16_t),
+                                   hipMemcpyHostToDevice, stream_);
         }
         if (e == hipSuccess && !a.req.carried.empty()) {
             // an escalated sample resumes from its FP32 state: no equilibrium step
             std::vector<double> st(a.req.carried.begin(), a.req.carried.end());
             std::vector<float>().swap(a.req.carried);
-            e = hipMemcpy2DAsync((char *)pops_[cur_] + (size_t)base * st_, (size_t)cap_ * st_, st.data(),
-                                 (size_t)a.req.npad * sizeof(double), (size_t)a.req.npad * sizeof(double), Q,
-                                 hipMemcpyHostToDevice, stream_);
+            e = hipMemcpyAsync((char *)pops_[cur_] + (size_t)(Q * base) * st_, st.data(), st.size() * sizeof(double),
+                               hipMemcpyHostToDevice, stream_);
             if (e == hipSuccess) e = hipStreamSynchronize(stream_);
             a.first_step = -1;
         }
@@ -1292,7 +1296,7 @@ hipError_t Server::prepare_on_device(Active &a)
     srv_prep_number_kernel<<<(unsigned)ntiles, 256, 0, stream_>>>(d_prep_pore_, V, d_prep_tile_, d_prep_idx_);
     const unsigned gl = (unsigned)((V + 255) / 256);
     srv_prep_links_kernel<false><<<gl, 256, 0, stream_>>>(d_prep_idx_, a.req.nx, a.req.ny, a.req.nz, a.req.N, d_nbr_,
-                                                           d_nbr_hi_, cap_, a.base, d_prep_flag_);
+                                                           d_nbr_hi_, a.base, d_prep_flag_);
     e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(h_prep_flag_, d_prep_flag_, sizeof(int32_t), hipMemcpyDeviceToHost, stream_);
     if (e == hipSuccess) e = hipStreamSynchronize(stream_);
@@ -1301,7 +1305,7 @@ hipError_t Server::prepare_on_device(Active &a)
     a.req.wide = (*h_prep_flag_ & PREP_WIDE) != 0;
     if (a.req.wide) {
         srv_prep_links_kernel<true><<<gl, 256, 0, stream_>>>(d_prep_idx_, a.req.nx, a.req.ny, a.req.nz, a.req.N, d_nbr_,
-                                                              d_nbr_hi_, cap_, a.base, d_prep_flag_);
+                                                              d_nbr_hi_, a.base, d_prep_flag_);
         e = hipGetLastError();
     }
     return e;
@@ -1372,30 +1376,29 @@ int Server::rebuild_tables(std::string &msg)
     return LBM_OK;
 }
 
+template <typename ST, int BLK, bool FIRST>
+void Server::launch_step()
+{
+    const int64_t nn = ntiles_narrow_, nw = ntiles_ - ntiles_narrow_;
+    const ST *src = (const ST *)pops_[cur_];
+    ST *dst = (ST *)pops_[cur_ ^ 1];
+    if (nn > 0)
+        srv_step_kernel<ST, BLK, false, FIRST><<<(unsigned)nn, BLK, 0, stream_>>>(d_tiles_, d_slots_, src, dst, d_nbr_,
+                                                                                  d_nbr_hi_, global_step_, 0);
+    if (nw > 0)
+        srv_step_kernel<ST, BLK, true, FIRST><<<(unsigned)nw, BLK, 0, stream_>>>(d_tiles_, d_slots_, src, dst, d_nbr_,
+                                                                                 d_nbr_hi_, global_step_, nn);
+}
+
+// Samples are admitted between calls, so only a call's first step can be a sample's first.
 template <int BLK>
 hipError_t Server::launch_steps(int nsteps)
 {
-    const int64_t nn = ntiles_narrow_, nw = ntiles_ - ntiles_narrow_;
     for (int s = 0; s < nsteps; ++s) {
-        if (prm_.precision == LBM_FP64) {
-            const double *src = (const double *)pops_[cur_];
-            double *dst = (double *)pops_[cur_ ^ 1];
-            if (nn > 0)
-                srv_step_kernel_wide<double, BLK, false><<<(unsigned)nn, BLK, 0, stream_>>>(
-                    d_tiles_, d_slots_, src, dst, d_nbr_, d_nbr_hi_, cap_, global_step_, 0);
-            if (nw > 0)
-                srv_step_kernel_wide<double, BLK, true><<<(unsigned)nw, BLK, 0, stream_>>>(
-                    d_tiles_, d_slots_, src, dst, d_nbr_, d_nbr_hi_, cap_, global_step_, nn);
-        } else {
-            const float *src = (const float *)pops_[cur_];
-            float *dst = (float *)pops_[cur_ ^ 1];
-            if (nn > 0)
-                srv_step_kernel<float, BLK, false><<<(unsigned)nn, BLK, 0, stream_>>>(
-                    d_tiles_, d_slots_, src, dst, d_nbr_, d_nbr_hi_, cap_, global_step_, 0);
-            if (nw > 0)
-                srv_step_kernel<float, BLK, true><<<(unsigned)nw, BLK, 0, stream_>>>(
-                    d_tiles_, d_slots_, src, dst, d_nbr_, d_nbr_hi_, cap_, global_step_, nn);
-        }
+        if (prm_.precision == LBM_FP64)
+            s == 0 ? launch_step<double, BLK, true>() : launch_step<double, BLK, false>();
+        else
+            s == 0 ? launch_step<float, BLK, true>() : launch_step<float, BLK, false>();
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         cur_ ^= 1;
@@ -1418,10 +1421,10 @@ hipError_t Server::launch_flux()
 {
     if (prm_.precision == LBM_FP64)
         srv_flux_kernel<double, BLK><<<(unsigned)ntiles_, BLK, 0, stream_>>>(d_tiles_, d_slots_, (const double *)pops_[cur_],
-                                                                             d_nbr_, d_nbr_hi_, cap_, d_partial_);
+                                                                             d_nbr_, d_nbr_hi_, d_partial_);
     else
         srv_flux_kernel<float, BLK><<<(unsigned)ntiles_, BLK, 0, stream_>>>(d_tiles_, d_slots_, (const float *)pops_[cur_],
-                                                                            d_nbr_, d_nbr_hi_, cap_, d_partial_);
+                                                                            d_nbr_, d_nbr_hi_, d_partial_);
     return hipGetLastError();
 }
 
@@ -1490,20 +1493,17 @@ int Server::run_chunk(std::unique_lock<std::mutex> &lk)
     if (e == hipSuccess) e = hipEventRecord(ev1_, stream_);
     if (e == hipSuccess) e = blk_ == 128 ? launch_flux<128>() : (blk_ == 512 ? launch_flux<512>() : launch_flux<256>());
     if (e == hipSuccess) {
-        srv_slot_sum_kernel<4><<<(unsigned)nact, BLOCK, 0, stream_>>>(d_partial_, d_tlo_, d_thi_, d_sums_);
+        srv_slot_sum_kernel<4><<<(unsigned)nact, BLOCK, 0, stream_>>>(d_partial_, d_tlo_, d_thi_, h_sums_);
         e = hipGetLastError();
     }
     if (e == hipSuccess && any_aa) {
         e = hipMemcpyAsync(d_aa_, hb, (size_t)nact * sizeof(AaDev), hipMemcpyHostToDevice, stream_);
         if (e == hipSuccess) e = blk_ == 128 ? launch_aa<128>(false) : (blk_ == 512 ? launch_aa<512>(false) : launch_aa<256>(false));
         if (e == hipSuccess) {
-            srv_slot_sum_kernel<AA_NV><<<(unsigned)nact, BLOCK, 0, stream_>>>(d_aa_partial_, d_tlo_, d_thi_, d_aa_sums_);
+            srv_slot_sum_kernel<AA_NV><<<(unsigned)nact, BLOCK, 0, stream_>>>(d_aa_partial_, d_tlo_, d_thi_, h_aa_sums_);
             e = hipGetLastError();
         }
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(h_aa_sums_, d_aa_sums_, (size_t)nact * AA_NV * sizeof(double), hipMemcpyDeviceToHost, stream_);
     }
-    if (e == hipSuccess) e = hipMemcpyAsync(h_sums_, d_sums_, (size_t)nact * 4 * sizeof(double), hipMemcpyDeviceToHost, stream_);
     if (e == hipSuccess) e = hipStreamSynchronize(stream_);
     float ms = 0.f;
     if (e == hipSuccess) e = hipEventElapsedTime(&ms, ev0_, ev1_);
@@ -1694,8 +1694,7 @@ int Server::autotune()
     a.req.volume = (int64_t)L * L * L;
     a.base = 0;
     a.first_step = 0;
-    LBM_HIP_TRY(hipMemcpy2DAsync(d_nbr_, (size_t)cap_ * sizeof(int16_t), d16.get(), (size_t)P * sizeof(int16_t),
-                                 (size_t)P * sizeof(int16_t), 18, hipMemcpyHostToDevice, stream_));
+    LBM_HIP_TRY(hipMemcpyAsync(d_nbr_, d16.get(), (size_t)18 * P * sizeof(int16_t), hipMemcpyHostToDevice, stream_));
     LBM_HIP_TRY(hipStreamSynchronize(stream_));
     active_.push_back(std::move(a));
     float best = 1e30f;

@@ -53,14 +53,14 @@ struct Links {
     uint32_t up[K];
     uint64_t bb[K];   // the wave's lanes with a solid upstream site
     uint64_t edge;    // the wave's lanes whose columns wrap round in z
+    uint32_t first;   // the index of their first record
     __device__ __forceinline__ bool solid(int q) const { return __builtin_amdgcn_inverse_ballot_w64(bb[q - 1]); }
 };
 
-// The links of row n < P, but for those of an edge lane with e_z != 0, which wrap_links adds: the
-// others can be followed while the edge records are on their way.  Lane k of the calling wave must
-// hold row k of one group of 64 (n & 63 == k for every active lane, n >> 6 the same for all),
-// which holds for launches whose workgroups are whole wavefronts over consecutive, 64-aligned
-// row ranges.
+// The links of row n < P, but for those of an edge lane with e_z != 0, which wrap_links adds.
+// Lane k of the calling wave must hold row k of one group of 64 (n & 63 == k for every active lane,
+// n >> 6 the same for all), which holds for launches whose workgroups are whole wavefronts over
+// consecutive, 64-aligned row ranges.
 template <int K>
 __device__ __forceinline__ void level_links(const NbrDev &d, int64_t P, int64_t n, Links<K> &l)
 {
@@ -75,6 +75,7 @@ __device__ __forceinline__ void level_links(const NbrDev &d, int64_t P, int64_t 
 #pragma unroll
     for (int q = 1; q <= K; ++q) l.bb[q - 1] = reinterpret_cast<const uint64_t *>(h + HDR_MASK)[q - 1];
     l.edge = reinterpret_cast<const uint64_t *>(h + HDR_EDGE)[0];
+    l.first = h[HDR_EDGE_BASE];
     const uint32_t slot = h[HDR_WIDE];
     // decoded whether the wave is compact or not: in an else branch, the rank loads would be
     // issued only when the header has arrived
@@ -97,14 +98,12 @@ __device__ __forceinline__ void level_links(const NbrDev &d, int64_t P, int64_t 
 }
 
 template <int K>
-__device__ __forceinline__ void wrap_links(const NbrDev &d, int64_t n, Links<K> &l)
+__device__ __forceinline__ void wrap_links(const NbrDev &d, Links<K> &l)
 {
     if (l.edge == 0) return;
-    const uint32_t w = __builtin_amdgcn_readfirstlane((uint32_t)(n >> 6));
-    const uint32_t base = d.hdr[(int64_t)w * HDR_WORDS + HDR_EDGE_BASE];
     const uint32_t before = __builtin_amdgcn_mbcnt_hi((uint32_t)(l.edge >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)l.edge, 0u));
     if (!__builtin_amdgcn_inverse_ballot_w64(l.edge)) return;
-    const uint4 *__restrict__ e = d.edge + ((int64_t)base + before) * (EDGE_WORDS / 4);
+    const uint4 *__restrict__ e = d.edge + ((int64_t)l.first + before) * (EDGE_WORDS / 4);
     const uint4 e0 = e[0];
     l.up[4] = e0.x;
     l.up[5] = e0.y;
@@ -120,7 +119,7 @@ template <int K>
 __device__ __forceinline__ void load_links(const NbrDev &d, int64_t P, int64_t n, Links<K> &l)
 {
     level_links(d, P, n, l);
-    wrap_links(d, n, l);
+    wrap_links(d, l);
 }
 
 }  // namespace lbm

@@ -125,7 +125,7 @@ __device__ __forceinline__ void cg_node_state(const CgArgs<ST> &a, int64_t n, ty
 {
     using C = typename Store<ST>::C;
     if (MODE == K_INIT) {
-        load_links(a.nbr, a.P, n, l);
+        load_links<LINK_16>(a.nbr, a.P, n, l);
         mc.rho = C(1);
         mc.drho = C(1) - a.rho0;
         mc.ux = a.ux_i;
@@ -135,8 +135,9 @@ __device__ __forceinline__ void cg_node_state(const CgArgs<ST> &a, int64_t n, ty
         return;
     }
     h[0] = Store<ST>::load(a.src[pop_at<Q>(0, n)], a.inv_scale);
-    gather_links(a.nbr, a.P, n, l, [&](int q) {
-        h[q] = Store<ST>::load(a.src[MODE == K_DIRECT ? pop_at<Q>(q, n) : pull_offset<Q>(l, n, q)], a.inv_scale);
+    // a colour-gradient handle's ranks have 16 bits
+    gather_links<LINK_16>(a.nbr, a.P, n, l, [&](int q) {
+        h[q] = Store<ST>::load(MODE == K_DIRECT ? a.src[pop_at<Q>(q, n)] : a.src[pull_offset<Q>(l, n, q)], a.inv_scale);
     });
     moments_fwd(h, m);
     if (MODE == K_DIRECT) {
@@ -373,7 +374,7 @@ __global__ void __launch_bounds__(BLOCK) cg_colour_kernel64(NbrDev nbr, const do
     double own[8];
     load_cs(cs, n, P, own);
     Links<Q - 1> src;
-    load_links(nbr, P, n, src);
+    load_links<LINK_16>(nbr, P, n, src);
     ColourSums64 acc;
     acc.begin(own);
     colour_gather64(cs, src, n, P, acc);
@@ -521,7 +522,7 @@ __global__ void __launch_bounds__(BLOCK) cg_colour_kernel_fx(NbrDev nbr, const f
     float own[8];
     load_cs(cs, n, P, own);
     Links<Q - 1> src;
-    load_links(nbr, P, n, src);
+    load_links<LINK_16>(nbr, P, n, src);
     ColourSums acc;
     acc.begin(own);
     ColourStep<1>::run(acc, src,
@@ -556,7 +557,7 @@ __global__ void __launch_bounds__(CW_BLOCK) cg_colour_kernel_win(NbrDev nbr, con
     const int64_t n = lane_row(n_own, P);   // lanes past the last node store nothing
     // the neighbour table first, in flight during the staging
     Links<Q - 1> src;
-    load_links(nbr, P, n, src);
+    load_links<LINK_16>(nbr, P, n, src);
     if (w.fast == CW_ALL) {   // the same for the whole block
         // slots threadIdx.x + i CW_BLOCK: all loads in flight before the first LDS write
         constexpr int NS = SLOTS / CW_BLOCK;
@@ -628,7 +629,7 @@ __global__ void __launch_bounds__(CW_BLOCK) cg_colour_kernel_win64(NbrDev nbr, c
     const int64_t n_own = b * CW_BLOCK + threadIdx.x;
     const int64_t n = lane_row(n_own, P);   // lanes past the last node store nothing
     Links<Q - 1> src;
-    load_links(nbr, P, n, src);
+    load_links<LINK_16>(nbr, P, n, src);
     if (w.fast == CW_ALL) {   // the same for the whole block
         constexpr int NS = SLOTS / CW_BLOCK;
         static_assert(SLOTS % CW_BLOCK == 0, "whole slots per lane");
@@ -1051,45 +1052,37 @@ int CgSolver::set_body_force(const double g[3])
     return LBM_OK;
 }
 
-template <typename ST, int NB>
-static void cg_launch_pull_nb(const CgArgs<ST> &a, bool store_u, hipStream_t s)
+template <typename ST, int NB, int SLOTS = 0>
+static void cg_launch_pull(const CgArgs<ST> &a, bool store_u, hipStream_t s)
 {
     const dim3 g((unsigned)((a.N + NB - 1) / NB)), b(NB);
-    store_u ? cg_collide_kernel<ST, K_PULL, true, NB><<<g, b, 0, s>>>(a)
-            : cg_collide_kernel<ST, K_PULL, false, NB><<<g, b, 0, s>>>(a);
-}
-
-template <typename ST, int SLOTS>
-static void cg_launch_pull_staged(const CgArgs<ST> &a, bool store_u, int64_t cw_grid, hipStream_t s)
-{
-    const dim3 g((unsigned)cw_grid), b(CW_BLOCK);
-    store_u ? cg_collide_kernel<ST, K_PULL, true, CW_BLOCK, SLOTS><<<g, b, 0, s>>>(a)
-            : cg_collide_kernel<ST, K_PULL, false, CW_BLOCK, SLOTS><<<g, b, 0, s>>>(a);
+    store_u ? cg_collide_kernel<ST, K_PULL, true, NB, SLOTS><<<g, b, 0, s>>>(a)
+            : cg_collide_kernel<ST, K_PULL, false, NB, SLOTS><<<g, b, 0, s>>>(a);
 }
 
 template <typename ST>
-static hipError_t cg_launch_collide(CgArgs<ST> a, int mode, bool store_u, int64_t grid, int64_t cw_grid,
+static hipError_t cg_launch_collide(CgArgs<ST> a, int mode, bool store_u, int64_t grid,
                                     const lbm_launch &ls, const void *wins, int slots, hipStream_t s)
 {
     dim3 g((unsigned)grid), b(BLOCK);
     a.order = ls.order;
     a.wins = (const ColourWin *)wins;
     if (mode == K_PULL && ls.variant == LBM_VARIANT_STAGED && slots == 1024)
-        cg_launch_pull_staged<ST, 1024>(a, store_u, cw_grid, s);
+        cg_launch_pull<ST, CW_BLOCK, 1024>(a, store_u, s);
     else if (mode == K_PULL && ls.variant == LBM_VARIANT_STAGED && slots == 1536)
-        cg_launch_pull_staged<ST, 1536>(a, store_u, cw_grid, s);
+        cg_launch_pull<ST, CW_BLOCK, 1536>(a, store_u, s);
     else if (mode == K_PULL && ls.variant == LBM_VARIANT_STAGED && slots == 2560)
-        cg_launch_pull_staged<ST, 2560>(a, store_u, cw_grid, s);
+        cg_launch_pull<ST, CW_BLOCK, 2560>(a, store_u, s);
     else if (mode == K_INIT)
         store_u ? cg_collide_kernel<ST, K_INIT, true><<<g, b, 0, s>>>(a) : cg_collide_kernel<ST, K_INIT, false><<<g, b, 0, s>>>(a);
     else if (mode == K_DIRECT)
         cg_collide_kernel<ST, K_DIRECT, false><<<g, b, 0, s>>>(a);
     else if (ls.block == 128)
-        cg_launch_pull_nb<ST, 128>(a, store_u, s);
+        cg_launch_pull<ST, 128>(a, store_u, s);
     else if (ls.block == 512)
-        cg_launch_pull_nb<ST, 512>(a, store_u, s);
+        cg_launch_pull<ST, 512>(a, store_u, s);
     else
-        store_u ? cg_collide_kernel<ST, K_PULL, true><<<g, b, 0, s>>>(a) : cg_collide_kernel<ST, K_PULL, false><<<g, b, 0, s>>>(a);
+        cg_launch_pull<ST, BLOCK>(a, store_u, s);
     return hipGetLastError();
 }
 
@@ -1100,10 +1093,10 @@ hipError_t CgSolver::launch_collide(int mode, bool store_u, const lbm_launch &ls
     if (prm_.precision == LBM_FP64)
         return cg_launch_collide(make_cg_args<double>(prm_, visc_, u_i_, src, dst, nbr_.view(), d_col_, d_psi_, d_cs_, d_u_,
                                                       d_rho_, N, P),
-                                 mode, store_u, grid_, cw_grid_, ls, d_cwin_, cwin_slots_, stream_);
+                                 mode, store_u, grid_, ls, d_cwin_, cwin_slots_, stream_);
     return cg_launch_collide(make_cg_args<float>(prm_, visc_, u_i_, src, dst, nbr_.view(), d_col_, d_psi_, d_cs_, d_u_,
                                                  d_rho_, N, P),
-                             mode, store_u, grid_, cw_grid_, ls, d_cwin_, cwin_slots_, stream_);
+                             mode, store_u, grid_, ls, d_cwin_, cwin_slots_, stream_);
 }
 
 // the colour-streaming launch: gathers, or (FP32) the LDS-staged variant

@@ -132,17 +132,19 @@ uint32_t unpack_link(const PackedNbr &p, int64_t P, int64_t n, int q)
     }
     const int c = COL.column[q];
     if (c == NCOL) return (uint32_t)(n - EZ[q]);
-    const uint32_t r = h[c] + p.res[(size_t)(((c / 4) * P + n) * 4 + c % 4)];
+    const size_t at = (size_t)(((c / 4) * P + n) * 4 + c % 4);
+    const uint32_t r = p.narrow ? h[c] + (uint32_t)n + p.res8[at] : h[c] + p.res[at];
     if (EZ[q] == 0) return r;
     return EZ[q] > 0 ? r - 1 : r + (mask(HDR_MASK + 2 * (COL.at[c] - 1)) >> lane & 1 ? 0u : 1u);
 }
 
 }  // namespace
 
-int pack_neighbours(const SparseGeometry &g, PackedNbr &out, std::string &err)
+int pack_neighbours(const SparseGeometry &g, PackedNbr &out, std::string &err, bool narrow_ok)
 {
     const int64_t P = g.P, N = g.N, W = P / 64;
-    out.res.assign((size_t)(NCOL * P), 0u);
+    std::vector<uint32_t> base8((size_t)(W * NCOL), 0u);
+    std::vector<uint8_t> wide8((size_t)W, 0u);
     out.hdr.assign((size_t)(W * HDR_WORDS), 0u);
     auto link = [&g, P](int64_t n, int q) { return g.nbr[(size_t)((q - 1) * P + n)]; };
     auto none = [](uint32_t v) { return (v & BB_FLAG) != 0; };
@@ -169,6 +171,7 @@ int pack_neighbours(const SparseGeometry &g, PackedNbr &out, std::string &err)
         bool wide = false;
         for (int c = 0; c <= NCOL; ++c) {
             uint32_t lo = 0xFFFFFFFFu, hi = 0, at, below, above;
+            int64_t lo8 = INT64_MAX, hi8 = INT64_MIN;   // of the rank less the node's own id
             for (int64_t n = n0; n < n1; ++n) {
                 column(n, c, at, below, above);
                 solid(at, COL.at[c], n - n0);
@@ -180,19 +183,32 @@ int pack_neighbours(const SparseGeometry &g, PackedNbr &out, std::string &err)
                     set(HDR_EDGE, n - n0);
                 lo = std::min(lo, r);
                 hi = std::max(hi, r);
+                lo8 = std::min(lo8, (int64_t)r - n);
+                hi8 = std::max(hi8, (int64_t)r - n);
             }
             if (c == NCOL || lo == 0xFFFFFFFFu) continue;   // the own column needs no ranks
             h[c] = lo;
             wide |= hi - lo > 0xFFFFu;
+            base8[(size_t)(w * NCOL + c)] = (uint32_t)lo8;
+            wide8[(size_t)w] |= hi8 - lo8 > 0xFF;
         }
         h[HDR_WIDE] = wide ? 0u : HDR_COMPACT;
         // lanes past the last node: solid all round, so that following their links stays in place
         for (int64_t n = std::max(n0, n1); n < n0 + 64; ++n)
             for (int q = 1; q < Q; ++q) set(HDR_MASK + 2 * (q - 1), n - n0);
     }
+    int64_t n_wide8 = 0;
+    for (uint8_t v : wide8) n_wide8 += v;
+    out.narrow = narrow_ok && n_wide8 <= W / NARROW_WIDE;
+    out.res.assign(out.narrow ? 0 : (size_t)(NCOL * P), 0u);
+    out.res8.assign(out.narrow ? (size_t)(NCOL * P) : 0, 0u);
     int64_t nw = 0, ne = 0;
     for (int64_t w = 0; w < W; ++w) {
         uint32_t *h = &out.hdr[(size_t)(w * HDR_WORDS)];
+        if (out.narrow) {
+            std::copy_n(&base8[(size_t)(w * NCOL)], NCOL, h);
+            h[HDR_WIDE] = wide8[(size_t)w] ? 0u : HDR_COMPACT;
+        }
         if (h[HDR_WIDE] != HDR_COMPACT) {
             h[HDR_WIDE] = (uint32_t)nw++;
             continue;
@@ -220,7 +236,10 @@ int pack_neighbours(const SparseGeometry &g, PackedNbr &out, std::string &err)
                 uint32_t at, below, above;
                 column(n, c, at, below, above);
                 if (none(at) && none(below) && none(above)) continue;
-                out.res[(size_t)(((c / 4) * P + n) * 4 + c % 4)] = (uint16_t)(rank(at, below, above) - h[c]);
+                const size_t i = (size_t)(((c / 4) * P + n) * 4 + c % 4);
+                const uint32_t r = rank(at, below, above) - h[c];
+                if (out.narrow) out.res8[i] = (uint8_t)(r - (uint32_t)n);
+                else out.res[i] = (uint16_t)r;
             }
             if (h[HDR_EDGE + ((n - n0) >> 5)] >> ((n - n0) & 31) & 1) {
                 for (int q = 1; q < Q; ++q)
@@ -241,29 +260,32 @@ int pack_neighbours(const SparseGeometry &g, PackedNbr &out, std::string &err)
     return LBM_OK;
 }
 
-hipError_t DeviceNbr::upload(const PackedNbr &p, int64_t P, hipStream_t s)
+hipError_t DeviceNbr::upload(const PackedNbr &p, int64_t, hipStream_t s)
 {
     release();
-    const size_t b_res = (size_t)NCOL * P * sizeof(uint16_t), b_hdr = p.hdr.size() * sizeof(uint32_t);
-    const size_t b_edge = p.edge.size() * sizeof(uint32_t), b_wide = p.wide.size() * sizeof(uint32_t);
+    const void *from[4] = {p.narrow ? (const void *)p.res8.data() : (const void *)p.res.data(), p.hdr.data(), p.edge.data(),
+                           p.wide.data()};
+    const size_t bytes[4] = {p.narrow ? p.res8.size() : p.res.size() * sizeof(uint16_t), p.hdr.size() * sizeof(uint32_t),
+                             p.edge.size() * sizeof(uint32_t), p.wide.size() * sizeof(uint32_t)};
+    size_t at[5] = {0};
+    for (int k = 0; k < 4; ++k) at[k + 1] = at[k] + (bytes[k] + 255) / 256 * 256;
     hipError_t e;
-    if ((e = hipMalloc(&res, b_res)) != hipSuccess) return e;
-    if ((e = hipMalloc(&hdr, b_hdr)) != hipSuccess) return e;
-    if ((e = hipMalloc(&edge, std::max<size_t>(b_edge, 16))) != hipSuccess) return e;
-    if ((e = hipMalloc(&wide, std::max<size_t>(b_wide, 16))) != hipSuccess) return e;
-    if ((e = hipMemcpyAsync(res, p.res.data(), b_res, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
-    if ((e = hipMemcpyAsync(hdr, p.hdr.data(), b_hdr, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
-    if (b_edge && (e = hipMemcpyAsync(edge, p.edge.data(), b_edge, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
-    if (b_wide && (e = hipMemcpyAsync(wide, p.wide.data(), b_wide, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
+    if ((e = hipMalloc(&res, at[4])) != hipSuccess) return e;
+    char *d = (char *)res;
+    hdr = (uint32_t *)(d + at[1]);
+    edge = (uint4 *)(d + at[2]);
+    wide = (uint32_t *)(d + at[3]);
+    narrow = p.narrow;
+    for (int k = 0; k < 4; ++k)
+        if (bytes[k] && (e = hipMemcpyAsync(d + at[k], from[k], bytes[k], hipMemcpyHostToDevice, s)) != hipSuccess) return e;
     return hipSuccess;
 }
 
 void DeviceNbr::release()
 {
     if (res) (void)hipFree(res), res = nullptr;
-    if (hdr) (void)hipFree(hdr), hdr = nullptr;
-    if (edge) (void)hipFree(edge), edge = nullptr;
-    if (wide) (void)hipFree(wide), wide = nullptr;
+    hdr = wide = nullptr;
+    edge = nullptr;
 }
 
 }  // namespace lbm

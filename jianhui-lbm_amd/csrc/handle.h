@@ -69,7 +69,7 @@ inline int64_t padded_stride(int64_t n) { return ((n + 255) / 256) * 256; }
 
 // Device form of the neighbour lists (decoded by load_links in nbrpack.h): per wavefront of 64
 // node ids one header with a base per neighbour column and a solid mask per direction, and per
-// node and column one 16-bit rank.
+// node and column one rank of 16 or 8 bits.
 constexpr int NCOL = 8;                        // neighbour columns (x - ex, y - ey), own one apart
 constexpr int HDR_WORDS = 48;                  // 32-bit words per wave
 constexpr int HDR_MASK = 8;                    // after the NCOL bases: 18 64-bit solid masks
@@ -79,8 +79,14 @@ constexpr int HDR_WIDE = 47;                   // wide slot
 constexpr uint32_t HDR_COMPACT = 0xFFFFFFFFu;  // wide slot of a compact wave
 constexpr int EDGE_WORDS = 12;                 // an edge record: the 10 directions with e_z != 0, padded
 
+// 8-bit ranks where at most one wave in NARROW_WIDE needs full words for them (nbrpack.h).
+constexpr int64_t NARROW_WIDE = 32;
+constexpr int64_t NARROW_NODES = int64_t(1) << 20;   // smaller boxes keep 16 bits
+
 struct PackedNbr {
     std::vector<uint16_t> res;    // 2 x P x 4: ranks in columns 0-3 (axis) and 4-7 (xy diagonals)
+    std::vector<uint8_t> res8;    // the same in 8 bits (narrow; else empty)
+    bool narrow = false;
     std::vector<uint32_t> hdr;    // (P / 64) x HDR_WORDS
     std::vector<uint32_t> edge;   // n_edge x EDGE_WORDS
     std::vector<uint32_t> wide;   // n_wide x 18 x 64
@@ -89,24 +95,26 @@ struct PackedNbr {
 
 // Pack g.nbr, then decode every entry and compare with the full table (LBM_ERR_STATE if any
 // differs, which would be a packing bug).
-int pack_neighbours(const SparseGeometry &g, PackedNbr &out, std::string &err);
+int pack_neighbours(const SparseGeometry &g, PackedNbr &out, std::string &err, bool narrow_ok = false);
 
 struct NbrDev {
-    const uint2 *__restrict__ res;      // 2 x P: four 16-bit ranks each
+    const void *__restrict__ res;       // 2 x P: four ranks each, 16-bit (uint2) or 8-bit (uint32_t)
     const uint32_t *__restrict__ hdr;   // (P / 64) x HDR_WORDS
     const uint4 *__restrict__ edge;     // n_edge x EDGE_WORDS / 4
     const uint32_t *__restrict__ wide;  // n_wide x 18 x 64
+    uint32_t narrow;
 };
 
-// Owner of the packed table in device memory.
+// Owner of the packed table in device memory, one allocation.
 struct DeviceNbr {
-    uint2 *res = nullptr;
+    void *res = nullptr;
     uint4 *edge = nullptr;
     uint32_t *hdr = nullptr, *wide = nullptr;
+    bool narrow = false;
     // allocate and queue the copies on s; p must stay alive until s has been synchronised
     hipError_t upload(const PackedNbr &p, int64_t P, hipStream_t s);
     void release();
-    NbrDev view() const { return NbrDev{res, hdr, edge, wide}; }
+    NbrDev view() const { return NbrDev{res, hdr, edge, wide, narrow}; }
 };
 
 // Face boundaries (lbm_sp_set_boundaries).  Every fluid node on an active face gets one

@@ -127,8 +127,8 @@ __device__ __forceinline__ Macro<typename Store<ST>::C> node_macro(const SpArgs<
 // their rule, and every launch saves the pre-collision state of the nodes the rules read.
 // PL: power-law collision (pull launches of reference steps n > 10, SP:2397).
 // FUSED: also the step of a coupled solute (pull launches).
-// NB: nodes (threads) per workgroup; a.order: the tile order.
-template <typename ST, int MODE, bool STORE_U, bool BC, bool PL = false, bool FUSED = false, int NB = BLOCK>
+// NB: nodes (threads) per workgroup; a.order: the tile order; LF: how links are followed (nbrpack.h).
+template <typename ST, int MODE, bool STORE_U, bool BC, bool PL = false, bool FUSED = false, int NB = BLOCK, int LF = LINK_FAR>
 __global__ void __launch_bounds__(NB) sp_step_kernel(SpArgs<ST> a)
 {
     using C = typename Store<ST>::C;
@@ -151,7 +151,7 @@ __global__ void __launch_bounds__(NB) sp_step_kernel(SpArgs<ST> a)
         }
     } else {
         Links<Q - 1> l;
-        gather_pops<ST, MODE>(a.src, a.nbr, a.P, n, a.inv_scale, h, l);
+        gather_pops<ST, MODE, LF>(a.src, a.nbr, a.P, n, a.inv_scale, h, l);
         if (n_own >= a.N) return;
         if (BC && MODE == K_PULL) bc_patch(a.bc, n, a.rho0, h);
         moments_fwd(h, m);
@@ -161,7 +161,7 @@ __global__ void __launch_bounds__(NB) sp_step_kernel(SpArgs<ST> a)
             C g[7];
             g[0] = a.st.src[pop_at<7>(0, n)];
 #pragma unroll
-            for (int q = 1; q < 7; ++q) g[q] = a.st.src[pull_offset<7>(l, n, q)];
+            for (int q = 1; q < 7; ++q) g[q] = pull_value<7, LF>(a.st.src, l, n, q);
             C c = g[0];
 #pragma unroll
             for (int q = 1; q < 7; ++q) c += g[q];
@@ -400,16 +400,21 @@ SpArgs<ST> make_args(const void *src, void *dst, const NbrDev &nbr, void *u_aux,
 }
 
 // the pull step without faces or power law, at a workgroup size NB
-template <typename ST, int NB>
+template <typename ST, bool FUSED, int NB>
 void launch_pull_nb(const SpArgs<ST> &a, bool store_u, int64_t N, hipStream_t s)
 {
     const dim3 g((unsigned)((N + NB - 1) / NB)), b(NB);
-    if (a.st.src)
-        store_u ? sp_step_kernel<ST, K_PULL, true, false, false, true, NB><<<g, b, 0, s>>>(a)
-                : sp_step_kernel<ST, K_PULL, false, false, false, true, NB><<<g, b, 0, s>>>(a);
-    else
-        store_u ? sp_step_kernel<ST, K_PULL, true, false, false, false, NB><<<g, b, 0, s>>>(a)
-                : sp_step_kernel<ST, K_PULL, false, false, false, false, NB><<<g, b, 0, s>>>(a);
+    // a coupled solute's 7 rows are of the compute type
+    const int lf = link_form(a.nbr, (uint64_t)a.P * std::max(Q * sizeof(ST), FUSED ? 7 * sizeof(typename Store<ST>::C) : 0));
+    if (store_u) sp_step_kernel<ST, K_PULL, true, false, false, FUSED, NB><<<g, b, 0, s>>>(a);
+    else if (lf == LINK_16) sp_step_kernel<ST, K_PULL, false, false, false, FUSED, NB, LINK_16><<<g, b, 0, s>>>(a);
+    else if (lf == LINK_8) sp_step_kernel<ST, K_PULL, false, false, false, FUSED, NB, LINK_8><<<g, b, 0, s>>>(a);
+    else sp_step_kernel<ST, K_PULL, false, false, false, FUSED, NB><<<g, b, 0, s>>>(a);
+}
+template <typename ST, int NB>
+void launch_pull(const SpArgs<ST> &a, bool store_u, int64_t N, hipStream_t s)
+{
+    a.st.src ? launch_pull_nb<ST, true, NB>(a, store_u, N, s) : launch_pull_nb<ST, false, NB>(a, store_u, N, s);
 }
 
 template <typename ST, bool BC>
@@ -419,7 +424,7 @@ void launch_step_bc(const SpArgs<ST> &a, int mode, bool store_u, dim3 g, dim3 b,
         if (a.nu_vn)
             store_u ? sp_step_kernel<ST, K_PULL, true, BC, true, true><<<g, b, 0, s>>>(a)
                     : sp_step_kernel<ST, K_PULL, false, BC, true, true><<<g, b, 0, s>>>(a);
-        else
+        else if constexpr (BC)   // without faces: launch_pull
             store_u ? sp_step_kernel<ST, K_PULL, true, BC, false, true><<<g, b, 0, s>>>(a)
                     : sp_step_kernel<ST, K_PULL, false, BC, false, true><<<g, b, 0, s>>>(a);
     } else if (mode == K_PULL && a.nu_vn)
@@ -430,7 +435,7 @@ void launch_step_bc(const SpArgs<ST> &a, int mode, bool store_u, dim3 g, dim3 b,
                 : sp_step_kernel<ST, K_INIT, false, BC><<<g, b, 0, s>>>(a);
     else if (mode == K_DIRECT)
         sp_step_kernel<ST, K_DIRECT, false, BC><<<g, b, 0, s>>>(a);
-    else
+    else if constexpr (BC)
         store_u ? sp_step_kernel<ST, K_PULL, true, BC><<<g, b, 0, s>>>(a)
                 : sp_step_kernel<ST, K_PULL, false, BC><<<g, b, 0, s>>>(a);
 }
@@ -454,11 +459,13 @@ hipError_t launch_step_t(SpArgs<ST> a, const BcDev &bc, void *nu_vn, double pl_m
         a.st.wq = (C)fs->wq;
         a.st.inv_cs2 = (C)fs->inv_cs2;
     }
-    if (mode == K_PULL && !bc.wave && !nu_vn && ls.block != BLOCK) {
+    if (mode == K_PULL && !bc.wave && !nu_vn) {
         if (ls.block == 128)
-            launch_pull_nb<ST, 128>(a, store_u, a.N, s);
+            launch_pull<ST, 128>(a, store_u, a.N, s);
+        else if (ls.block == 512)
+            launch_pull<ST, 512>(a, store_u, a.N, s);
         else
-            launch_pull_nb<ST, 512>(a, store_u, a.N, s);
+            launch_pull<ST, BLOCK>(a, store_u, a.N, s);
     } else if (bc.wave) {
         launch_step_bc<ST, true>(a, mode, store_u, g, b, s);
     } else {
@@ -580,7 +587,7 @@ int SpSolver::create(const lbm_sp_params &p, const int32_t *solid)
     LBM_HIP_TRY(hipMalloc(&d_result_, 32 * sizeof(double)));
     LBM_HIP_TRY(hipHostMalloc((void **)&h_result_, 32 * sizeof(double), hipHostMallocDefault));
     PackedNbr packed;
-    rc = pack_neighbours(geo_, packed, err);
+    rc = pack_neighbours(geo_, packed, err, geo_.N >= NARROW_NODES);
     if (rc != LBM_OK) return fail(rc, err);
     LBM_HIP_TRY(nbr_.upload(packed, P, stream_));
     LBM_HIP_TRY(hipMemcpyAsync(d_supinv_, geo_.supinv.data(), geo_.supinv.size() * sizeof(int32_t),

@@ -52,7 +52,7 @@ __device__ __forceinline__ C axis_dot(int q, C ux, C uy, C uz)
 }
 
 // the 7 post-streaming populations of node n
-template <typename C, int MODE>
+template <typename C, int MODE, int LF = LINK_FAR>
 __device__ __forceinline__ void st_gather(const StArgs<C> &a, int64_t n, C (&g)[Q7])
 {
     g[0] = a.src[pop_at<Q7>(0, n)];
@@ -62,10 +62,10 @@ __device__ __forceinline__ void st_gather(const StArgs<C> &a, int64_t n, C (&g)[
         return;
     }
     Links<6> l;
-    gather_links(a.nbr, a.P, n, l, [&](int q) { g[q] = a.src[pull_offset<Q7>(l, n, q)]; });
+    gather_links<LF>(a.nbr, a.P, n, l, [&](int q) { g[q] = a.src[pull_offset<Q7>(l, n, q)]; });
 }
 
-template <typename C, int MODE, int NB = BLOCK>
+template <typename C, int MODE, int NB = BLOCK, int LF = LINK_FAR>
 __global__ void __launch_bounds__(NB) st_step_kernel(StArgs<C> a, int32_t order)
 {
     // lanes past the last node leave before the stores (see sp_step_kernel)
@@ -76,7 +76,7 @@ __global__ void __launch_bounds__(NB) st_step_kernel(StArgs<C> a, int32_t order)
     if (MODE == K_INIT) {
         c = a.cinit[n];   // g = g_eq(C, u): its collision leaves it unchanged
     } else {
-        st_gather<C, MODE>(a, n, g);
+        st_gather<C, MODE, LF>(a, n, g);
         c = g[0];
 #pragma unroll
         for (int q = 1; q < Q7; ++q) c += g[q];
@@ -201,6 +201,15 @@ StArgs<C> make_st_args(const void *src, void *dst, NbrDev nbr, const void *u, co
     return a;
 }
 
+template <typename C, int NB>
+void launch_st_pull(const StArgs<C> &a, int32_t order, hipStream_t s)
+{
+    const dim3 g((unsigned)((a.N + NB - 1) / NB)), b(NB);
+    // a solute's own table has 16-bit ranks, that of a coupled flow may be narrow
+    a.nbr.narrow ? st_step_kernel<C, K_PULL, NB><<<g, b, 0, s>>>(a, order)
+                 : st_step_kernel<C, K_PULL, NB, LINK_16><<<g, b, 0, s>>>(a, order);
+}
+
 template <typename C>
 hipError_t launch_st_t(const StArgs<C> &a, int mode, int64_t grid, const lbm_launch &ls, hipStream_t s)
 {
@@ -210,11 +219,11 @@ hipError_t launch_st_t(const StArgs<C> &a, int mode, int64_t grid, const lbm_lau
     else if (mode == K_DIRECT)
         st_step_kernel<C, K_DIRECT><<<g, b, 0, s>>>(a, ls.order);
     else if (ls.block == 128)
-        st_step_kernel<C, K_PULL, 128><<<dim3((unsigned)((a.N + 127) / 128)), dim3(128), 0, s>>>(a, ls.order);
+        launch_st_pull<C, 128>(a, ls.order, s);
     else if (ls.block == 512)
-        st_step_kernel<C, K_PULL, 512><<<dim3((unsigned)((a.N + 511) / 512)), dim3(512), 0, s>>>(a, ls.order);
+        launch_st_pull<C, 512>(a, ls.order, s);
     else
-        st_step_kernel<C, K_PULL><<<g, b, 0, s>>>(a, ls.order);
+        launch_st_pull<C, BLOCK>(a, ls.order, s);
     return hipGetLastError();
 }
 

@@ -1087,9 +1087,12 @@ static hipError_t cg_launch_collide(CgArgs<ST> a, int mode, bool store_u, int64_
 }
 
 // the collide launch from buffer src to dst
-hipError_t CgSolver::launch_collide(int mode, bool store_u, const lbm_launch &ls, const void *src, void *dst)
+hipError_t CgSolver::launch_collide(int mode, bool store_u, const lbm_launch &set, const void *src, void *dst)
 {
     const int64_t N = geo_.N, P = geo_.P;
+    lbm_launch ls = set;
+    back_ = N >= BACK_NODES && dst == pops_[0];   // see BACK_NODES
+    if (back_) ls.order |= ORDER_BACK;
     if (prm_.precision == LBM_FP64)
         return cg_launch_collide(make_cg_args<double>(prm_, visc_, u_i_, src, dst, nbr_.view(), d_col_, d_psi_, d_cs_, d_u_,
                                                       d_rho_, N, P),
@@ -1100,8 +1103,11 @@ hipError_t CgSolver::launch_collide(int mode, bool store_u, const lbm_launch &ls
 }
 
 // the colour-streaming launch: gathers, or (FP32) the LDS-staged variant
-hipError_t CgSolver::launch_colour(const lbm_launch &ls)
+hipError_t CgSolver::launch_colour(const lbm_launch &set)
 {
+    lbm_launch ls = set;
+    // against the collide launch, whose last colour states it reads first
+    if (geo_.N >= BACK_NODES && !back_) ls.order |= ORDER_BACK;
     const int64_t N = geo_.N, P = geo_.P;
     const dim3 g((unsigned)grid_), b(BLOCK);
     const dim3 gw((unsigned)cw_grid_), bw(CW_BLOCK);

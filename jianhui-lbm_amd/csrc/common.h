@@ -52,12 +52,14 @@ __device__ __forceinline__ uint32_t xcd_slab_tile(uint32_t b, uint32_t grid)
 }
 
 // Tile orders a launch can use (chosen per kernel and geometry by the autotuner, or set through
-// lbm_set_launch): the hardware order, runs of 8 tiles per XCD, or one slab per XCD.
-enum TileOrder : int32_t { ORDER_HW = 0, ORDER_RUNS8 = 1, ORDER_SLAB = 2 };
+// lbm_set_launch): the hardware order, runs of 8 tiles per XCD, or one slab per XCD.  ORDER_BACK, set by
+// the handles (tune.h): from the last tile to the first.
+enum TileOrder : int32_t { ORDER_HW = 0, ORDER_RUNS8 = 1, ORDER_SLAB = 2, ORDER_BACK = 4 };
 __device__ __forceinline__ int64_t tile_of(int32_t order, uint32_t b, uint32_t grid)
 {
     const uint32_t runs = stream_tile(b, grid), slab = xcd_slab_tile(b, grid);
-    return order == ORDER_RUNS8 ? runs : (order == ORDER_SLAB ? slab : b);
+    const uint32_t t = (order & 3) == ORDER_RUNS8 ? runs : ((order & 3) == ORDER_SLAB ? slab : b);
+    return order & ORDER_BACK ? grid - 1 - t : t;
 }
 
 template <typename T>

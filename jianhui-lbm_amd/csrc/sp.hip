@@ -711,11 +711,13 @@ int SpSolver::load_state(const double *f, const double *u, const double *rho)
 
 // one step launch from buffer src to buffer dst; faces and the power law as the handle has them
 // unless bare (the autotuner's timing launches: the plain pull step, state untouched)
-hipError_t SpSolver::launch_kernel(int mode, bool store_u, const FusedSolute *fs, const lbm_launch &ls, const void *src,
+hipError_t SpSolver::launch_kernel(int mode, bool store_u, const FusedSolute *fs, const lbm_launch &set, const void *src,
                                    void *dst, bool bare)
 {
     // the power-law collision acts from the reference's loop step n = 11 on (SP:2397); the
     // launches since init or load_state are that loop's n
+    lbm_launch ls = set;
+    if (geo_.N >= BACK_NODES && dst == pops_[0]) ls.order |= ORDER_BACK;   // see BACK_NODES
     void *pl_nu = (!bare && d_nu_vn_ && steps_ > 10) ? d_nu_vn_ : nullptr;
     const BcDev bc = bare ? BcDev{nullptr, nullptr, nullptr, nullptr, 0} : bc_view(true);
     if (prm_.precision == LBM_FP64)

@@ -28,6 +28,13 @@ constexpr int64_t ST_SLAB_NODES = int64_t(1) << 18;
 // 16.2 -> 10.5 / 14.3 | 13.9 / 21.7 us, 131,072 16.4 / 26.8 -> 13.7 / 24.9 | 14.0 / 25.9, 184,320 22.3 /
 // 38.4 -> 20.1 / 37.8 | 23.4 / 44.9, 240,000 27.4 / 48.5 -> 26.4 / 48.3 | 24.2 / 47.6, 649,605 56.7 /
 // 109.2 -> 57.4 / 110.5 | 50.4 / 99.3, 921,600 77.3 / 153.9 -> 79.1 / 157.4 | 66.2 / 135.1.
+// From this size on, launches into one of the two buffers run through the tiles from the last to the
+// first, so that a step begins with what the one before has written last, some of it still in the
+// 256 MB memory-side cache; a colour launch runs against its collide launch.  Step on device: 171 x
+// 203 x 187 FP64 105.4 -> 103.6 us, 256^3 sphere pack FP32 167.1 -> 166.2 us, 192^3 fibres with solute
+// FP32 213.0 -> 212.1 us, colour gradient 192^3 FP32 209.8 -> 207.4 us and FP64 443.3 -> 437.3 us (colour
+// launch with its collide launch: 209.3 and 441.2 us).  Smaller boxes fit the cache in any order.
+constexpr int64_t BACK_NODES = int64_t(1) << 20;
 constexpr int64_t CG_STAGED_NODES = 215000;
 constexpr double CG_STAGED_FAST = 0.85;
 constexpr int64_t CG_SMALL_NODES = int64_t(1) << 15;   // 128-node collide tiles: 16,384 nodes 9.8 -> 9.3 us, 55,296 10.5 -> 10.9

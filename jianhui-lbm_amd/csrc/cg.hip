@@ -154,7 +154,7 @@ __device__ __forceinline__ void cg_node_state(const CgArgs<ST> &a, int64_t n, ty
 // One node of the collide kernel.  SLOTS > 0 and FAST: the phase field of the block's
 // neighbourhood is in LDS (lpsi, at the slots of ColourWin w); otherwise it is read from global
 // memory.  A lane that is not live stores nothing.
-template <typename ST, int MODE, bool STORE_U, int SLOTS, bool FAST>
+template <typename ST, int MODE, bool STORE_U, int SLOTS, bool FAST, int SK>
 __device__ __forceinline__ void cg_collide_node(const CgArgs<ST> &a, int64_t n, bool live, const typename Store<ST>::C *lpsi,
                                                 const ColourWin &w)
 {
@@ -221,8 +221,15 @@ __device__ __forceinline__ void cg_collide_node(const CgArgs<ST> &a, int64_t n, 
         a.u_aux[2 * a.P + n] = mc.uz;
     }
     cg_relax(m, mc, gx, gy, gz, sv, a.cap_a * cc, nx, ny, nz, h);
+    if (store_keeps<SK>(a.order)) {
+        KEEP_APART();
 #pragma unroll
-    for (int q = 0; q < Q; ++q) Store<ST>::store_nt(&a.dst[pop_at<Q>(q, n)], h[q], a.scale);
+        for (int q = 0; q < Q; ++q) a.dst[pop_at<Q>(q, n)] = Store<ST>::put(h[q], a.scale);
+        KEEP_APART();
+    } else {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) Store<ST>::store_nt(&a.dst[pop_at<Q>(q, n)], h[q], a.scale);
+    }
     const C st[6] = {mc.ux, mc.uy, mc.uz, nx, ny, nz};
     store_cs(a.cs, n, a.P, rr_raw, rb_raw, st);
 }
@@ -231,7 +238,7 @@ __device__ __forceinline__ void cg_collide_node(const CgArgs<ST> &a, int64_t n, 
 // runs of node ids of the colour kernel's staging (ColourWin) -- is copied to LDS first, and the
 // colour gradient reads its 18 neighbour values from there; a block with a read outside its runs
 // reads them from global memory.
-template <typename ST, int MODE, bool STORE_U, int NB = BLOCK, int SLOTS = 0>
+template <typename ST, int MODE, bool STORE_U, int NB = BLOCK, int SLOTS = 0, int SK = STORE_ANY>
 __global__ void __launch_bounds__(NB) cg_collide_kernel(CgArgs<ST> a)
 {
     using C = typename Store<ST>::C;
@@ -255,9 +262,9 @@ __global__ void __launch_bounds__(NB) cg_collide_kernel(CgArgs<ST> a)
     }
     if (SLOTS > 0 && !live) return;   // its slots may lie past the block's
     if (SLOTS > 0 && w.fast == CW_ALL)
-        cg_collide_node<ST, MODE, STORE_U, SLOTS, true>(a, n, live, lpsi, w);
+        cg_collide_node<ST, MODE, STORE_U, SLOTS, true, SK>(a, n, live, lpsi, w);
     else
-        cg_collide_node<ST, MODE, STORE_U, SLOTS, false>(a, n, live, lpsi, w);
+        cg_collide_node<ST, MODE, STORE_U, SLOTS, false, SK>(a, n, live, lpsi, w);
 }
 
 // e_q . (x, y, z) with the zero components left out (0 * v is not folded away in IEEE arithmetic)
@@ -1052,12 +1059,16 @@ int CgSolver::set_body_force(const double g[3])
     return LBM_OK;
 }
 
+// what a step reads and writes: populations (twice), colour states, colour densities, phase field, links
+static int64_t cg_step_bytes(int64_t P, size_t st) { return P * (int64_t)((2 * Q + 11) * st + 19); }
+
 template <typename ST, int NB, int SLOTS = 0>
 static void cg_launch_pull(const CgArgs<ST> &a, bool store_u, hipStream_t s)
 {
     const dim3 g((unsigned)((a.N + NB - 1) / NB)), b(NB);
-    store_u ? cg_collide_kernel<ST, K_PULL, true, NB, SLOTS><<<g, b, 0, s>>>(a)
-            : cg_collide_kernel<ST, K_PULL, false, NB, SLOTS><<<g, b, 0, s>>>(a);
+    if (store_u) cg_collide_kernel<ST, K_PULL, true, NB, SLOTS><<<g, b, 0, s>>>(a);
+    else if (a.order & ORDER_KEEP) cg_collide_kernel<ST, K_PULL, false, NB, SLOTS, STORE_KEEP><<<g, b, 0, s>>>(a);
+    else cg_collide_kernel<ST, K_PULL, false, NB, SLOTS, STORE_NT><<<g, b, 0, s>>>(a);
 }
 
 template <typename ST>
@@ -1065,7 +1076,7 @@ static hipError_t cg_launch_collide(CgArgs<ST> a, int mode, bool store_u, int64_
                                     const lbm_launch &ls, const void *wins, int slots, hipStream_t s)
 {
     dim3 g((unsigned)grid), b(BLOCK);
-    a.order = ls.order;
+    a.order = ls.order | (keep_stores(cg_step_bytes(a.P, sizeof(ST)), a.P * (int64_t)(Q * sizeof(ST)), sizeof(ST)) ? ORDER_KEEP : 0);
     a.wins = (const ColourWin *)wins;
     if (mode == K_PULL && ls.variant == LBM_VARIANT_STAGED && slots == 1024)
         cg_launch_pull<ST, CW_BLOCK, 1024>(a, store_u, s);
@@ -1091,7 +1102,7 @@ hipError_t CgSolver::launch_collide(int mode, bool store_u, const lbm_launch &se
 {
     const int64_t N = geo_.N, P = geo_.P;
     lbm_launch ls = set;
-    back_ = N >= BACK_NODES && dst == pops_[0];   // see BACK_NODES
+    back_ = N >= BACK_NODES && !fits_cache(cg_step_bytes(P, ct_bytes_)) && dst == pops_[0];
     if (back_) ls.order |= ORDER_BACK;
     if (prm_.precision == LBM_FP64)
         return cg_launch_collide(make_cg_args<double>(prm_, visc_, u_i_, src, dst, nbr_.view(), d_col_, d_psi_, d_cs_, d_u_,
@@ -1107,7 +1118,7 @@ hipError_t CgSolver::launch_colour(const lbm_launch &set)
 {
     lbm_launch ls = set;
     // against the collide launch, whose last colour states it reads first
-    if (geo_.N >= BACK_NODES && !back_) ls.order |= ORDER_BACK;
+    if (geo_.N >= BACK_NODES && !fits_cache(cg_step_bytes(geo_.P, ct_bytes_)) && !back_) ls.order |= ORDER_BACK;
     const int64_t N = geo_.N, P = geo_.P;
     const dim3 g((unsigned)grid_), b(BLOCK);
     const dim3 gw((unsigned)cw_grid_), bw(CW_BLOCK);

@@ -53,13 +53,24 @@ __device__ __forceinline__ uint32_t xcd_slab_tile(uint32_t b, uint32_t grid)
 
 // Tile orders a launch can use (chosen per kernel and geometry by the autotuner, or set through
 // lbm_set_launch): the hardware order, runs of 8 tiles per XCD, or one slab per XCD.  ORDER_BACK, set by
-// the handles (tune.h): from the last tile to the first.
-enum TileOrder : int32_t { ORDER_HW = 0, ORDER_RUNS8 = 1, ORDER_SLAB = 2, ORDER_BACK = 4 };
+// the handles (tune.h): from the last tile to the first.  ORDER_KEEP: stores without the nontemporal hint.
+enum TileOrder : int32_t { ORDER_HW = 0, ORDER_RUNS8 = 1, ORDER_SLAB = 2, ORDER_BACK = 4, ORDER_KEEP = 8 };
 __device__ __forceinline__ int64_t tile_of(int32_t order, uint32_t b, uint32_t grid)
 {
     const uint32_t runs = stream_tile(b, grid), slab = xcd_slab_tile(b, grid);
     const uint32_t t = (order & 3) == ORDER_RUNS8 ? runs : ((order & 3) == ORDER_SLAB ? slab : b);
     return order & ORDER_BACK ? grid - 1 - t : t;
+}
+
+// How a step stores its populations: with the nontemporal hint, without it, or as the launch's order
+// says (ORDER_KEEP).  A kernel with both kinds of stores is slower where it is compiled for it (colour
+// gradient 192^3 FP32 207 -> 219 us, 208 x 224 x 240 FP16 69.3 -> 70.6 us), so the step kernels that
+// run nearly all steps are compiled for one.
+enum StoreKind : int { STORE_NT = 0, STORE_KEEP = 1, STORE_ANY = 2 };
+template <int KIND>
+__device__ __forceinline__ bool store_keeps(int32_t order)
+{
+    return KIND == STORE_ANY ? (order & ORDER_KEEP) != 0 : KIND == STORE_KEEP;
 }
 
 template <typename T>

@@ -46,6 +46,7 @@
 #include "handle.h"
 #include "pull.h"
 #include "storage.h"
+#include "tune.h"
 
 namespace lbm {
 
@@ -117,11 +118,12 @@ __global__ void __launch_bounds__(BLK) srv_step_kernel(const TileDev *__restrict
                                                        const ST *__restrict__ src, ST *__restrict__ dst,
                                                        const int16_t *__restrict__ nbr,
                                                        const int16_t *__restrict__ nbr_hi, int64_t step,
-                                                       int64_t tile0)
+                                                       int64_t tile0, bool keep)
 {
     using C = typename Store<ST>::C;
     constexpr uint32_t SZ = sizeof(ST);
-    const TileDev t = tiles[tile0 + stream_tile(blockIdx.x, gridDim.x)];
+    const uint32_t runs = stream_tile(blockIdx.x, gridDim.x), slab = xcd_slab_tile(blockIdx.x, gridDim.x);
+    const TileDev t = tiles[tile0 + (keep ? slab : runs)];
     const int64_t n = t.begin + threadIdx.x;
     if (n >= t.end) return;
     const SlotDev sl = slots[t.slot];
@@ -165,8 +167,15 @@ __global__ void __launch_bounds__(BLK) srv_step_kernel(const TileDev *__restrict
     }
     sp_relax(m, mc, gx, gy, gz, (C)sl.sv, (C)sl.sq, h);
     ST *__restrict__ D = dst + t.base * Q;
+    if (keep) {
+        KEEP_APART();
 #pragma unroll
-    for (int q = 0; q < Q; ++q) Store<ST>::store_nt(byte_at(D, own + row_bytes(q, SZ)), h[q], 1.0f);
+        for (int q = 0; q < Q; ++q) *byte_at(D, own + row_bytes(q, SZ)) = Store<ST>::put(h[q], 1.0f);
+        KEEP_APART();
+    } else {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) Store<ST>::store_nt(byte_at(D, own + row_bytes(q, SZ)), h[q], 1.0f);
+    }
 }
 
 // per-tile flux partials Q[3] and a non-finite flag, from the current (pulled) state
@@ -1382,12 +1391,13 @@ void Server::launch_step()
     const int64_t nn = ntiles_narrow_, nw = ntiles_ - ntiles_narrow_;
     const ST *src = (const ST *)pops_[cur_];
     ST *dst = (ST *)pops_[cur_ ^ 1];
+    const bool keep = fits_cache(ntiles_ * BLK * (2 * Q * (int64_t)sizeof(ST) + 2 * (Q - 1)));
     if (nn > 0)
         srv_step_kernel<ST, BLK, false, FIRST><<<(unsigned)nn, BLK, 0, stream_>>>(d_tiles_, d_slots_, src, dst, d_nbr_,
-                                                                                  d_nbr_hi_, global_step_, 0);
+                                                                                  d_nbr_hi_, global_step_, 0, keep);
     if (nw > 0)
         srv_step_kernel<ST, BLK, true, FIRST><<<(unsigned)nw, BLK, 0, stream_>>>(d_tiles_, d_slots_, src, dst, d_nbr_,
-                                                                                 d_nbr_hi_, global_step_, nn);
+                                                                                 d_nbr_hi_, global_step_, nn, keep);
 }
 
 // Samples are admitted between calls, so only a call's first step can be a sample's first.

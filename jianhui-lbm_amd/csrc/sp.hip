@@ -127,8 +127,10 @@ __device__ __forceinline__ Macro<typename Store<ST>::C> node_macro(const SpArgs<
 // their rule, and every launch saves the pre-collision state of the nodes the rules read.
 // PL: power-law collision (pull launches of reference steps n > 10, SP:2397).
 // FUSED: also the step of a coupled solute (pull launches).
-// NB: nodes (threads) per workgroup; a.order: the tile order; LF: how links are followed (nbrpack.h).
-template <typename ST, int MODE, bool STORE_U, bool BC, bool PL = false, bool FUSED = false, int NB = BLOCK, int LF = LINK_FAR>
+// NB: nodes (threads) per workgroup; a.order: the tile order; LF: how links are followed (nbrpack.h);
+// SK: how populations are stored.
+template <typename ST, int MODE, bool STORE_U, bool BC, bool PL = false, bool FUSED = false, int NB = BLOCK, int LF = LINK_FAR,
+          int SK = STORE_ANY>
 __global__ void __launch_bounds__(NB) sp_step_kernel(SpArgs<ST> a)
 {
     using C = typename Store<ST>::C;
@@ -166,12 +168,21 @@ __global__ void __launch_bounds__(NB) sp_step_kernel(SpArgs<ST> a)
 #pragma unroll
             for (int q = 1; q < 7; ++q) c += g[q];
             const C wc = a.st.wq * c;
-            __builtin_nontemporal_store(g[0] - a.st.omega * (g[0] - a.st.w0 * c), &a.st.dst[pop_at<7>(0, n)]);
+            g[0] = g[0] - a.st.omega * (g[0] - a.st.w0 * c);
 #pragma unroll
             for (int q = 1; q < 7; ++q) {
                 const C eu = q == 1 ? mc.ux : q == 2 ? -mc.ux : q == 3 ? mc.uy : q == 4 ? -mc.uy : q == 5 ? mc.uz : -mc.uz;
                 const C eq = wc * (C(1) + eu * a.st.inv_cs2);
-                __builtin_nontemporal_store(g[q] - a.st.omega * (g[q] - eq), &a.st.dst[pop_at<7>(q, n)]);
+                g[q] = g[q] - a.st.omega * (g[q] - eq);
+            }
+            if (store_keeps<SK>(a.order)) {
+                KEEP_APART();
+#pragma unroll
+                for (int q = 0; q < 7; ++q) a.st.dst[pop_at<7>(q, n)] = g[q];
+                KEEP_APART();
+            } else {
+#pragma unroll
+                for (int q = 0; q < 7; ++q) __builtin_nontemporal_store(g[q], &a.st.dst[pop_at<7>(q, n)]);
             }
         }
     }
@@ -183,8 +194,15 @@ __global__ void __launch_bounds__(NB) sp_step_kernel(SpArgs<ST> a)
     C sv = a.sv, sq = a.sq;
     if (PL && MODE == K_PULL) power_law_rates(h, mc, a.nu_vn, n, a.pl_m, a.pl_n, sv, sq);
     sp_relax(m, mc, a.gx, a.gy, a.gz, sv, sq, h);
+    if (store_keeps<SK>(a.order)) {
+        KEEP_APART();
 #pragma unroll
-    for (int q = 0; q < Q; ++q) Store<ST>::store_nt(&a.dst[pop_at<Q>(q, n)], h[q], a.scale);
+        for (int q = 0; q < Q; ++q) a.dst[pop_at<Q>(q, n)] = Store<ST>::put(h[q], a.scale);
+        KEEP_APART();
+    } else {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) Store<ST>::store_nt(&a.dst[pop_at<Q>(q, n)], h[q], a.scale);
+    }
 }
 
 template <typename C>
@@ -399,6 +417,9 @@ SpArgs<ST> make_args(const void *src, void *dst, const NbrDev &nbr, void *u_aux,
     return a;
 }
 
+// what a step reads and writes: populations (19 rows of st bytes, twice), links, a solute's rows
+int64_t sp_step_bytes(int64_t P, size_t st, size_t solute) { return P * (int64_t)(2 * Q * st + solute + 19); }
+
 // the pull step without faces or power law, at a workgroup size NB
 template <typename ST, bool FUSED, int NB>
 void launch_pull_nb(const SpArgs<ST> &a, bool store_u, int64_t N, hipStream_t s)
@@ -407,8 +428,12 @@ void launch_pull_nb(const SpArgs<ST> &a, bool store_u, int64_t N, hipStream_t s)
     // a coupled solute's 7 rows are of the compute type
     const int lf = link_form(a.nbr, (uint64_t)a.P * std::max(Q * sizeof(ST), FUSED ? 7 * sizeof(typename Store<ST>::C) : 0));
     if (store_u) sp_step_kernel<ST, K_PULL, true, false, false, FUSED, NB><<<g, b, 0, s>>>(a);
-    else if (lf == LINK_16) sp_step_kernel<ST, K_PULL, false, false, false, FUSED, NB, LINK_16><<<g, b, 0, s>>>(a);
-    else if (lf == LINK_8) sp_step_kernel<ST, K_PULL, false, false, false, FUSED, NB, LINK_8><<<g, b, 0, s>>>(a);
+    else if (lf == LINK_16)
+        a.order & ORDER_KEEP ? sp_step_kernel<ST, K_PULL, false, false, false, FUSED, NB, LINK_16, STORE_KEEP><<<g, b, 0, s>>>(a)
+                             : sp_step_kernel<ST, K_PULL, false, false, false, FUSED, NB, LINK_16, STORE_NT><<<g, b, 0, s>>>(a);
+    else if (lf == LINK_8)
+        a.order & ORDER_KEEP ? sp_step_kernel<ST, K_PULL, false, false, false, FUSED, NB, LINK_8, STORE_KEEP><<<g, b, 0, s>>>(a)
+                             : sp_step_kernel<ST, K_PULL, false, false, false, FUSED, NB, LINK_8, STORE_NT><<<g, b, 0, s>>>(a);
     else sp_step_kernel<ST, K_PULL, false, false, false, FUSED, NB><<<g, b, 0, s>>>(a);
 }
 template <typename ST, int NB>
@@ -459,6 +484,9 @@ hipError_t launch_step_t(SpArgs<ST> a, const BcDev &bc, void *nu_vn, double pl_m
         a.st.wq = (C)fs->wq;
         a.st.inv_cs2 = (C)fs->inv_cs2;
     }
+    const size_t solute = fs ? 7 * sizeof(C) : 0;
+    if (keep_stores(sp_step_bytes(a.P, sizeof(ST), 2 * solute), a.P * (int64_t)(Q * sizeof(ST) + solute), sizeof(ST)))
+        a.order |= ORDER_KEEP;
     if (mode == K_PULL && !bc.wave && !nu_vn) {
         if (ls.block == 128)
             launch_pull<ST, 128>(a, store_u, a.N, s);
@@ -611,6 +639,7 @@ int SpSolver::create(const lbm_sp_params &p, const int32_t *solid)
 int SpSolver::autotune()
 {
     if (geo_.N < SP_SLAB_NODES) launch_ = lbm_launch{128, ORDER_SLAB, 0, 0, 0.0};
+    else if (geo_.N >= SP_KEEP_SLAB_NODES && fits_cache(sp_step_bytes(geo_.P, st_bytes_, 0))) launch_.order = ORDER_SLAB;
     if (geo_.N < TUNE_MIN_NODES) return LBM_OK;
     lbm_launch c;
     if (tune_cache_get(LBM_KERNEL_SP_STEP, prm_.precision, geo_.N, c)) {
@@ -717,7 +746,7 @@ hipError_t SpSolver::launch_kernel(int mode, bool store_u, const FusedSolute *fs
     // the power-law collision acts from the reference's loop step n = 11 on (SP:2397); the
     // launches since init or load_state are that loop's n
     lbm_launch ls = set;
-    if (geo_.N >= BACK_NODES && dst == pops_[0]) ls.order |= ORDER_BACK;   // see BACK_NODES
+    if (geo_.N >= BACK_NODES && !fits_cache(sp_step_bytes(geo_.P, st_bytes_, 0)) && dst == pops_[0]) ls.order |= ORDER_BACK;
     void *pl_nu = (!bare && d_nu_vn_ && steps_ > 10) ? d_nu_vn_ : nullptr;
     const BcDev bc = bare ? BcDev{nullptr, nullptr, nullptr, nullptr, 0} : bc_view(true);
     if (prm_.precision == LBM_FP64)

@@ -83,16 +83,19 @@ __global__ void __launch_bounds__(NB) st_step_kernel(StArgs<C> a, int32_t order)
     }
     if (n_own >= a.N) return;
     const C wc = a.wq * c;
-    {
-        const C eq = a.w0 * c;
-        const C v = MODE == K_INIT ? eq : g[0] - a.omega * (g[0] - eq);
-        __builtin_nontemporal_store(v, &a.dst[pop_at<Q7>(0, n)]);
-    }
 #pragma unroll
-    for (int q = 1; q < Q7; ++q) {
-        const C eq = wc * (C(1) + axis_dot(q, ux, uy, uz) * a.inv_cs2);
-        const C v = MODE == K_INIT ? eq : g[q] - a.omega * (g[q] - eq);
-        __builtin_nontemporal_store(v, &a.dst[pop_at<Q7>(q, n)]);
+    for (int q = 0; q < Q7; ++q) {
+        const C eq = q == 0 ? a.w0 * c : wc * (C(1) + axis_dot(q, ux, uy, uz) * a.inv_cs2);
+        g[q] = MODE == K_INIT ? eq : g[q] - a.omega * (g[q] - eq);
+    }
+    if (order & ORDER_KEEP) {
+        KEEP_APART();
+#pragma unroll
+        for (int q = 0; q < Q7; ++q) a.dst[pop_at<Q7>(q, n)] = g[q];
+        KEEP_APART();
+    } else {
+#pragma unroll
+        for (int q = 0; q < Q7; ++q) __builtin_nontemporal_store(g[q], &a.dst[pop_at<Q7>(q, n)]);
     }
 }
 
@@ -205,6 +208,7 @@ template <typename C, int NB>
 void launch_st_pull(const StArgs<C> &a, int32_t order, hipStream_t s)
 {
     const dim3 g((unsigned)((a.N + NB - 1) / NB)), b(NB);
+    if (fits_cache(a.P * (int64_t)(17 * sizeof(C) + 11))) order |= ORDER_KEEP;   // populations, velocity, links
     // a solute's own table has 16-bit ranks, that of a coupled flow may be narrow
     a.nbr.narrow ? st_step_kernel<C, K_PULL, NB><<<g, b, 0, s>>>(a, order)
                  : st_step_kernel<C, K_PULL, NB, LINK_16><<<g, b, 0, s>>>(a, order);
@@ -237,6 +241,7 @@ int st_kmode(StateMode m) { return m == STATE_INIT ? K_INIT : (m == STATE_DIRECT
 int StSolver::autotune()
 {
     if (N_ < ST_SLAB_NODES) launch_ = launch_own_ = lbm_launch{128, ORDER_SLAB, 0, 0, 0.0};
+    else if (fits_cache(P_ * (int64_t)(52 * st_bytes_ + 19))) launch_.order = launch_own_.order = ORDER_SLAB;
     if (N_ < TUNE_MIN_NODES) return LBM_OK;
     const int kind = flow_ ? -LBM_KERNEL_ST_STEP : LBM_KERNEL_ST_STEP;   // separate cache entries
     lbm_launch c;

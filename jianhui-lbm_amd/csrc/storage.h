@@ -6,12 +6,17 @@
 //
 // store_nt writes a post-collision value with a nontemporal hint: the next read of it is a
 // whole time step away, so keeping it out of the caches leaves them to the pull gathers
-// (measured 4 % faster on the 256^3 single-phase step).
+// (measured 4 % faster on the 256^3 single-phase step).  Steps whose arrays fit the memory-side cache
+// store without it (keep_stores, tune.h).
 #pragma once
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
 namespace lbm {
+
+// At both ends of the stores without the hint: keeps the compiler from merging them with the ones on
+// the other side of the branch, which would leave neither with it.
+#define KEEP_APART() asm volatile("")
 
 template <typename ST>
 struct Store;

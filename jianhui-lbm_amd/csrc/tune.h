@@ -20,7 +20,7 @@ constexpr int64_t TUNE_MIN_NODES = int64_t(1) << 20;
 // (398,131 FP32 16.2 -> 15.8, FP64 27.0 -> 26.7, above the line: no gain worth a setting); solute
 // 26,214 nodes 3.07 -> 2.75, 209,715 4.22 -> 3.90, with the flow 5.36 -> 4.71 and 12.6 -> 11.6 us
 // (707,788: 11.7 -> 11.7 and 31.3 -> 32.5).
-constexpr int64_t SP_SLAB_NODES = int64_t(1) << 17;
+constexpr int64_t SP_SLAB_NODES = int64_t(1) << 17, SP_KEEP_SLAB_NODES = int64_t(1) << 18;
 constexpr int64_t ST_SLAB_NODES = int64_t(1) << 18;
 // Colour gradient, both launches in slabs (one gathers what the other has just written), collide
 // and colour gathering below the line, staged above it where most blocks read from their runs.
@@ -28,16 +28,33 @@ constexpr int64_t ST_SLAB_NODES = int64_t(1) << 18;
 // 16.2 -> 10.5 / 14.3 | 13.9 / 21.7 us, 131,072 16.4 / 26.8 -> 13.7 / 24.9 | 14.0 / 25.9, 184,320 22.3 /
 // 38.4 -> 20.1 / 37.8 | 23.4 / 44.9, 240,000 27.4 / 48.5 -> 26.4 / 48.3 | 24.2 / 47.6, 649,605 56.7 /
 // 109.2 -> 57.4 / 110.5 | 50.4 / 99.3, 921,600 77.3 / 153.9 -> 79.1 / 157.4 | 66.2 / 135.1.
-// From this size on, launches into one of the two buffers run through the tiles from the last to the
-// first, so that a step begins with what the one before has written last, some of it still in the
-// 256 MB memory-side cache; a colour launch runs against its collide launch.  Step on device: 171 x
-// 203 x 187 FP64 105.4 -> 103.6 us, 256^3 sphere pack FP32 167.1 -> 166.2 us, 192^3 fibres with solute
-// FP32 213.0 -> 212.1 us, colour gradient 192^3 FP32 209.8 -> 207.4 us and FP64 443.3 -> 437.3 us (colour
-// launch with its collide launch: 209.3 and 441.2 us).  Smaller boxes fit the cache in any order.
-constexpr int64_t BACK_NODES = int64_t(1) << 20;
 constexpr int64_t CG_STAGED_NODES = 215000;
 constexpr double CG_STAGED_FAST = 0.85;
 constexpr int64_t CG_SMALL_NODES = int64_t(1) << 15;   // 128-node collide tiles: 16,384 nodes 9.8 -> 9.3 us, 55,296 10.5 -> 10.9
+// Steps whose arrays fit the 256 MB memory-side cache together store without the nontemporal hint, so
+// that the next step finds them there, and from 2^18 nodes on run in slabs, 256 nodes a tile.  Step on
+// device, hint -> none -> none and slabs: single phase FP64 256,000 nodes 17.6 -> 15.4 -> 13.4 us,
+// 702,464 (227 MB) 41.7 -> 39.7 -> 34.4, 1,048,576 (339 MB) 59.4 -> 63.7; FP32 442,368 16.8 -> 15.2 -> 13.0,
+// 1,492,992 (255 MB) 45.7 -> 37.9, 2,048,000 (350 MB) 61.4 -> 69.2; FP16 702,464 18.6 -> 16.9 -> 16.0;
+// 815,257 nodes FP32 with faces and power law 30.3 -> 25.0; colour gradient FP32 864,000 (185 MB) 67.4 -> 56.5,
+// 1,492,992 (321 MB) 104.2 -> 105.4, FP64 562,432 91.4 -> 80.7; solute FP32 530,841 9.0 -> 8.3 -> 7.3, with the
+// flow 25.6 -> 23.7 -> 20.0; sixteen served samples of edges 32 to 88 155 -> 140 ms a batch.
+constexpr int64_t CACHE_BYTES = 256000000;
+inline bool fits_cache(int64_t step_bytes) { return step_bytes <= CACHE_BYTES; }
+// Values of 2 and 4 bytes keep the hint where a buffer has 4.5 to 12 MB, in which its stores were the
+// slower ones without it: FP32 131,072 nodes 6.73 -> 7.04 us, 186,624 (14 MB) 8.99 -> 8.19; FP16 131,072 5.6 ->
+// 5.9, 256,000 8.0 -> 8.4, 340,736 (13 MB) 10.6 -> 10.3; but FP64 70,304 (11 MB) 5.9 -> 5.65.
+inline bool keep_stores(int64_t step_bytes, int64_t buffer_bytes, size_t width)
+{
+    return fits_cache(step_bytes) && (width > 4 || buffer_bytes < 4500000 || buffer_bytes > 12000000);
+}
+// Where they do not fit, from this size on, launches into one of the two buffers run through the tiles
+// from the last to the first, so that a step begins with what the one before has written last, some of
+// it still in that cache; a colour launch runs against its collide launch.  Step on device: 171 x 203 x
+// 187 FP64 105.4 -> 103.6 us, 256^3 sphere pack FP32 167.1 -> 166.2 us, 192^3 fibres with solute FP32
+// 213.0 -> 212.1 us, colour gradient 192^3 FP32 209.8 -> 207.4 us and FP64 443.3 -> 437.3 us (colour launch
+// with its collide launch: 209.3 and 441.2 us).
+constexpr int64_t BACK_NODES = int64_t(1) << 20;
 // an alternative replaces the default only when it is faster by this fraction
 constexpr double TUNE_MARGIN = 0.01;
 

@@ -14,32 +14,39 @@ def _same(a, b):
     return all(np.array_equal(x, y) for x, y in zip(a, b))
 
 
-@pytest.mark.parametrize("edge,small", [(5, True), (50, True), (51, False)])   # line at 131,072 nodes
-def test_single_phase(pkg, edge, small):
+# lines at 131,072 nodes and, for steps that fit the memory-side cache (FP64: 792,569 nodes), at 262,144
+@pytest.mark.parametrize("precision,edge,want", [("fp32", 5, (128, "slab")), ("fp32", 50, (128, "slab")),
+                                                 ("fp32", 51, (256, "runs8")), ("fp32", 63, (256, "runs8")),
+                                                 ("fp32", 64, (256, "slab")), ("fp16", 66, (256, "slab")),
+                                                 ("fp64", 92, (256, "slab")), ("fp64", 93, (256, "runs8"))])
+def test_single_phase(pkg, precision, edge, want):
     states = []
     for fixed in (False, True):
-        s = pkg.SinglePhase(_box(edge), 0.1, (1e-5, 0, 0), precision="fp32")
+        s = pkg.SinglePhase(_box(edge), 0.1, (1e-5, 0, 0), precision=precision)
         if fixed:
             s.set_launch(256, "hw")
         else:
-            assert (s.launch()["block"], s.launch()["order"]) == ((128, "slab") if small else (256, "runs8"))
+            assert (s.launch()["block"], s.launch()["order"]) == want
         s.init(1.0, (0.01, 0.0, 0.0))
         s.step(4)
         states.append(s.state())
     assert _same(*states)
 
 
-@pytest.mark.parametrize("edge,small", [(5, True), (64, False)])               # line at 262,144 nodes
+# line at 262,144 nodes, and where the steps stop to fit the memory-side cache (FP64: 588,505 nodes)
+@pytest.mark.parametrize("precision,edge,want", [("fp32", 5, (128, "slab")), ("fp32", 63, (128, "slab")),
+                                                 ("fp32", 64, (256, "slab")), ("fp64", 83, (256, "slab")),
+                                                 ("fp64", 84, (256, "hw"))])
 @pytest.mark.parametrize("coupled", [False, True])
-def test_solute(pkg, edge, small, coupled):
+def test_solute(pkg, precision, edge, want, coupled):
     states = []
     for fixed in (False, True):
-        flow = pkg.SinglePhase(_box(edge), 0.1, (1e-5, 0, 0), precision="fp32") if coupled else None
-        st = pkg.Solute(0.02, solid=None if coupled else _box(edge), flow=flow, precision="fp32")
+        flow = pkg.SinglePhase(_box(edge), 0.1, (1e-5, 0, 0), precision=precision) if coupled else None
+        st = pkg.Solute(0.02, solid=None if coupled else _box(edge), flow=flow, precision=precision)
         if fixed:
             st.set_launch(256, "runs8")
         else:
-            assert (st.launch()["block"], st.launch()["order"]) == ((128, "slab") if small else (256, "hw"))
+            assert (st.launch()["block"], st.launch()["order"]) == want
         st.init(np.random.default_rng(4).uniform(size=(edge,) * 3))
         st.step(4)
         states.append(st.state())

@@ -111,8 +111,9 @@ constexpr uint32_t row_bytes(int row, uint32_t size) { return (uint32_t)row * PO
 // (behind the branch the compiler asked for them in three batches).
 // Sixteen samples of edges 32 to 88, rows of CAP nodes and the branch -> blocks of 256 and no branch:
 // 27,900 -> 29,300 million node updates a second in FP32, 15,900 -> 17,100 in FP64; one sample of
-// 8,753 nodes 4.0 -> 3.8 us a step.  (Blocks with the branch: 28,300 and 16,900.  A slab of tiles for
-// each XCD gains nothing here: 3.8 us as well.)
+// 8,753 nodes 4.0 -> 3.8 us a step.  (Blocks with the branch: 28,300 and 16,900.)
+// keep: the active samples fit the memory-side cache (fits_cache, tune.h); their tiles run in slabs and
+// the stores carry no hint: such a batch with samples that do not converge 149 -> 139 ms.
 template <typename ST, int BLK, bool WIDE, bool FIRST>
 __global__ void __launch_bounds__(BLK) srv_step_kernel(const TileDev *__restrict__ tiles, const SlotDev *__restrict__ slots,
                                                        const ST *__restrict__ src, ST *__restrict__ dst,

@@ -11,7 +11,7 @@
 //   pops[2]  19 x P  storage type (double / float / half), deviations f - w*rho0, in blocks of
 //            256 nodes (pop_at, lattice.h)
 //   nbr      packed upstream node of direction q = 1..18 or bounce back (nbrpack.h): 8 x P
-//            uint16 column ranks + a header per wave
+//            16-bit or 8-bit column ranks + a header per wave
 //   u_aux     3 x P  compute type, u of the previous step (for the Error diagnostic)
 //   rho_aux   1 x P  compute type, density of a loaded checkpoint (first step only)
 #include <algorithm>
@@ -420,26 +420,29 @@ SpArgs<ST> make_args(const void *src, void *dst, const NbrDev &nbr, void *u_aux,
 // what a step reads and writes: populations (19 rows of st bytes, twice), links, a solute's rows
 int64_t sp_step_bytes(int64_t P, size_t st, size_t solute) { return P * (int64_t)(2 * Q * st + solute + 19); }
 
-// the pull step without faces or power law, at a workgroup size NB
-template <typename ST, bool FUSED, int NB>
+// The pull step at a workgroup size NB, in the form that the box allows.  Steps with faces or power law,
+// general form -> this: 256^3 sphere pack FP32 173.7 -> 171.7 and 178.4 -> 175.9 us, 131,072 nodes FP64 with
+// power law 11.2 -> 10.9, 2.05 M nodes FP16 with faces 36.4 -> 34.7.
+template <typename ST, bool BC, bool PL, bool FUSED, int NB>
 void launch_pull_nb(const SpArgs<ST> &a, bool store_u, int64_t N, hipStream_t s)
 {
     const dim3 g((unsigned)((N + NB - 1) / NB)), b(NB);
     // a coupled solute's 7 rows are of the compute type
     const int lf = link_form(a.nbr, (uint64_t)a.P * std::max(Q * sizeof(ST), FUSED ? 7 * sizeof(typename Store<ST>::C) : 0));
-    if (store_u) sp_step_kernel<ST, K_PULL, true, false, false, FUSED, NB><<<g, b, 0, s>>>(a);
+    if (store_u) sp_step_kernel<ST, K_PULL, true, BC, PL, FUSED, NB><<<g, b, 0, s>>>(a);
     else if (lf == LINK_16)
-        a.order & ORDER_KEEP ? sp_step_kernel<ST, K_PULL, false, false, false, FUSED, NB, LINK_16, STORE_KEEP><<<g, b, 0, s>>>(a)
-                             : sp_step_kernel<ST, K_PULL, false, false, false, FUSED, NB, LINK_16, STORE_NT><<<g, b, 0, s>>>(a);
+        a.order & ORDER_KEEP ? sp_step_kernel<ST, K_PULL, false, BC, PL, FUSED, NB, LINK_16, STORE_KEEP><<<g, b, 0, s>>>(a)
+                             : sp_step_kernel<ST, K_PULL, false, BC, PL, FUSED, NB, LINK_16, STORE_NT><<<g, b, 0, s>>>(a);
     else if (lf == LINK_8)
-        a.order & ORDER_KEEP ? sp_step_kernel<ST, K_PULL, false, false, false, FUSED, NB, LINK_8, STORE_KEEP><<<g, b, 0, s>>>(a)
-                             : sp_step_kernel<ST, K_PULL, false, false, false, FUSED, NB, LINK_8, STORE_NT><<<g, b, 0, s>>>(a);
-    else sp_step_kernel<ST, K_PULL, false, false, false, FUSED, NB><<<g, b, 0, s>>>(a);
+        a.order & ORDER_KEEP ? sp_step_kernel<ST, K_PULL, false, BC, PL, FUSED, NB, LINK_8, STORE_KEEP><<<g, b, 0, s>>>(a)
+                             : sp_step_kernel<ST, K_PULL, false, BC, PL, FUSED, NB, LINK_8, STORE_NT><<<g, b, 0, s>>>(a);
+    else sp_step_kernel<ST, K_PULL, false, BC, PL, FUSED, NB><<<g, b, 0, s>>>(a);
 }
 template <typename ST, int NB>
 void launch_pull(const SpArgs<ST> &a, bool store_u, int64_t N, hipStream_t s)
 {
-    a.st.src ? launch_pull_nb<ST, true, NB>(a, store_u, N, s) : launch_pull_nb<ST, false, NB>(a, store_u, N, s);
+    a.st.src ? launch_pull_nb<ST, false, false, true, NB>(a, store_u, N, s)
+             : launch_pull_nb<ST, false, false, false, NB>(a, store_u, N, s);
 }
 
 template <typename ST, bool BC>
@@ -452,17 +455,20 @@ void launch_step_bc(const SpArgs<ST> &a, int mode, bool store_u, dim3 g, dim3 b,
         else if constexpr (BC)   // without faces: launch_pull
             store_u ? sp_step_kernel<ST, K_PULL, true, BC, false, true><<<g, b, 0, s>>>(a)
                     : sp_step_kernel<ST, K_PULL, false, BC, false, true><<<g, b, 0, s>>>(a);
-    } else if (mode == K_PULL && a.nu_vn)
-        store_u ? sp_step_kernel<ST, K_PULL, true, BC, true><<<g, b, 0, s>>>(a)
-                : sp_step_kernel<ST, K_PULL, false, BC, true><<<g, b, 0, s>>>(a);
+    } else if (mode == K_PULL && a.nu_vn) {
+        if constexpr (BC)   // the general form: 815,257 nodes FP32 24.7 us, in the box's form 25.1
+            store_u ? sp_step_kernel<ST, K_PULL, true, BC, true><<<g, b, 0, s>>>(a)
+                    : sp_step_kernel<ST, K_PULL, false, BC, true><<<g, b, 0, s>>>(a);
+        else
+            launch_pull_nb<ST, false, true, false, BLOCK>(a, store_u, a.N, s);
+    }
     else if (mode == K_INIT)
         store_u ? sp_step_kernel<ST, K_INIT, true, BC><<<g, b, 0, s>>>(a)
                 : sp_step_kernel<ST, K_INIT, false, BC><<<g, b, 0, s>>>(a);
     else if (mode == K_DIRECT)
         sp_step_kernel<ST, K_DIRECT, false, BC><<<g, b, 0, s>>>(a);
     else if constexpr (BC)
-        store_u ? sp_step_kernel<ST, K_PULL, true, BC><<<g, b, 0, s>>>(a)
-                : sp_step_kernel<ST, K_PULL, false, BC><<<g, b, 0, s>>>(a);
+        launch_pull_nb<ST, true, false, false, BLOCK>(a, store_u, a.N, s);
 }
 
 template <typename ST>

@@ -58,3 +58,25 @@ def test_both_sides_of_four_gigabytes(pkg, shape):
     for _ in range(4):
         s.step(1)
     assert np.array_equal(together, s.velocity())
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-13), ("fp32", 1e-6)])
+@pytest.mark.parametrize("faces,law", [(True, 0.0), (False, 0.8)])
+def test_faces_and_power_law_on_eight_bit_ranks(pkg, precision, tol, faces, law):
+    """Steps in one call (the form the box allows) against steps one by one (the general form); the
+    power law acts from the eleventh on.  The arithmetic is the same up to how it is contracted:
+    the tolerances are the precisions' of the other comparisons."""
+    print("[gpu] link forms", precision, faces, law, flush=True)
+    solid = (np.random.default_rng(13).uniform(size=(40, 170, 160)) > 0.97).astype(np.int32)
+    states = []
+    for calls in ((14,), (1,) * 14):
+        s = pkg.SinglePhase(solid, 0.1, (0.0, 0.0, 0.0) if faces else G, precision=precision)
+        s.init(1.0, U0)
+        if faces:
+            s.set_boundaries(3, pre={"xp": 1.0 - 2e-4, "xn": 1.0 + 2e-4})
+        if law:
+            s.set_power_law(0.05, law)
+        for n in calls:
+            s.step(n)
+        states.append(s.state()[0])
+    assert rel_err(*states) < tol

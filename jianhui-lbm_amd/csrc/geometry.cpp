@@ -117,25 +117,34 @@ struct ColumnTables {
 };
 constexpr ColumnTables COL;
 
-// Upstream word of node n in direction q from the packed form, as load_links decodes it.
-uint32_t unpack_link(const PackedNbr &p, int64_t P, int64_t n, int q)
+// Whether the packed form of node n's links, as load_links decodes it, is not what link(q) gives.
+template <typename F>
+bool unpacks_wrong(const PackedNbr &p, int64_t P, int64_t n, F &&link)
 {
     const uint32_t *h = &p.hdr[(size_t)((n >> 6) * HDR_WORDS)];
     const int lane = (int)(n & 63);
-    auto mask = [h](int at) { return (uint64_t)h[at] | (uint64_t)h[at + 1] << 32; };
-    if (mask(HDR_MASK + 2 * (q - 1)) >> lane & 1) return (uint32_t)n | BB_FLAG;
-    if (h[HDR_WIDE] != HDR_COMPACT) return p.wide[(size_t)(((int64_t)h[HDR_WIDE] * 18 + q - 1) * 64 + lane)];
-    const uint64_t edge = mask(HDR_EDGE);
-    if (EZ[q] != 0 && (edge >> lane & 1)) {
-        const int64_t rec = (int64_t)h[HDR_EDGE_BASE] + __builtin_popcountll(edge & ((1ull << lane) - 1));
-        return p.edge[(size_t)(rec * EDGE_WORDS + COL.slot[q])];
+    auto lane_in = [h, lane](int at) { return (h[at + (lane >> 5)] >> (lane & 31) & 1u) != 0; };
+    const bool wide = h[HDR_WIDE] != HDR_COMPACT, is_edge = !wide && lane_in(HDR_EDGE);
+    const uint64_t edge = (uint64_t)h[HDR_EDGE] | (uint64_t)h[HDR_EDGE + 1] << 32;
+    const int64_t rec = is_edge ? (int64_t)h[HDR_EDGE_BASE] + __builtin_popcountll(edge & ((1ull << lane) - 1)) : 0;
+    uint32_t rank[NCOL];
+    for (int c = 0; c < NCOL && !wide; ++c) {
+        const size_t at = (size_t)(((c / 4) * P + n) * 4 + c % 4);
+        rank[c] = p.narrow ? h[c] + (uint32_t)n + p.res8[at] : h[c] + p.res[at];
     }
-    const int c = COL.column[q];
-    if (c == NCOL) return (uint32_t)(n - EZ[q]);
-    const size_t at = (size_t)(((c / 4) * P + n) * 4 + c % 4);
-    const uint32_t r = p.narrow ? h[c] + (uint32_t)n + p.res8[at] : h[c] + p.res[at];
-    if (EZ[q] == 0) return r;
-    return EZ[q] > 0 ? r - 1 : r + (mask(HDR_MASK + 2 * (COL.at[c] - 1)) >> lane & 1 ? 0u : 1u);
+    bool wrong = false;
+    for (int q = 1; q < Q; ++q) {
+        const int c = COL.column[q];
+        uint32_t up;
+        if (lane_in(HDR_MASK + 2 * (q - 1))) up = (uint32_t)n | BB_FLAG;
+        else if (wide) up = p.wide[(size_t)(((int64_t)h[HDR_WIDE] * 18 + q - 1) * 64 + lane)];
+        else if (EZ[q] != 0 && is_edge) up = p.edge[(size_t)(rec * EDGE_WORDS + COL.slot[q])];
+        else if (c == NCOL) up = (uint32_t)(n - EZ[q]);
+        else if (EZ[q] == 0) up = rank[c];
+        else up = EZ[q] > 0 ? rank[c] - 1 : rank[c] + (lane_in(HDR_MASK + 2 * (COL.at[c] - 1)) ? 0u : 1u);
+        wrong |= up != link(q);
+    }
+    return wrong;
 }
 
 }  // namespace
@@ -251,10 +260,9 @@ int pack_neighbours(const SparseGeometry &g, PackedNbr &out, std::string &err, b
     // decode everything as the device does and compare
     int64_t bad = 0;
 #pragma omp parallel for schedule(static) reduction(+ : bad)
-    for (int64_t n = 0; n < N; ++n)
-        for (int q = 1; q < Q; ++q) bad += unpack_link(out, P, n, q) != link(n, q);
+    for (int64_t n = 0; n < N; ++n) bad += unpacks_wrong(out, P, n, [&](int q) { return link(n, q); });
     if (bad) {
-        err = "neighbour table packing failed its decode check (" + std::to_string(bad) + " entries)";
+        err = "neighbour table packing failed its decode check (" + std::to_string(bad) + " nodes)";
         return LBM_ERR_STATE;
     }
     return LBM_OK;

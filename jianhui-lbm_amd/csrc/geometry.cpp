@@ -135,14 +135,14 @@ bool unpacks_wrong(const PackedNbr &p, int64_t P, int64_t n, F &&link)
     bool wrong = false;
     for (int q = 1; q < Q; ++q) {
         const int c = COL.column[q];
+        const bool solid = lane_in(HDR_MASK + 2 * (q - 1));
         uint32_t up;
-        if (lane_in(HDR_MASK + 2 * (q - 1))) up = (uint32_t)n | BB_FLAG;
-        else if (wide) up = p.wide[(size_t)(((int64_t)h[HDR_WIDE] * 18 + q - 1) * 64 + lane)];
+        if (wide) up = p.wide[(size_t)(((int64_t)h[HDR_WIDE] * 18 + q - 1) * 64 + lane)];
         else if (EZ[q] != 0 && is_edge) up = p.edge[(size_t)(rec * EDGE_WORDS + COL.slot[q])];
         else if (c == NCOL) up = (uint32_t)(n - EZ[q]);
         else if (EZ[q] == 0) up = rank[c];
-        else up = EZ[q] > 0 ? rank[c] - 1 : rank[c] + (lane_in(HDR_MASK + 2 * (COL.at[c] - 1)) ? 0u : 1u);
-        wrong |= up != link(q);
+        else up = EZ[q] > 0 ? rank[c] - 1 : rank[c] + !lane_in(HDR_MASK + 2 * (COL.at[c] - 1));
+        wrong |= (solid ? (uint32_t)n | BB_FLAG : up) != link(q);   // selected last: no branch on what is close to random
     }
     return wrong;
 }
@@ -152,8 +152,9 @@ bool unpacks_wrong(const PackedNbr &p, int64_t P, int64_t n, F &&link)
 int pack_neighbours(const SparseGeometry &g, PackedNbr &out, std::string &err, bool narrow_ok)
 {
     const int64_t P = g.P, N = g.N, W = P / 64;
-    std::vector<uint32_t> base8((size_t)(W * NCOL), 0u);
-    std::vector<uint8_t> wide8((size_t)W, 0u);
+    // the 8-bit form, worked out only where the caller may take it
+    std::vector<uint32_t> base8((size_t)(narrow_ok ? W * NCOL : 0), 0u);
+    std::vector<uint8_t> wide8((size_t)(narrow_ok ? W : 0), 0u);
     out.hdr.assign((size_t)(W * HDR_WORDS), 0u);
     auto link = [&g, P](int64_t n, int q) { return g.nbr[(size_t)((q - 1) * P + n)]; };
     auto none = [](uint32_t v) { return (v & BB_FLAG) != 0; };
@@ -173,38 +174,49 @@ int pack_neighbours(const SparseGeometry &g, PackedNbr &out, std::string &err, b
     for (int64_t w = 0; w < W; ++w) {
         const int64_t n0 = w * 64, n1 = std::min(n0 + 64, N);
         uint32_t *h = &out.hdr[(size_t)(w * HDR_WORDS)];
-        auto set = [h](int at, int64_t lane) { h[at + (lane >> 5)] |= 1u << (lane & 31); };
-        auto solid = [&](uint32_t v, int q, int64_t lane) {
-            if (none(v) && q) set(HDR_MASK + 2 * (q - 1), lane);
+        auto set = [h](int at, uint64_t lanes) {
+            h[at] |= (uint32_t)lanes;
+            h[at + 1] |= (uint32_t)(lanes >> 32);
         };
         bool wide = false;
         for (int c = 0; c <= NCOL; ++c) {
             uint32_t lo = 0xFFFFFFFFu, hi = 0, at, below, above;
             int64_t lo8 = INT64_MAX, hi8 = INT64_MIN;   // of the rank less the node's own id
+            uint64_t no_at = 0, no_below = 0, no_above = 0, edge = 0;
+            // without branches: which sites are solid is close to random
             for (int64_t n = n0; n < n1; ++n) {
                 column(n, c, at, below, above);
-                solid(at, COL.at[c], n - n0);
-                solid(below, COL.below[c], n - n0);
-                solid(above, COL.above[c], n - n0);
-                if (none(at) && none(below) && none(above)) continue;
+                const uint64_t na = none(at), nb = none(below), nv = none(above);
+                const int lane = (int)(n - n0);
+                no_at |= na << lane;
+                no_below |= nb << lane;
+                no_above |= nv << lane;
                 const uint32_t r = rank(at, below, above);
-                if ((!none(below) && below != r - 1) || (!none(above) && above != r + !none(at)))
-                    set(HDR_EDGE, n - n0);
-                lo = std::min(lo, r);
-                hi = std::max(hi, r);
-                lo8 = std::min(lo8, (int64_t)r - n);
-                hi8 = std::max(hi8, (int64_t)r - n);
+                const bool any = !(na & nb & nv);
+                const bool jumps = (!nb & (below != r - 1)) | (!nv & (above != r + !na));
+                edge |= (uint64_t)(any & jumps) << lane;
+                lo = std::min(lo, any ? r : lo);
+                hi = std::max(hi, any ? r : hi);
+                if (narrow_ok) {
+                    lo8 = std::min(lo8, any ? (int64_t)r - n : lo8);
+                    hi8 = std::max(hi8, any ? (int64_t)r - n : hi8);
+                }
             }
+            if (COL.at[c]) set(HDR_MASK + 2 * (COL.at[c] - 1), no_at);
+            if (COL.below[c]) set(HDR_MASK + 2 * (COL.below[c] - 1), no_below);
+            if (COL.above[c]) set(HDR_MASK + 2 * (COL.above[c] - 1), no_above);
+            set(HDR_EDGE, edge);
             if (c == NCOL || lo == 0xFFFFFFFFu) continue;   // the own column needs no ranks
             h[c] = lo;
             wide |= hi - lo > 0xFFFFu;
+            if (!narrow_ok) continue;
             base8[(size_t)(w * NCOL + c)] = (uint32_t)lo8;
             wide8[(size_t)w] |= hi8 - lo8 > 0xFF;
         }
         h[HDR_WIDE] = wide ? 0u : HDR_COMPACT;
         // lanes past the last node: solid all round, so that following their links stays in place
         for (int64_t n = std::max(n0, n1); n < n0 + 64; ++n)
-            for (int q = 1; q < Q; ++q) set(HDR_MASK + 2 * (q - 1), n - n0);
+            for (int q = 1; q < Q; ++q) set(HDR_MASK + 2 * (q - 1), 1ull << (n - n0));
     }
     int64_t n_wide8 = 0;
     for (uint8_t v : wide8) n_wide8 += v;

@@ -327,8 +327,8 @@ double lbm_srv_clock(const lbm_handle *h);
  * the tiles of consecutive nodes are dealt to the MI355X's 8 XCDs (each with its own L2), and,
  * for the colour streaming, the variant.  No counterpart in the reference (a CPU program).  By
  * default a handle chooses them itself: at create, on its own geometry, it times every candidate
- * and keeps the fastest (the autotuner; choices are cached per kernel, precision and size class
- * for the life of the process; boxes under 2^20 fluid nodes take settings by their size).
+ * and keeps the fastest (the autotuner; choices are cached per kernel, precision, size class and
+ * form of the launch for the life of the process; boxes under 2^20 fluid nodes take settings by their size).
  * lbm_set_launch fixes a setting, e.g. to compare two; results are identical for every setting. */
 #define LBM_KERNEL_SP_STEP 1      /* single-phase step (sp_step_kernel) */
 #define LBM_KERNEL_CG_COLLIDE 2   /* colour-gradient collide (cg_collide_kernel) */

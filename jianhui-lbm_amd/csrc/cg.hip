@@ -1174,9 +1174,10 @@ int CgSolver::autotune()
         launch_colour_ = lbm_launch{block, ORDER_SLAB, variant, 0, 0.0};
         return LBM_OK;
     }
+    const bool fits = fits_cache(cg_step_bytes(geo_.P, ct_bytes_));
+    const TuneKey k1{LBM_KERNEL_CG_COLLIDE, prm_.precision, geo_.N, fits}, k2{LBM_KERNEL_CG_COLOUR, prm_.precision, geo_.N, fits};
     lbm_launch c1, c2;
-    if (tune_cache_get(LBM_KERNEL_CG_COLLIDE, prm_.precision, geo_.N, c1) &&
-        tune_cache_get(LBM_KERNEL_CG_COLOUR, prm_.precision, geo_.N, c2)) {
+    if (tune_cache_get(k1, c1) && tune_cache_get(k2, c2)) {
         launch_collide_ = c1;
         launch_colour_ = c2;
         return LBM_OK;
@@ -1230,8 +1231,8 @@ int CgSolver::autotune()
                             },
                             best));
     launch_colour_ = best;
-    tune_cache_put(LBM_KERNEL_CG_COLLIDE, prm_.precision, geo_.N, launch_collide_);
-    tune_cache_put(LBM_KERNEL_CG_COLOUR, prm_.precision, geo_.N, launch_colour_);
+    tune_cache_put(k1, launch_collide_);
+    tune_cache_put(k2, launch_colour_);
     return LBM_OK;
 }
 

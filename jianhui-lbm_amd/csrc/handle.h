@@ -244,6 +244,7 @@ public:
     hipStream_t stream() const { return stream_; }
     int device() const { return device_; }
     size_t compute_bytes() const { return ct_bytes_; }
+    size_t storage_bytes() const { return st_bytes_; }
     bool initialised() const { return mode_ != STATE_EMPTY; }
 
 private:

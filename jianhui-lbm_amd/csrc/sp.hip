@@ -417,9 +417,6 @@ SpArgs<ST> make_args(const void *src, void *dst, const NbrDev &nbr, void *u_aux,
     return a;
 }
 
-// what a step reads and writes: populations (19 rows of st bytes, twice), links, a solute's rows
-int64_t sp_step_bytes(int64_t P, size_t st, size_t solute) { return P * (int64_t)(2 * Q * st + solute + 19); }
-
 // The pull step at a workgroup size NB, in the form that the box allows.  Steps with faces or power law,
 // general form -> this: 256^3 sphere pack FP32 173.7 -> 171.7 and 178.4 -> 175.9 us, 131,072 nodes FP64 with
 // power law 11.2 -> 10.9, 2.05 M nodes FP16 with faces 36.4 -> 34.7.
@@ -647,8 +644,9 @@ int SpSolver::autotune()
     if (geo_.N < SP_SLAB_NODES) launch_ = lbm_launch{128, ORDER_SLAB, 0, 0, 0.0};
     else if (geo_.N >= SP_KEEP_SLAB_NODES && fits_cache(sp_step_bytes(geo_.P, st_bytes_, 0))) launch_.order = ORDER_SLAB;
     if (geo_.N < TUNE_MIN_NODES) return LBM_OK;
+    const TuneKey key{LBM_KERNEL_SP_STEP, prm_.precision, geo_.N, fits_cache(sp_step_bytes(geo_.P, st_bytes_, 0)), nbr_.narrow};
     lbm_launch c;
-    if (tune_cache_get(LBM_KERNEL_SP_STEP, prm_.precision, geo_.N, c)) {
+    if (tune_cache_get(key, c)) {
         launch_ = c;
         return LBM_OK;
     }
@@ -666,7 +664,7 @@ int SpSolver::autotune()
                             },
                             best));
     launch_ = best;
-    tune_cache_put(LBM_KERNEL_SP_STEP, prm_.precision, geo_.N, best);
+    tune_cache_put(key, best);
     return LBM_OK;
 }
 

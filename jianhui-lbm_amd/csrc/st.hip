@@ -204,11 +204,14 @@ StArgs<C> make_st_args(const void *src, void *dst, NbrDev nbr, const void *u, co
     return a;
 }
 
+// what a standalone step reads and writes: populations (twice), velocity, links
+int64_t st_step_bytes(int64_t P, size_t st) { return P * (int64_t)(17 * st + 11); }
+
 template <typename C, int NB>
 void launch_st_pull(const StArgs<C> &a, int32_t order, hipStream_t s)
 {
     const dim3 g((unsigned)((a.N + NB - 1) / NB)), b(NB);
-    if (fits_cache(a.P * (int64_t)(17 * sizeof(C) + 11))) order |= ORDER_KEEP;   // populations, velocity, links
+    if (fits_cache(st_step_bytes(a.P, sizeof(C)))) order |= ORDER_KEEP;
     // a solute's own table has 16-bit ranks, that of a coupled flow may be narrow
     a.nbr.narrow ? st_step_kernel<C, K_PULL, NB><<<g, b, 0, s>>>(a, order)
                  : st_step_kernel<C, K_PULL, NB, LINK_16><<<g, b, 0, s>>>(a, order);
@@ -243,9 +246,14 @@ int StSolver::autotune()
     if (N_ < ST_SLAB_NODES) launch_ = launch_own_ = lbm_launch{128, ORDER_SLAB, 0, 0, 0.0};
     else if (fits_cache(P_ * (int64_t)(52 * st_bytes_ + 19))) launch_.order = launch_own_.order = ORDER_SLAB;
     if (N_ < TUNE_MIN_NODES) return LBM_OK;
-    const int kind = flow_ ? -LBM_KERNEL_ST_STEP : LBM_KERNEL_ST_STEP;   // separate cache entries
+    TuneKey key{LBM_KERNEL_ST_STEP, prm_.precision, N_, fits_cache(st_step_bytes(P_, st_bytes_))};
+    if (flow_) {
+        const size_t width = flow_->storage_bytes();
+        key = {-LBM_KERNEL_ST_STEP, prm_.precision, N_, fits_cache(sp_step_bytes(P_, width, 2 * Q7 * st_bytes_)), nbr_.narrow != 0,
+               width, fits_cache(sp_step_bytes(P_, width, 0))};
+    }
     lbm_launch c;
-    if (tune_cache_get(kind, prm_.precision, N_, c)) {
+    if (tune_cache_get(key, c)) {
         (flow_ ? launch_ : launch_own_) = c;
         return LBM_OK;
     }
@@ -278,7 +286,7 @@ int StSolver::autotune()
         LBM_HIP_TRY(tune_launch(stream_, cands, run, best));
         launch_own_ = best;
     }
-    tune_cache_put(kind, prm_.precision, N_, best);
+    tune_cache_put(key, best);
     return LBM_OK;
 }
 

@@ -11,25 +11,31 @@ namespace lbm {
 
 namespace {
 std::mutex cache_mu;
-std::map<std::tuple<int, int, int>, lbm_launch> cache;
+using Key = std::tuple<int, int, int, bool, bool, size_t, bool>;
+std::map<Key, lbm_launch> cache;
 
 // two size classes per octave of the node count
 int size_class(int64_t N) { return (int)std::floor(2.0 * std::log2((double)std::max<int64_t>(N, 1))); }
+
+Key key_of(const TuneKey &k)
+{
+    return {k.kernel, k.precision, size_class(k.nodes), k.fits, k.narrow, k.flow_width, k.flow_fits};
+}
 }  // namespace
 
-bool tune_cache_get(int kernel, int precision, int64_t N, lbm_launch &out)
+bool tune_cache_get(const TuneKey &key, lbm_launch &out)
 {
     std::lock_guard<std::mutex> lk(cache_mu);
-    auto it = cache.find(std::make_tuple(kernel, precision, size_class(N)));
+    auto it = cache.find(key_of(key));
     if (it == cache.end()) return false;
     out = it->second;
     return true;
 }
 
-void tune_cache_put(int kernel, int precision, int64_t N, const lbm_launch &ls)
+void tune_cache_put(const TuneKey &key, const lbm_launch &ls)
 {
     std::lock_guard<std::mutex> lk(cache_mu);
-    cache[std::make_tuple(kernel, precision, size_class(N))] = ls;
+    cache[key_of(key)] = ls;
 }
 
 std::vector<lbm_launch> tune_candidates(const lbm_launch &def, const std::vector<int> &blocks,

@@ -58,9 +58,23 @@ constexpr int64_t BACK_NODES = int64_t(1) << 20;
 // an alternative replaces the default only when it is faster by this fraction
 constexpr double TUNE_MARGIN = 0.01;
 
-// cached choice for (kernel, precision, size class of N); false if none
-bool tune_cache_get(int kernel, int precision, int64_t N, lbm_launch &out);
-void tune_cache_put(int kernel, int precision, int64_t N, const lbm_launch &ls);
+// what a flow step reads and writes: populations (19 rows of st bytes, twice), links, a solute's rows
+inline int64_t sp_step_bytes(int64_t P, size_t st, size_t solute) { return P * (int64_t)(2 * 19 * st + solute + 19); }
+
+// What a choice is kept under: the kernel, the precision, the size class (two an octave) and all else
+// that decides which form of the kernel a launch runs and in which direction.  Both lines of the cache
+// fall inside a size class, and an FP16 and an FP32 flow carry the same FP32 solute.
+struct TuneKey {
+    int kernel, precision;
+    int64_t nodes;
+    bool fits;               // the step fits the memory-side cache
+    bool narrow = false;     // 8-bit ranks
+    size_t flow_width = 0;   // coupled solute: bytes of a stored flow value,
+    bool flow_fits = false;  // and whether the flow's own step fits
+};
+// cached choice; false if none
+bool tune_cache_get(const TuneKey &key, lbm_launch &out);
+void tune_cache_put(const TuneKey &key, const lbm_launch &ls);
 
 // The fastest of `cands` (cands[0] is the default): each candidate is launched `warm` times,
 // then timed as the median of `rounds` rounds of `reps` launches between HIP events on s.

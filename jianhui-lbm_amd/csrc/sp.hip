@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <functional>
 #include <mutex>
 
 #include "boundary.h"
@@ -750,7 +751,9 @@ hipError_t SpSolver::launch_kernel(int mode, bool store_u, const FusedSolute *fs
     // the power-law collision acts from the reference's loop step n = 11 on (SP:2397); the
     // launches since init or load_state are that loop's n
     lbm_launch ls = set;
-    if (geo_.N >= BACK_NODES && !fits_cache(sp_step_bytes(geo_.P, st_bytes_, 0)) && dst == pops_[0]) ls.order |= ORDER_BACK;
+    // of two buffers that launches go between, those into the lower one run backwards
+    if (geo_.N >= BACK_NODES && !fits_cache(sp_step_bytes(geo_.P, st_bytes_, 0)) && std::less<const void *>()(dst, src))
+        ls.order |= ORDER_BACK;
     void *pl_nu = (!bare && d_nu_vn_ && steps_ > 10) ? d_nu_vn_ : nullptr;
     const BcDev bc = bare ? BcDev{nullptr, nullptr, nullptr, nullptr, 0} : bc_view(true);
     if (prm_.precision == LBM_FP64)

@@ -238,9 +238,13 @@ int st_kmode(StateMode m) { return m == STATE_INIT ? K_INIT : (m == STATE_DIRECT
 
 }  // namespace
 
-// Standalone: time the solute step's block sizes and tile orders (on a zero field, in the spare
-// buffer: init or load_state sets the state).  Coupled: time the fused flow + solute launch on
-// the flow's state, writing only both handles' spare buffers, so neither state changes.
+// Standalone: time the solute step's block sizes and tile orders, back and forth between the handle's
+// buffers, zeroed (init or load_state sets the state).  Coupled: time the fused flow + solute launch the
+// same way, the flow's populations between its spare buffer and one allocated for the timing, as its
+// current one may hold a state in mid-run.  Timed from that state into the spare buffer again and
+// again, all launches in one direction, a box found much of its source in the memory-side cache:
+// 2,186,632 nodes FP32 took slabs for 65 us, which were 88 us a step in a run (256-node runs of 8: 81);
+// 1,066,428 nodes FP64 slabs for 62 us, 86 in a run (128-node runs of 8: 78).
 int StSolver::autotune()
 {
     if (N_ < ST_SLAB_NODES) launch_ = launch_own_ = lbm_launch{128, ORDER_SLAB, 0, 0, 0.0};
@@ -262,14 +266,23 @@ int StSolver::autotune()
     if (flow_) {
         const double cs2 = (1.0 - prm_.w0) / 3.0;
         FusedSolute fs{pops_[0], pops_[1], 1.0 / (prm_.D / cs2 + 0.5), prm_.w0, (1.0 - prm_.w0) / 6.0, 1.0 / cs2, launch_};
-        const void *state = flow_->pops(flow_->current());
-        void *spare = flow_->pops(flow_->current() ^ 1);
+        void *flow[2] = {flow_->pops(flow_->current() ^ 1), nullptr};
+        if (hipMalloc(&flow[1], (size_t)Q * P_ * flow_->storage_bytes()) != hipSuccess) {
+            (void)hipGetLastError();   // no room for it: the launches go by their default
+            return LBM_OK;
+        }
         const auto cands = tune_candidates(launch_, {128, 256, 512}, {ORDER_HW, ORDER_RUNS8, ORDER_SLAB}, {0});
-        LBM_HIP_TRY(tune_launch(stream_, cands,
-                                [&](const lbm_launch &ls) {
-                                    return flow_->launch_kernel(K_PULL, false, &fs, ls, state, spare, true);
-                                },
-                                best));
+        int from = 0;
+        const hipError_t e = tune_launch(stream_, cands,
+                                         [&](const lbm_launch &ls) {
+                                             from ^= 1;
+                                             fs.src = pops_[from];
+                                             fs.dst = pops_[from ^ 1];
+                                             return flow_->launch_kernel(K_PULL, false, &fs, ls, flow[from], flow[from ^ 1], true);
+                                         },
+                                         best);
+        (void)hipFree(flow[1]);
+        LBM_HIP_TRY(e);
         launch_ = best;
     } else {
         const void *u = d_u_own_;

@@ -51,7 +51,7 @@ PinnedUser::~PinnedUser()
     idle().clear();
 }
 
-hipError_t pinned_take(int device, PinnedSet &out)
+bool pinned_take(int device, PinnedSet &out)
 {
     {
         std::lock_guard<std::mutex> lk(mu);
@@ -59,7 +59,7 @@ hipError_t pinned_take(int device, PinnedSet &out)
             if (idle()[k].device == device) {
                 out = idle()[k];
                 idle().erase(idle().begin() + (ptrdiff_t)k);
-                return hipSuccess;
+                return true;
             }
     }
     out = PinnedSet{};
@@ -69,8 +69,10 @@ hipError_t pinned_take(int device, PinnedSet &out)
         e = hipHostMalloc(&out.slot[k], PIN_BYTES, hipHostMallocDefault);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&out.done[k], hipEventDisableTiming);
     }
-    if (e != hipSuccess) free_set(out);
-    return e;
+    if (e == hipSuccess) return true;
+    free_set(out);
+    (void)hipGetLastError();   // not for the next call to report
+    return false;
 }
 
 void pinned_return(PinnedSet &s)

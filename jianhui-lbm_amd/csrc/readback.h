@@ -27,7 +27,8 @@ struct PinnedSet {
     hipEvent_t done[PIN_SLOTS] = {nullptr};
     int device = -1;   // the events' device
 };
-hipError_t pinned_take(int device, PinnedSet &out);
+// a set for a read on the device; false where page-locked memory cannot be had (no error is left pending)
+bool pinned_take(int device, PinnedSet &out);
 void pinned_return(PinnedSet &s);
 // a member of every handle that reads back
 struct PinnedUser {
@@ -50,6 +51,38 @@ void read_scatter(const ReadPart *parts, int np, int64_t i0, int64_t i1, size_t 
 // write to every page of the parts' arrays, with a team of threads
 void read_touch(const ReadPart *parts, int np, int64_t items);
 
+// the wanted parts of items [i0, i1) in device memory from base on, one after the other, to p; their bytes
+inline size_t place_parts(const ReadPart *parts, int np, int64_t i0, int64_t i1, char *base, double **p)
+{
+    size_t at = 0;
+    for (int k = 0; k < np; ++k) {
+        p[k] = parts[k].dst ? (double *)(base + at) : nullptr;
+        if (parts[k].dst) at += sizeof(double) * (size_t)parts[k].width * (size_t)(i1 - i0);
+    }
+    return at;
+}
+
+// read_back without page-locked slots or an allocation: each chunk straight into the caller's arrays
+template <typename F>
+hipError_t read_direct(hipStream_t s, int64_t n, const ReadPart *parts, int np, void *buf, size_t buf_bytes, size_t item,
+                       int64_t step, F &&fill)
+{
+    const int64_t chunk = std::max<int64_t>(step, (int64_t)(buf_bytes / item) / step * step);
+    hipError_t e = hipSuccess;
+    for (int64_t i0 = 0; i0 < n && e == hipSuccess; i0 += chunk) {
+        const int64_t i1 = std::min(n, i0 + chunk);
+        double *p[READ_PARTS] = {nullptr};
+        place_parts(parts, np, i0, i1, (char *)buf, p);
+        e = fill(i0, i1, p);
+        for (int k = 0; k < np && e == hipSuccess; ++k)
+            if (p[k])
+                e = hipMemcpyAsync(parts[k].dst + i0 * parts[k].width, p[k],
+                                   sizeof(double) * (size_t)parts[k].width * (size_t)(i1 - i0), hipMemcpyDeviceToHost, s);
+    }
+    const hipError_t es = hipStreamSynchronize(s);
+    return e == hipSuccess ? es : e;
+}
+
 // Read items 0 .. n-1 of the parts.  fill(i0, i1, p) queues on s the work that writes items
 // [i0, i1) of each wanted part k to p[k].  buf: device memory, buf_bytes.  step: items per chunk
 // are a multiple of it.  Every copy has ended when the call returns, with an error too.
@@ -61,10 +94,10 @@ hipError_t read_back(int device, hipStream_t s, int64_t n, const ReadPart *parts
     for (int k = 0; k < np; ++k) width += parts[k].dst ? parts[k].width : 0;
     if (width == 0 || n <= 0) return hipSuccess;
     const size_t item = sizeof(double) * (size_t)width;
-    const int64_t chunk = std::max<int64_t>(step, (int64_t)(buf_bytes / 2 / item) / step * step);
     PinnedSet set;
-    hipError_t e = pinned_take(device, set);
-    if (e != hipSuccess) return e;
+    if (!pinned_take(device, set)) return read_direct(s, n, parts, np, buf, buf_bytes, item, step, fill);
+    hipError_t e = hipSuccess;
+    const int64_t chunk = std::max<int64_t>(step, (int64_t)(buf_bytes / 2 / item) / step * step);
     struct Piece {
         int64_t i0, i1;
         size_t at, bytes;
@@ -87,12 +120,7 @@ hipError_t read_back(int device, hipStream_t s, int64_t n, const ReadPart *parts
         // the half's last copies are ahead of this chunk's kernels on the stream
         char *base = (char *)buf + (half ? buf_bytes / 2 : 0);
         double *p[READ_PARTS] = {nullptr};
-        size_t at = 0;
-        for (int k = 0; k < np; ++k)
-            if (parts[k].dst) {
-                p[k] = (double *)(base + at);
-                at += sizeof(double) * (size_t)parts[k].width * (size_t)(i1 - i0);
-            }
+        const size_t at = place_parts(parts, np, i0, i1, base, p);
         e = fill(i0, i1, p);
         for (size_t o = 0; o < at && e == hipSuccess; o += PIN_BYTES) {
             if (queued - taken == PIN_SLOTS) e = take();

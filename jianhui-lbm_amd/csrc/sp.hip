@@ -950,29 +950,18 @@ int SpSolver::get_state(double *f, double *u, double *rho)
     return LBM_OK;
 }
 
-// for a caller that must not allocate: the state crosses through buf in chunks of whole blocks of nodes; each chunk's copies are
-// ordered on the stream before the next chunk's kernel overwrites buf
+// for a caller that must not allocate: the state crosses through buf
 int SpSolver::get_state_via(double *f, double *u, double *rho, void *buf, size_t bytes)
 {
     const int per_node = (f ? Q : 0) + (u ? 3 : 0) + (rho ? 1 : 0);
     if (per_node == 0) return LBM_OK;
-    if (!buf || bytes < (size_t)BLOCK * per_node * sizeof(double))
-        return fail(LBM_ERR_ARG, "state transfer buffer smaller than one block of nodes");
-    const int64_t N = geo_.N, chunk = stage_chunk(bytes, per_node);
-    hipError_t e = hipSuccess;
-    for (int64_t n0 = 0; n0 < N && e == hipSuccess; n0 += chunk) {
-        const int64_t c = std::min(chunk, N - n0);
-        double *df = f ? (double *)buf : nullptr;
-        double *du = u ? (double *)buf + (f ? c * Q : 0) : nullptr;
-        double *dr = rho ? (double *)buf + (f ? c * Q : 0) + (u ? c * 3 : 0) : nullptr;
-        e = state_to_device(n0, n0 + c, nullptr, 0, df, du, dr);
-        if (e == hipSuccess && f) e = hipMemcpyAsync(f + n0 * Q, df, (size_t)c * Q * sizeof(double), hipMemcpyDeviceToHost, stream_);
-        if (e == hipSuccess && u) e = hipMemcpyAsync(u + n0 * 3, du, (size_t)c * 3 * sizeof(double), hipMemcpyDeviceToHost, stream_);
-        if (e == hipSuccess && rho) e = hipMemcpyAsync(rho + n0, dr, (size_t)c * sizeof(double), hipMemcpyDeviceToHost, stream_);
-    }
-    const hipError_t es = hipStreamSynchronize(stream_);
-    LBM_HIP_TRY(e);
-    LBM_HIP_TRY(es);
+    const size_t item = (size_t)per_node * sizeof(double);
+    if (!buf || bytes < BLOCK * item) return fail(LBM_ERR_ARG, "state transfer buffer smaller than one block of nodes");
+    const ReadPart parts[3] = {{f, Q}, {u, 3}, {rho, 1}};
+    LBM_HIP_TRY(read_direct(stream_, geo_.N, parts, 3, buf, bytes, item, BLOCK,
+                            [&](int64_t n0, int64_t n1, double *const *p) {
+                                return state_to_device(n0, n1, nullptr, 0, p[0], p[1], p[2]);
+                            }));
     return LBM_OK;
 }
 

@@ -1,0 +1,113 @@
+// sanitize_readback.cpp -- the state reads (readback.h) under the sanitizers, on a stand-in for the device
+// runtime: "device" memory is host memory, copies are made at once, and page-locked allocations and copies
+// can be made to fail.  Arguments name the check.
+#include <atomic>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <string>
+#include <vector>
+
+#include "readback.h"
+
+namespace {
+std::atomic<int> live{0}, made{0};        // page-locked slots: alive, ever made
+std::atomic<int> made_at_most{1 << 30};   // allocations that succeed
+std::atomic<int> copies_at_most{1 << 30};
+std::atomic<int> pending{0};   // as the runtime keeps the last error
+hipError_t failed(hipError_t e) { return pending = (int)e, e; }
+}  // namespace
+
+extern "C" {
+hipError_t hipHostMalloc(void **p, size_t n, unsigned int)
+{
+    if (made >= made_at_most) return failed(hipErrorOutOfMemory);
+    *p = std::malloc(n);
+    ++live, ++made;
+    return hipSuccess;
+}
+hipError_t hipHostFree(void *p) { return std::free(p), --live, hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return *e = (hipEvent_t)std::malloc(1), hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { return std::free(e), hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipGetLastError() { return (hipError_t)pending.exchange(0); }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
+{
+    if (copies_at_most-- <= 0) return failed(hipErrorUnknown);
+    return std::memcpy(d, s, n), hipSuccess;
+}
+}
+
+using namespace lbm;
+
+namespace {
+constexpr size_t BUF = size_t(16) << 20;
+int failures = 0;
+void expect(bool ok, const char *what)
+{
+    if (!ok) std::fprintf(stderr, "FAIL %s\n", what), ++failures;
+}
+
+double value(int part, int64_t at) { return 1.0 + part + 1e-3 * (double)at; }
+
+struct Reader {
+    PinnedUser user;
+    std::vector<char> buf = std::vector<char>(BUF);
+    int64_t n;
+    std::vector<double> f, u;
+    explicit Reader(int64_t items) : n(items), f((size_t)items * 19, -1.0), u((size_t)items * 3, -2.0) {}
+    template <typename G>
+    hipError_t read(G &&meanwhile)
+    {
+        const ReadPart parts[3] = {{f.data(), 19}, {nullptr, 5}, {u.data(), 3}};
+        return read_back(0, nullptr, n, parts, 3, buf.data(), BUF, 256, [&](int64_t i0, int64_t i1, double *const *p) {
+            meanwhile();
+            for (int64_t i = i0 * 19; i < i1 * 19; ++i) p[0][i - i0 * 19] = value(0, i);
+            for (int64_t i = i0 * 3; i < i1 * 3; ++i) p[2][i - i0 * 3] = value(2, i);
+            return hipGetLastError();   // as the kernels' launches report
+        });
+    }
+    // items whose values are neither those that are read nor those from before
+    int64_t wrong(bool read) const
+    {
+        int64_t bad = 0;
+        for (int64_t i = 0; i < n * 19; ++i) bad += f[(size_t)i] != value(0, i) && (read || f[(size_t)i] != -1.0);
+        for (int64_t i = 0; i < n * 3; ++i) bad += u[(size_t)i] != value(2, i) && (read || u[(size_t)i] != -2.0);
+        return bad;
+    }
+};
+
+// one piece, several pieces, several chunks with a remainder
+const int64_t SIZES[] = {1, 255, 4224, 40329, 157286};
+
+// no page-locked memory, or not all of a set: the values all the same, and no error left behind
+void refused()
+{
+    for (int slots : {0, 3})
+        for (int64_t n : SIZES) {
+            made = 0;
+            made_at_most = slots;
+            Reader r(n);
+            expect(r.read([] {}) == hipSuccess && r.wrong(true) == 0, "read without page-locked memory");
+            expect(live == 0 && pending == 0, "nothing left of a refused set");
+        }
+    made_at_most = 1 << 30;
+    for (int64_t n : SIZES) {
+        Reader r(n);
+        expect(r.read([] {}) == hipSuccess && r.wrong(true) == 0 && live == PIN_SLOTS, "read through the slots");
+    }
+    expect(live == 0, "slots given back");
+}
+}  // namespace
+
+int main(int, char **argv)
+{
+    const std::string what = argv[1];
+    if (what == "refused") refused();
+    else return 2;
+    if (failures) return 1;
+    std::printf("sanitized checks passed\n");
+    return 0;
+}

@@ -24,3 +24,8 @@ def _run(unit, *args):
 
 def test_tuning_cache():
     assert "checks passed" in _run("tune")
+
+
+@pytest.mark.parametrize("check", ["refused"])
+def test_state_reads(check):
+    assert "checks passed" in _run("readback", check)

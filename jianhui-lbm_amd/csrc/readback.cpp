@@ -116,12 +116,14 @@ void read_touch(const ReadPart *parts, int np, int64_t items)
         const size_t bytes = sizeof(double) * (size_t)parts[k].width * (size_t)items;
         const int nt = team(bytes / 4);
         if (nt == 1) continue;
-        volatile char *p = (volatile char *)parts[k].dst;
+        char *p = (char *)parts[k].dst;
 #pragma omp parallel for num_threads(nt) schedule(static)
         for (int t = 0; t < nt; ++t)
             for (size_t o = bytes / (size_t)nt * (size_t)t, end = t == nt - 1 ? bytes : bytes / (size_t)nt * (size_t)(t + 1); o < end;
-                 o += 4096)
-                p[o] = 0;
+                 o += 4096) {
+                char was = 0;   // zero for zero: a write in any case, of what is there
+                __atomic_compare_exchange_n(p + o, &was, (char)0, false, __ATOMIC_RELAXED, __ATOMIC_RELAXED);
+            }
     }
 }
 

@@ -48,7 +48,7 @@ constexpr int READ_PARTS = 6;
 // host side of a read: `bytes` bytes at byte offset `at` of the device chunk that holds items
 // [i0, i1) of the parts, one after the other
 void read_scatter(const ReadPart *parts, int np, int64_t i0, int64_t i1, size_t at, size_t bytes, const void *from);
-// write to every page of the parts' arrays, with a team of threads
+// write to every page of the parts' arrays, with a team of threads, leaving what is in them
 void read_touch(const ReadPart *parts, int np, int64_t items);
 
 // the wanted parts of items [i0, i1) in device memory from base on, one after the other, to p; their bytes

@@ -100,12 +100,29 @@ void refused()
     }
     expect(live == 0, "slots given back");
 }
+
+// a copy that fails: its error, and of every array what was read so far and else what was there before
+void failing()
+{
+    for (int good : {0, 3, 5, 9})
+        for (int64_t n : {int64_t(40329), int64_t(157286)}) {
+            const int64_t copies = (n * 22 * 8 + (int64_t)PIN_BYTES - 1) / (int64_t)PIN_BYTES;
+            copies_at_most = good;
+            Reader r(n);
+            const hipError_t e = r.read([] {});
+            expect(good >= copies + 1 || e == hipErrorUnknown, "a failed copy is reported");
+            expect(r.wrong(false) == 0, "arrays of a failed read");
+            pending = 0;
+        }
+    copies_at_most = 1 << 30;
+}
 }  // namespace
 
 int main(int, char **argv)
 {
     const std::string what = argv[1];
     if (what == "refused") refused();
+    else if (what == "failing") failing();
     else return 2;
     if (failures) return 1;
     std::printf("sanitized checks passed\n");

@@ -5,23 +5,15 @@
 
 #include <cstring>
 #include <mutex>
-#include <vector>
 
 namespace lbm {
 
 namespace {
-constexpr size_t PIN_IDLE = 2;
 std::mutex mu;
-int users = 0;
-std::vector<PinnedSet> &idle()
-{
-    static std::vector<PinnedSet> *v = [] {   // alive at process exit
-        auto *p = new std::vector<PinnedSet>;
-        p->reserve(PIN_IDLE);
-        return p;
-    }();
-    return *v;
-}
+int users = 0;                // handles
+int sets = 0;                 // page-locked sets there are, idle or in a read
+PinnedSet idle[PIN_SETS];     // the first n_idle
+int n_idle = 0;
 
 void free_set(PinnedSet &s)
 {
@@ -46,21 +38,27 @@ PinnedUser::PinnedUser()
 PinnedUser::~PinnedUser()
 {
     std::lock_guard<std::mutex> lk(mu);
-    if (--users > 0) return;
-    for (PinnedSet &s : idle()) free_set(s);
-    idle().clear();
+    --users;
+    // a handle reads with one set at a time
+    for (; sets > users && n_idle > 0; --sets) free_set(idle[--n_idle]);
 }
 
 bool pinned_take(int device, PinnedSet &out)
 {
     {
         std::lock_guard<std::mutex> lk(mu);
-        for (size_t k = 0; k < idle().size(); ++k)
-            if (idle()[k].device == device) {
-                out = idle()[k];
-                idle().erase(idle().begin() + (ptrdiff_t)k);
+        for (int k = 0; k < n_idle; ++k)
+            if (idle[k].device == device) {
+                out = idle[k];
+                idle[k] = idle[--n_idle];
                 return true;
             }
+        if (sets == PIN_SETS) {
+            if (n_idle == 0) return false;
+            free_set(idle[--n_idle]);   // of another device
+            --sets;
+        }
+        ++sets;
     }
     out = PinnedSet{};
     out.device = device;
@@ -72,19 +70,15 @@ bool pinned_take(int device, PinnedSet &out)
     if (e == hipSuccess) return true;
     free_set(out);
     (void)hipGetLastError();   // not for the next call to report
+    std::lock_guard<std::mutex> lk(mu);
+    --sets;
     return false;
 }
 
 void pinned_return(PinnedSet &s)
 {
-    {
-        std::lock_guard<std::mutex> lk(mu);
-        if (idle().size() < PIN_IDLE) {
-            idle().push_back(s);
-            return;
-        }
-    }
-    free_set(s);
+    std::lock_guard<std::mutex> lk(mu);
+    idle[n_idle++] = s;
 }
 
 void read_scatter(const ReadPart *parts, int np, int64_t i0, int64_t i1, size_t at, size_t bytes, const void *from)

@@ -18,8 +18,10 @@
 namespace lbm {
 
 // Page-locked slots of the reads under way, shared by the handles of the process: a read takes a
-// set for its duration.  Idle sets are kept (two at most) while some handle is alive, since a
-// new set costs 3 ms in page faults, and freed with the last one.  Thread-safe.
+// set for its duration.  Idle sets are kept, at most one for each handle alive, since a new set costs
+// 3 ms in page faults.  There are PIN_SETS at most (128 MiB); further reads at the same time copy
+// straight into the caller's arrays.  Thread-safe.
+constexpr int PIN_SETS = 16;
 constexpr int PIN_SLOTS = 4;
 constexpr size_t PIN_BYTES = size_t(2) << 20;
 struct PinnedSet {
@@ -27,7 +29,8 @@ struct PinnedSet {
     hipEvent_t done[PIN_SLOTS] = {nullptr};
     int device = -1;   // the events' device
 };
-// a set for a read on the device; false where page-locked memory cannot be had (no error is left pending)
+// a set for a read on the device; false where all are in use or page-locked memory cannot be had (no error
+// is left pending)
 bool pinned_take(int device, PinnedSet &out);
 void pinned_return(PinnedSet &s);
 // a member of every handle that reads back

@@ -5,7 +5,9 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "readback.h"
@@ -116,6 +118,39 @@ void failing()
         }
     copies_at_most = 1 << 30;
 }
+
+// handles that read at once, all of them in the middle of a read together: their slots are made once, for
+// as many as may be at a time, the others read without; given back as the handles go
+void at_once()
+{
+    for (int count : {2, 5, 20}) {
+        made = 0;
+        std::vector<std::unique_ptr<Reader>> readers;
+        for (int k = 0; k < count; ++k) readers.emplace_back(new Reader(4224));
+        for (int round = 0; round < 3; ++round) {
+            std::atomic<int> here{0};
+            std::vector<std::thread> threads;
+            std::atomic<int> bad{0};
+            for (auto &r : readers)
+                threads.emplace_back([&, r = r.get()] {
+                    std::fill(r->f.begin(), r->f.end(), -1.0);
+                    const hipError_t e = r->read([&] {
+                        ++here;
+                        while (here < count) std::this_thread::yield();
+                    });
+                    bad += e != hipSuccess || r->wrong(true) != 0;
+                });
+            for (auto &t : threads) t.join();
+            expect(bad == 0, "reads at once");
+        }
+        const int want = std::min(count, PIN_SETS) * PIN_SLOTS;
+        expect(made == want && live == want, "slots made once");
+        readers.resize(1);
+        expect(live == PIN_SLOTS, "slots given back as handles go");
+        readers.clear();
+        expect(live == 0, "slots given back");
+    }
+}
 }  // namespace
 
 int main(int, char **argv)
@@ -123,6 +158,7 @@ int main(int, char **argv)
     const std::string what = argv[1];
     if (what == "refused") refused();
     else if (what == "failing") failing();
+    else if (what == "at_once") at_once();
     else return 2;
     if (failures) return 1;
     std::printf("sanitized checks passed\n");

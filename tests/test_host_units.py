@@ -26,6 +26,6 @@ def test_tuning_cache():
     assert "checks passed" in _run("tune")
 
 
-@pytest.mark.parametrize("check", ["refused", "failing"])
+@pytest.mark.parametrize("check", ["refused", "failing", "at_once"])
 def test_state_reads(check):
     assert "checks passed" in _run("readback", check)

@@ -867,7 +867,20 @@ int SpSolver::get_viscosity(double *nu)
         for (int64_t i = 0; i < N; ++i) nu[i] = prm_.nu;
         return LBM_OK;
     }
-    LBM_HIP_TRY(stage_.ensure());
+    if (stage_.ensure() != hipSuccess) {
+        // no device memory for the transfer buffer: straight into the caller's array, FP32 values into its
+        // second half, from where they are widened in ascending order
+        (void)hipGetLastError();
+        char *at = (char *)nu + (size_t)N * (8 - ct_bytes_);
+        LBM_HIP_TRY(hipMemcpyAsync(at, d_nu_vn_, (size_t)N * ct_bytes_, hipMemcpyDeviceToHost, stream_));
+        LBM_HIP_TRY(hipStreamSynchronize(stream_));
+        for (int64_t i = 0; i < N && ct_bytes_ == 4; ++i) {
+            float v;
+            std::memcpy(&v, at + 4 * i, 4);
+            nu[i] = (double)v;
+        }
+        return LBM_OK;
+    }
     const ReadPart part{nu, 1};
     LBM_HIP_TRY(read_back(device_, stream_, N, &part, 1, stage_.buf, STAGE_BYTES, BLOCK,
                           [&](int64_t n0, int64_t n1, double *const *p) {

@@ -237,8 +237,6 @@ int pack_neighbours(const SparseGeometry &g, PackedNbr &out, std::string &err, b
         h[HDR_EDGE_BASE] = (uint32_t)ne;
         ne += __builtin_popcount(h[HDR_EDGE]) + __builtin_popcount(h[HDR_EDGE + 1]);
     }
-    out.n_wide = nw;
-    out.n_edge = ne;
     out.wide.assign((size_t)(nw * 18 * 64), 0u);
     out.edge.assign((size_t)(ne * EDGE_WORDS), 0u);
 #pragma omp parallel for schedule(static)
@@ -280,7 +278,7 @@ int pack_neighbours(const SparseGeometry &g, PackedNbr &out, std::string &err, b
     return LBM_OK;
 }
 
-hipError_t DeviceNbr::upload(const PackedNbr &p, int64_t, hipStream_t s)
+hipError_t DeviceNbr::upload(const PackedNbr &p, hipStream_t s)
 {
     release();
     const void *from[4] = {p.narrow ? (const void *)p.res8.data() : (const void *)p.res.data(), p.hdr.data(), p.edge.data(),

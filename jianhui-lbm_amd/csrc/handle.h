@@ -88,9 +88,8 @@ struct PackedNbr {
     std::vector<uint8_t> res8;    // the same in 8 bits (narrow; else empty)
     bool narrow = false;
     std::vector<uint32_t> hdr;    // (P / 64) x HDR_WORDS
-    std::vector<uint32_t> edge;   // n_edge x EDGE_WORDS
-    std::vector<uint32_t> wide;   // n_wide x 18 x 64
-    int64_t n_wide = 0, n_edge = 0;
+    std::vector<uint32_t> edge;   // EDGE_WORDS for each edge lane of a compact wave
+    std::vector<uint32_t> wide;   // 18 x 64 for each other wave
 };
 
 // Pack g.nbr, then decode every entry and compare with the full table (LBM_ERR_STATE if any
@@ -100,8 +99,8 @@ int pack_neighbours(const SparseGeometry &g, PackedNbr &out, std::string &err, b
 struct NbrDev {
     const void *__restrict__ res;       // 2 x P: four ranks each, 16-bit (uint2) or 8-bit (uint32_t)
     const uint32_t *__restrict__ hdr;   // (P / 64) x HDR_WORDS
-    const uint4 *__restrict__ edge;     // n_edge x EDGE_WORDS / 4
-    const uint32_t *__restrict__ wide;  // n_wide x 18 x 64
+    const uint4 *__restrict__ edge;     // records of EDGE_WORDS / 4
+    const uint32_t *__restrict__ wide;  // 18 x 64 for each wave that is not compact
     uint32_t narrow;
 };
 
@@ -112,7 +111,7 @@ struct DeviceNbr {
     uint32_t *hdr = nullptr, *wide = nullptr;
     bool narrow = false;
     // allocate and queue the copies on s; p must stay alive until s has been synchronised
-    hipError_t upload(const PackedNbr &p, int64_t P, hipStream_t s);
+    hipError_t upload(const PackedNbr &p, hipStream_t s);
     void release();
     NbrDev view() const { return NbrDev{res, hdr, edge, wide, narrow}; }
 };

@@ -621,7 +621,7 @@ int SpSolver::create(const lbm_sp_params &p, const int32_t *solid)
     PackedNbr packed;
     rc = pack_neighbours(geo_, packed, err, geo_.N >= NARROW_NODES);
     if (rc != LBM_OK) return fail(rc, err);
-    LBM_HIP_TRY(nbr_.upload(packed, P, stream_));
+    LBM_HIP_TRY(nbr_.upload(packed, stream_));
     LBM_HIP_TRY(hipMemcpyAsync(d_supinv_, geo_.supinv.data(), geo_.supinv.size() * sizeof(int32_t),
                                hipMemcpyHostToDevice, stream_));
     LBM_HIP_TRY(hipMemsetAsync(d_u_, 0, (size_t)3 * P * ct_bytes_, stream_));

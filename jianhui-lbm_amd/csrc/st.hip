@@ -377,7 +377,7 @@ int StSolver::create(const lbm_st_params &p, const int32_t *solid)
     PackedNbr packed;
     rc = pack_neighbours(geo_, packed, err);
     if (rc != LBM_OK) return fail(rc, err);
-    LBM_HIP_TRY(own_nbr_.upload(packed, P_, stream_));
+    LBM_HIP_TRY(own_nbr_.upload(packed, stream_));
     nbr_ = own_nbr_.view();
     LBM_HIP_TRY(hipMalloc(&own_supinv_, (size_t)P_ * sizeof(int32_t)));
     LBM_HIP_TRY(hipMemcpyAsync(own_supinv_, geo_.supinv.data(), geo_.supinv.size() * sizeof(int32_t),

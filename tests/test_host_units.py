@@ -4,7 +4,10 @@ import os
 import shutil
 import subprocess
 
+import numpy as np
 import pytest
+
+import test_gpu_link_forms as forms
 
 SAN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "sanitize")
 
@@ -29,3 +32,25 @@ def test_tuning_cache():
 @pytest.mark.parametrize("check", ["refused", "failing", "at_once"])
 def test_state_reads(check):
     assert "checks passed" in _run("readback", check)
+
+
+def test_packed_links():
+    assert "checks passed" in _run("links", "pack")
+
+
+def _width(tmp_path, solid):
+    solid.astype(np.int32).tofile(tmp_path / "solid.bin")
+    return int(_run("links", "width", *[str(n) for n in solid.shape], str(tmp_path / "solid.bin")).split()[0])
+
+
+@pytest.mark.parametrize("box", range(3))
+def test_boxes_of_the_oracle_comparison_lie_on_both_sides_of_the_width_rule(tmp_path, box):
+    """The boxes that test_gpu_link_forms compares with the oracle, drawn as it draws them."""
+    boxes = next(m for m in forms.test_large_boxes_match_the_oracle.pytestmark if m.name == "parametrize").args[1]
+    shape, porosity = boxes[box]
+    solid = np.random.default_rng(11).uniform(size=shape) > porosity
+    assert _width(tmp_path, solid) == [8, 8, 16][box]
+
+
+def test_box_of_faces_and_power_law_has_eight_bit_ranks(tmp_path):
+    assert _width(tmp_path, np.random.default_rng(13).uniform(size=(40, 170, 160)) > 0.97) == 8

@@ -41,7 +41,8 @@ PKG_DIR = os.path.join(ROOT, "jianhui-lbm_amd")
 
 HBM_PEAK_GBS = 8000.0           # MI355X HBM3E, vendor figure
 # algorithmic bytes per fluid-node update: 19 populations read + 19 written + 18 int32
-# upstream indices read
+# upstream indices read.  The device keeps the links packed in 11 to 19 bytes a node, so "frac" is a
+# rate of updates in these bytes and can pass 1; "traffic_frac" is the measured traffic's share.
 B_ALG = {"fp32": 2 * 19 * 4 + 18 * 4, "fp64": 2 * 19 * 8 + 18 * 4, "fp16": 2 * 19 * 2 + 18 * 4}
 DTYPE = {"fp32": "f32", "fp64": "f64", "fp16": "f16 storage / f32 compute"}
 
@@ -68,6 +69,12 @@ def read_traffic(tag):
         if line.startswith("traffic_bytes_per_launch:"):
             return float(line.split(":", 1)[1])
     return None
+
+
+def traffic_frac(tag, seconds):
+    """The share of the peak that the measured traffic makes in this time, where it was measured."""
+    traffic = read_traffic(tag)
+    return None if traffic is None else round(traffic / seconds / 1e9 / HBM_PEAK_GBS, 4)
 
 
 def cpu_baseline(solid, nu, g, budget_s, faces=None, power_law=None):
@@ -354,6 +361,7 @@ def cg_bench(pkg, steps, warmup, precision, edge=192, cpu_s=15.0, no_cpu=False):
            "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": round(achieved / HBM_PEAK_GBS, 4),
                         "traffic": read_traffic(f"cg_step_{precision}_{edge}cube"), "bytes_per_node": b_alg,
+                        "traffic_frac": traffic_frac(f"cg_step_{precision}_{edge}cube", ms / 1e3 / steps),
                         "kernels": "cg_collide_kernel + cg_colour_kernel per step",
                         "avg_step_us": round(ms * 1e3 / steps, 2)},
            "saturation": d["wet_count"] / d["count_in_box"], "nan_count": d["nan_count"],
@@ -434,6 +442,7 @@ def solute_bench(pkg, steps, warmup, precision, edge=384, cpu_s=15.0, no_cpu=Fal
            "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": round(achieved / HBM_PEAK_GBS, 4),
                         "traffic": read_traffic(f"sp_st_step_{precision}_{edge}cube"), "bytes_per_node": b_step,
+                        "traffic_frac": traffic_frac(f"sp_st_step_{precision}_{edge}cube", ms / 1e3 / steps),
                         "kernels": "one sp_step_kernel launch per step with the solute step fused in",
                         "avg_step_us": round(ms * 1e3 / steps, 2)},
            "mass_rel_drift": abs(d["mass"] - m0) / m0, "pore_velocity_at_end": u_pore,
@@ -458,7 +467,8 @@ def solute_bench(pkg, steps, warmup, precision, edge=384, cpu_s=15.0, no_cpu=Fal
                             "unit": "MLUPS", "kernel": "st_step_kernel", "bytes_per_node": B_ALG_ST[precision],
                             "avg_launch_us": round(avg * 1e6, 2), "achieved": round(ach, 1), "peak": HBM_PEAK_GBS,
                             "frac": round(ach / HBM_PEAK_GBS, 4),
-                            "traffic": read_traffic(f"st_step_{precision}_{edge}cube"), "launch": fs.launch()}
+                            "traffic": read_traffic(f"st_step_{precision}_{edge}cube"),
+                            "traffic_frac": traffic_frac(f"st_step_{precision}_{edge}cube", avg), "launch": fs.launch()}
     fs.close()
     if not no_cpu:
         out["cpu_baseline"] = solute_cpu_baseline(solid, nu, g, D, w0, cpu_s)
@@ -621,6 +631,7 @@ def sp_record(pkg, solid, precision, steps, warmup, nu, g, faces=None, power_law
            "ms_per_step": round(wall * 1e3 / steps, 5), "dtype": DTYPE[precision], "fluid_nodes": N,
            "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": read_traffic(tag),
+                        "traffic_frac": traffic_frac(tag, avg_launch_s),
                         "kernel": "sp_step_kernel", "bytes_per_node": b_node,
                         "avg_launch_us": round(avg_launch_s * 1e6, 2)},
            "launch": s.launch()}

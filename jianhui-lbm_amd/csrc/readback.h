@@ -3,11 +3,12 @@
 // A direct copy into pageable memory runs at 5-15 GB/s: the runtime bounces it through its own
 // buffer with one host thread, which also takes the page faults of a fresh array.  Here the
 // kernels fill the handle's device buffer by halves, copies of 2 MiB bring it to page-locked
-// slots (up to four under way), and a team of host threads moves each slot on as it arrives,
-// after touching the pages of the caller's arrays while the first copies run.  Measured on fresh
-// arrays, before -> now: a dense velocity and density of 208 MB 20.6 -> 7.9 ms, a colour-gradient
-// state of 135 MB 12.2 -> 4.8 ms, a state of 29 MB 1.77 -> 0.87 ms, one of 0.8 MB with its run of ten
-// steps 198 -> 180 us.
+// slots (up to four under way), and a team of host threads moves each slot on as it arrives.
+// Before the first one the team touches all pages of the caller's arrays, beside the first four
+// copies only: the link then waits for it through most of a long read's touching.  Measured on
+// fresh arrays, before -> now: a dense velocity and density of 208 MB 20.6 -> 7.9 ms, a
+// colour-gradient state of 135 MB 12.2 -> 4.8 ms, a state of 29 MB 1.77 -> 0.87 ms, one of 0.8 MB with
+// its run of ten steps 198 -> 180 us.
 #pragma once
 #include <hip/hip_runtime.h>
 

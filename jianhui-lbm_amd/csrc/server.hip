@@ -101,8 +101,8 @@ __device__ __forceinline__ const T *byte_at(const T *base, uint32_t off)
 
 constexpr uint32_t row_bytes(int row, uint32_t size) { return (uint32_t)row * POP_BLOCK * size; }
 
-// The step, bounded by memory: 188 bytes a node in FP32, 340 in FP64 (two round trips in a row, the
-// deltas and the gathers, for the few tiles of a small sample).
+// The step, bounded by memory: 188 bytes a node in FP32, 340 in FP64 (for the few tiles of a small
+// sample by three round trips in a row: the tile's record, the deltas and the slot, the gathers).
 // WIDE: the launch covers the tiles of wide samples only (tiles tile0 .. tile0 + gridDim.x - 1;
 // the tile table lists narrow samples' tiles first), so a launch over narrow samples carries no
 // code or registers for the high halves.
@@ -113,7 +113,7 @@ constexpr uint32_t row_bytes(int row, uint32_t size) { return (uint32_t)row * PO
 // 27,900 -> 29,300 million node updates a second in FP32, 15,900 -> 17,100 in FP64; one sample of
 // 8,753 nodes 4.0 -> 3.8 us a step.  (Blocks with the branch: 28,300 and 16,900.)
 // keep: the active samples fit the memory-side cache (fits_cache, tune.h); their tiles run in slabs and
-// the stores carry no hint: such a batch with samples that do not converge 149 -> 139 ms.
+// the stores carry no hint: a batch of these samples in FP32 58.5 -> 49.3 ms.
 template <typename ST, int BLK, bool WIDE, bool FIRST>
 __global__ void __launch_bounds__(BLK) srv_step_kernel(const TileDev *__restrict__ tiles, const SlotDev *__restrict__ slots,
                                                        const ST *__restrict__ src, ST *__restrict__ dst,

@@ -38,12 +38,21 @@ constexpr int64_t CG_SMALL_NODES = int64_t(1) << 15;   // 128-node collide tiles
 // 1,492,992 (255 MB) 45.7 -> 37.9, 2,048,000 (350 MB) 61.4 -> 69.2; FP16 702,464 18.6 -> 16.9 -> 16.0;
 // 815,257 nodes FP32 with faces and power law 30.3 -> 25.0; colour gradient FP32 864,000 (185 MB) 67.4 -> 56.5,
 // 1,492,992 (321 MB) 104.2 -> 105.4, FP64 562,432 91.4 -> 80.7; solute FP32 530,841 9.0 -> 8.3 -> 7.3, with the
-// flow 25.6 -> 23.7 -> 20.0; sixteen served samples of edges 32 to 88 155 -> 140 ms a batch.
+// flow 25.6 -> 23.7 -> 20.0; sixteen served samples of edges 32 to 88 58.5 -> 49.3 ms a batch.  A solute's
+// slabs go by the bytes of the step with its flow, also on its own: FP64 boxes of 588,505 to 1.05 M nodes
+// with a frozen velocity store without the hint but keep the hardware's order (788,456 nodes 18.5 us, in
+// slabs 17.2).
+// The rule counts the step of one handle.  Where several step at once and do not fit together, the hint
+// would be the better choice: FP64 501,992 nodes (162 MB) in two threads 25.9 us a step, with the hint
+// 29.0, in four 28.7 and 28.7, in eight 30.3 and 28.5; FP32 1,102,614 nodes (189 MB) 30.7 and 31.7, 33.0 and
+// 30.7, 34.8 and 31.2.
 constexpr int64_t CACHE_BYTES = 256000000;
 inline bool fits_cache(int64_t step_bytes) { return step_bytes <= CACHE_BYTES; }
-// Values of 2 and 4 bytes keep the hint where a buffer has 4.5 to 12 MB, in which its stores were the
-// slower ones without it: FP32 131,072 nodes 6.73 -> 7.04 us, 186,624 (14 MB) 8.99 -> 8.19; FP16 131,072 5.6 ->
-// 5.9, 256,000 8.0 -> 8.4, 340,736 (13 MB) 10.6 -> 10.3; but FP64 70,304 (11 MB) 5.9 -> 5.65.
+// Values of 2 and 4 bytes keep the hint where a buffer has 4.5 to 12 MB, in most of which the flow step
+// was slower without it: FP32 131,072 nodes 6.73 -> 7.04 us, 186,624 (14 MB) 8.99 -> 8.19; FP16 131,072 5.6 ->
+// 5.9, 256,000 8.0 -> 8.4, 340,736 (13 MB) 10.6 -> 10.3; but FP64 70,304 (11 MB) 5.9 -> 5.65.  Not in all of it: in
+// 128-node tiles, FP32 72,565 nodes 4.47 -> 4.22 and 122,507 5.58 -> 5.16, FP16 122,507 4.70 -> 4.55.  The
+// colour gradient, FP32: 72,565 nodes 12.5 -> 12.5, 95,375 12.6 -> 12.7, 122,507 12.8 -> 13.3, 137,837 17.3 -> 16.2.
 inline bool keep_stores(int64_t step_bytes, int64_t buffer_bytes, size_t width)
 {
     return fits_cache(step_bytes) && (width > 4 || buffer_bytes < 4500000 || buffer_bytes > 12000000);

@@ -43,27 +43,30 @@ PinnedUser::~PinnedUser()
     for (; sets > users && n_idle > 0; --sets) free_set(idle[--n_idle]);
 }
 
-bool pinned_take(int device, PinnedSet &out)
+bool pinned_take(int device, int slots, PinnedSet &out)
 {
-    {
-        std::lock_guard<std::mutex> lk(mu);
-        for (int k = 0; k < n_idle; ++k)
-            if (idle[k].device == device) {
-                out = idle[k];
-                idle[k] = idle[--n_idle];
-                return true;
-            }
-        if (sets == PIN_SETS) {
-            if (n_idle == 0) return false;
-            free_set(idle[--n_idle]);   // of another device
-            --sets;
-        }
-        ++sets;
-    }
     out = PinnedSet{};
     out.device = device;
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        int pick = -1;   // an idle set of the device, one that has the slots if there is
+        for (int k = 0; k < n_idle; ++k)
+            if (idle[k].device == device && (pick < 0 || !idle[pick].done[slots - 1])) pick = k;
+        if (pick >= 0) {
+            out = idle[pick];
+            idle[pick] = idle[--n_idle];
+        } else {
+            if (sets == PIN_SETS) {
+                if (n_idle == 0) return false;
+                free_set(idle[--n_idle]);   // of another device
+                --sets;
+            }
+            ++sets;
+        }
+    }
     hipError_t e = hipSuccess;
-    for (int k = 0; k < PIN_SLOTS && e == hipSuccess; ++k) {
+    for (int k = 0; k < slots && e == hipSuccess; ++k) {
+        if (out.done[k]) continue;
         e = hipHostMalloc(&out.slot[k], PIN_BYTES, hipHostMallocDefault);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&out.done[k], hipEventDisableTiming);
     }

@@ -19,9 +19,9 @@
 namespace lbm {
 
 // Page-locked slots of the reads under way, shared by the handles of the process: a read takes a
-// set for its duration.  Idle sets are kept, at most one for each handle alive, since a new set costs
-// 3 ms in page faults.  There are PIN_SETS at most (128 MiB); further reads at the same time copy
-// straight into the caller's arrays.  Thread-safe.
+// set for its duration, with as many slots as its bytes fill.  Idle sets are kept, at most one for each
+// handle alive: making and freeing a set of four slots costs 0.2 ms.  There are PIN_SETS at most (128
+// MiB); further reads at the same time copy straight into the caller's arrays.  Thread-safe.
 constexpr int PIN_SETS = 16;
 constexpr int PIN_SLOTS = 4;
 constexpr size_t PIN_BYTES = size_t(2) << 20;
@@ -30,9 +30,9 @@ struct PinnedSet {
     hipEvent_t done[PIN_SLOTS] = {nullptr};
     int device = -1;   // the events' device
 };
-// a set for a read on the device; false where all are in use or page-locked memory cannot be had (no error
-// is left pending)
-bool pinned_take(int device, PinnedSet &out);
+// a set for a read on the device, with its first `slots` slots; false where all are in use or page-locked
+// memory cannot be had (no error is left pending)
+bool pinned_take(int device, int slots, PinnedSet &out);
 void pinned_return(PinnedSet &s);
 // a member of every handle that reads back
 struct PinnedUser {
@@ -99,7 +99,8 @@ hipError_t read_back(int device, hipStream_t s, int64_t n, const ReadPart *parts
     if (width == 0 || n <= 0) return hipSuccess;
     const size_t item = sizeof(double) * (size_t)width;
     PinnedSet set;
-    if (!pinned_take(device, set)) return read_direct(s, n, parts, np, buf, buf_bytes, item, step, fill);
+    const int slots = (int)std::min<size_t>(PIN_SLOTS, ((size_t)n * item + PIN_BYTES - 1) / PIN_BYTES);
+    if (!pinned_take(device, slots, set)) return read_direct(s, n, parts, np, buf, buf_bytes, item, step, fill);
     hipError_t e = hipSuccess;
     const int64_t chunk = std::max<int64_t>(step, (int64_t)(buf_bytes / 2 / item) / step * step);
     struct Piece {
@@ -113,7 +114,7 @@ hipError_t read_back(int device, hipStream_t s, int64_t n, const ReadPart *parts
             touched = true;
             read_touch(parts, np, n);
         }
-        const int k = (int)(taken++ % PIN_SLOTS);
+        const int k = (int)(taken++ % slots);
         const hipError_t w = hipEventSynchronize(set.done[k]);
         if (w == hipSuccess) read_scatter(parts, np, ring[k].i0, ring[k].i1, ring[k].at, ring[k].bytes, set.slot[k]);
         return w;
@@ -127,9 +128,9 @@ hipError_t read_back(int device, hipStream_t s, int64_t n, const ReadPart *parts
         const size_t at = place_parts(parts, np, i0, i1, base, p);
         e = fill(i0, i1, p);
         for (size_t o = 0; o < at && e == hipSuccess; o += PIN_BYTES) {
-            if (queued - taken == PIN_SLOTS) e = take();
+            if (queued - taken == slots) e = take();
             if (e != hipSuccess) break;
-            const int k = (int)(queued % PIN_SLOTS);
+            const int k = (int)(queued % slots);
             ring[k] = Piece{i0, i1, o, std::min(PIN_BYTES, at - o)};
             e = hipMemcpyAsync(set.slot[k], base + o, ring[k].bytes, hipMemcpyDeviceToHost, s);
             if (e == hipSuccess) e = hipEventRecord(set.done[k], s);

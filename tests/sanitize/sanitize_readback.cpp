@@ -1,6 +1,7 @@
 // sanitize_readback.cpp -- the state reads (readback.h) under the sanitizers, on a stand-in for the device
 // runtime: "device" memory is host memory, copies are made at once, and page-locked allocations and copies
 // can be made to fail.  Arguments name the check.
+#include <algorithm>
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
@@ -81,24 +82,28 @@ struct Reader {
     }
 };
 
+// the slots that a read of n items fills
+int slots_of(int64_t n) { return (int)std::min<int64_t>(PIN_SLOTS, (n * 22 * 8 + (int64_t)PIN_BYTES - 1) / (int64_t)PIN_BYTES); }
+
 // one piece, several pieces, several chunks with a remainder
 const int64_t SIZES[] = {1, 255, 4224, 40329, 157286};
 
 // no page-locked memory, or not all of a set: the values all the same, and no error left behind
 void refused()
 {
-    for (int slots : {0, 3})
+    for (int slots : {0, 2})
         for (int64_t n : SIZES) {
             made = 0;
             made_at_most = slots;
             Reader r(n);
             expect(r.read([] {}) == hipSuccess && r.wrong(true) == 0, "read without page-locked memory");
-            expect(live == 0 && pending == 0, "nothing left of a refused set");
+            const int used = slots_of(n);
+            expect(live == (used <= slots ? used : 0) && pending == 0, "nothing left of a refused set");
         }
     made_at_most = 1 << 30;
     for (int64_t n : SIZES) {
         Reader r(n);
-        expect(r.read([] {}) == hipSuccess && r.wrong(true) == 0 && live == PIN_SLOTS, "read through the slots");
+        expect(r.read([] {}) == hipSuccess && r.wrong(true) == 0 && live == slots_of(n), "read through the slots");
     }
     expect(live == 0, "slots given back");
 }
@@ -143,13 +148,22 @@ void at_once()
             for (auto &t : threads) t.join();
             expect(bad == 0, "reads at once");
         }
-        const int want = std::min(count, PIN_SETS) * PIN_SLOTS;
+        const int each = slots_of(4224), want = std::min(count, PIN_SETS) * each;
         expect(made == want && live == want, "slots made once");
         readers.resize(1);
-        expect(live == PIN_SLOTS, "slots given back as handles go");
+        expect(live == each, "slots given back as handles go");
         readers.clear();
         expect(live == 0, "slots given back");
     }
+    // a set that grows with the reads, and is kept at its largest
+    made = 0;
+    Reader small(255), large(157286);
+    for (int k = 0; k < 3; ++k)
+        for (Reader *r : {&small, &large}) {
+            std::fill(r->f.begin(), r->f.end(), -1.0);
+            expect(r->read([] {}) == hipSuccess && r->wrong(true) == 0, "reads in turn");
+        }
+    expect(made == PIN_SLOTS && live == PIN_SLOTS, "one set for reads in turn");
 }
 }  // namespace
 
